@@ -629,6 +629,134 @@ SG_D uint32_t leaf_pair(const TriSoA& t, const LeafParams& L, GridHeader* h, uin
     return (uint32_t)c;
 }
 
+// Wide leaf boxes: one triangle that crosses a finely divided top cell (a
+// large triangle through a dense cluster) spans up to 255^3 leaf cells, and
+// one lane walking them sets the time of the whole launch (10,368 + 66,612
+// cells in a 502,000-triangle cluster: k_leaf_count 5.6 ms, its emission
+// 8.6 ms).  A box of at least kWideBox cells is therefore visited by its
+// block, one (y, z) row of leaf cells per thread (k_leaf_count lists it and
+// k_leaf_scan's one block counts it; the emission kernels emit it in place).
+// Along a row the plane distance never changes direction -- each binary32
+// operation between the cell centre and the distance is monotone -- so a
+// row's accepted cells are one interval, found by two binary searches.  The
+// cell centres are the running sums of leaf_visit, formed once per axis in
+// LDS.  The rebuild of that cluster went from 14.6 to 0.37 ms.  Below kWideBox
+// cells the lanes of a wave walk their boxes side by side; a shared visit
+// costs its block about as long as such a walk.
+constexpr uint32_t kWideBox = 1024;
+constexpr uint32_t kWideCap = 1024;   // wide boxes a build counts this way; the rest are walked by their lanes
+constexpr int kAxisMax = 256;      // leaf cells along an axis (resolution bytes)
+
+SG_D bool plane_tested(const LeafSetup& s) {
+    return s.hp[0] - s.lo[0] > 1 && s.hp[1] - s.lo[1] > 1 && s.hp[2] - s.lo[2] > 1;
+}
+
+// Monotone needs finite terms: coordinates below 1e18 keep every product of
+// the distance in range (a normal of zeros, infinities or NaN then rejects
+// every cell or, all zero, accepts every cell, in the search as in the walk).
+SG_D bool wide_box(const LeafParams& L, const LeafSetup& s, uint32_t c) {
+    if (c < kWideBox) return false;
+    auto ok = [](v3 a) { return fabsf(a.x) < 1e18f && fabsf(a.y) < 1e18f && fabsf(a.z) < 1e18f; };
+    return ok(s.v0) && ok(s.v1) && ok(s.v2) && ok(s.org) && ok(s.org + L.cs);
+}
+
+// Every thread of the block calls this with the same pair.  f(live, key0, xa,
+// xb) once per round of rows: cells [xa, xb) of the thread's row are accepted,
+// key0 the key of the row's cell 0 (live false: no row, xa == xb).
+template <class F>
+SG_D void wide_visit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], F&& f) {
+    const int ex = s.hp[0] - s.lo[0], ey = s.hp[1] - s.lo[1], ez = s.hp[2] - s.lo[2];
+    const uint32_t crx = f2u(s.cres.x), crxy = f2u(s.cres.x * s.cres.y);
+    const bool plane = plane_tested(s);
+    const v3 n_ = normalize(cross(s.v1 - s.v0, s.v2 - s.v0));
+    const v3 scs = L.cs / s.cres;
+    __syncthreads();   // tab is free again
+    if (threadIdx.x < 3) {
+        const int a = (int)threadIdx.x;
+        const v3 c0 = (mk((float)s.lo[0], (float)s.lo[1], (float)s.lo[2]) * scs + s.org) + scl(scs, 0.5f);
+        const float step = comp(scs, a);
+        float c = comp(c0, a) - step;
+        const int m = a == 0 ? ex : (a == 1 ? ey : ez);
+        for (int i = 0; i < m && i < kAxisMax; ++i) {
+            c += step;
+            tab[a][i] = c;
+        }
+    }
+    __syncthreads();
+    const float hx = scs.x * 0.5f + kEps, hy = scs.y * 0.5f + kEps, hz = scs.z * 0.5f + kEps;
+    const int rows = ey * ez;
+    for (int r0 = 0; r0 < rows; r0 += (int)blockDim.x) {
+        const int r = r0 + (int)threadIdx.x;
+        const bool live = r < rows;
+        int xa = 0, xb = 0;
+        uint32_t key0 = 0;
+        if (live) {
+            const int z = r / ey, y = r - z * ey;
+            key0 = (uint32_t)s.lo[0] + (uint32_t)(s.lo[1] + y) * crx + (uint32_t)(s.lo[2] + z) * crxy + s.px;
+            xb = ex;
+            if (plane) {
+                const float dy = (tab[1][y] - s.v0.y) * n_.y, dz = (tab[2][z] - s.v0.z) * n_.z;
+                auto dist = [&](int x) { return ((tab[0][x] - s.v0.x) * n_.x + dy) + dz; };
+                auto in = [&](float d) {
+                    return fabsf(n_.x * d) <= hx && fabsf(n_.y * d) <= hy && fabsf(n_.z * d) <= hz;
+                };
+                // cells before the interval lie on one side of the plane, those
+                // after it on the other
+                const bool up = n_.x >= 0.f;
+                int lo = 0, hi = ex;   // first cell not before the interval
+                while (lo < hi) {
+                    const int m = (lo + hi) >> 1;
+                    const float d = dist(m);
+                    if (!in(d) && (d < 0.f) == up) lo = m + 1;
+                    else hi = m;
+                }
+                xa = lo;
+                hi = ex;               // first cell after it
+                while (lo < hi) {
+                    const int m = (lo + hi) >> 1;
+                    if (in(dist(m))) lo = m + 1;
+                    else hi = m;
+                }
+                xb = lo;
+            }
+            const int room = key0 < L.C2 ? (int)min(L.C2 - key0, (uint32_t)ex) : 0;   // keys at C2 are rejected
+            xb = min(xb, room);
+            xa = min(xa, xb);
+        }
+        f(live, key0, xa, xb);
+    }
+}
+
+// accepted cells of a wide box (the block's sum, known to every thread)
+template <int NW>
+SG_D uint32_t wide_count(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], uint32_t* s_red) {
+    uint32_t acc = 0;
+    wide_visit(L, s, tab, [&](bool, uint32_t, int xa, int xb) { acc += (uint32_t)(xb - xa); });
+    return block_sum<NW>(acc, s_red);
+}
+
+// The leaf pairs of a wide box: accepted ones from slot pa in z/y/x order,
+// the `rej` rejected ones from slot pr (all alike: key C2).
+SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], uint32_t* s_scan, uint32_t tri,
+                    uint32_t pa, uint32_t pr, uint32_t rej, uint32_t cap, uint32_t* __restrict__ keys,
+                    uint32_t* __restrict__ vals) {
+    wide_visit(L, s, tab, [&](bool, uint32_t key0, int xa, int xb) {
+        uint32_t agg;
+        uint32_t p = pa + block_excl_scan<kBlock / 64>((uint32_t)(xb - xa), &agg, s_scan);
+        for (int x = xa; x < xb; ++x, ++p)
+            if (p < cap) {
+                keys[p] = key0 + (uint32_t)x;
+                vals[p] = tri;
+            }
+        pa += agg;
+    });
+    for (uint32_t j = threadIdx.x; j < rej; j += kBlock)
+        if (pr + j < cap) {
+            keys[pr + j] = L.C2;
+            vals[pr + j] = tri;
+        }
+}
+
 // Leaf tile of a sorted top pair: tile t holds the top cells that start in
 // [t*kLeafTile, (t+1)*kLeafTile), so pair i belongs to tile
 // floor(start of its top cell / kLeafTile).  Per tile the count kernel
@@ -674,31 +802,39 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
         const uint32_t c = leaf_pair(t, L, h, key, tri, cells, st);
         if (dbg_counts) dbg_counts[i] = c;
         uint32_t acc = 0;
+        bool counted = true;
         if (c) {
             // a box of one leaf cell on some axis has no plane test: every
             // cell is accepted unless its key reaches C2, and the largest
             // key is that of the far corner -- then the count is the volume
-            const bool plane = st.hp[0] - st.lo[0] > 1 && st.hp[1] - st.lo[1] > 1 && st.hp[2] - st.lo[2] > 1;
             const uint32_t crx = f2u(st.cres.x), crxy = f2u(st.cres.x * st.cres.y);
             const uint32_t kmax = (uint32_t)(st.hp[0] - 1) + (uint32_t)(st.hp[1] - 1) * crx +
                                   (uint32_t)(st.hp[2] - 1) * crxy + st.px;
-            if (!plane && kmax < L.C2)
+            if (!plane_tested(st) && kmax < L.C2) {
                 acc = c;
-            else
-                leaf_visit(L, st, [&](uint32_t, bool ok) { acc += ok ? 1u : 0u; });
+            } else {
+                if (wide_box(L, st, c)) {   // k_leaf_scan counts it
+                    const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
+                    counted = w >= kWideCap;
+                    if (!counted) sums[2 * (size_t)Tp + 4 + w] = i;
+                }
+                if (counted) leaf_visit(L, st, [&](uint32_t, bool ok) { acc += ok ? 1u : 0u; });
+            }
         }
-        if (pacc) {   // per-pair totals for the parallel emission of oversize tiles
+        if (counted && pacc) {   // per-pair totals for the parallel emission of oversize tiles
             pacc[i] = acc;
             prej[i] = c - acc;
         }
         if (tile < T) {
-            const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
-            if (slot < kSlots) {
-                if (acc) atomicAdd(&s_acc[slot], acc);
-                if (c - acc) atomicAdd(&s_rej[slot], c - acc);
-            } else {
-                atomicAdd(&sums[tile], acc);
-                atomicAdd(&sums[Tp + tile], c - acc);
+            if (counted) {
+                const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
+                if (slot < kSlots) {
+                    if (acc) atomicAdd(&s_acc[slot], acc);
+                    if (c - acc) atomicAdd(&s_rej[slot], c - acc);
+                } else {
+                    atomicAdd(&sums[tile], acc);
+                    atomicAdd(&sums[Tp + tile], c - acc);
+                }
             }
             if (rg.x == i) {   // first pair of its top cell
                 const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
@@ -721,16 +857,46 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
     }
 }
 
-// Exclusive scan, in place, of the accepted (sums[0..T)) and rejected
-// (sums[Tp..Tp+T)) tile totals, both halves at once (waves 0-7 and 8-15);
-// sums[2Tp], sums[2Tp+1] receive the grand totals and the header the
+// First the wide boxes k_leaf_count listed are counted into their tiles'
+// totals.  Then the exclusive scan, in place, of the accepted (sums[0..T)) and
+// rejected (sums[Tp..Tp+T)) tile totals, both halves at once (waves 0-7 and
+// 8-15); sums[2Tp], sums[2Tp+1] receive the grand totals and the header the
 // leaf-pair counts (one block of 1024 threads).
-__global__ __launch_bounds__(1024) void k_leaf_scan(GridHeader* h, BuildArgs a, uint32_t* __restrict__ sums,
-                                                    uint32_t T) {
+__global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, BuildArgs a,
+                                                    const uint32_t* __restrict__ top_keys,
+                                                    const uint32_t* __restrict__ top_vals,
+                                                    const uint32_t* __restrict__ ranges,
+                                                    const uint32_t* __restrict__ cells, uint32_t* __restrict__ sums,
+                                                    uint32_t T, uint32_t* __restrict__ pacc,
+                                                    uint32_t* __restrict__ prej) {
     constexpr int kPer = 16;
     __shared__ uint32_t s_w[16];
     __shared__ uint32_t s_tot[2];
+    __shared__ float s_tab[3][kAxisMax];
     const uint32_t Tp = leaf_sums_stride(T);
+    const uint32_t n_wide = min(sums[2 * (size_t)Tp + 2], kWideCap);
+    if (n_wide) {
+        const LeafParams L = read_leaf_params(h);
+        for (uint32_t k = 0; k < n_wide; ++k) {
+            const uint32_t i = sums[2 * (size_t)Tp + 4 + k], key = top_keys[i];
+            LeafSetup st;
+            const uint32_t c = leaf_pair(t, L, h, key, top_vals[i], cells, st);
+            const uint32_t acc = wide_count<16>(L, st, s_tab, s_w);
+            if (threadIdx.x == 0) {
+                const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
+                if (pacc) {
+                    pacc[i] = acc;
+                    prej[i] = c - acc;
+                }
+                if (tile < T) {
+                    sums[tile] += acc;
+                    sums[Tp + tile] += c - acc;
+                }
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
     const int w = wave_id(), half = w >> 3;
     const uint32_t tt = threadIdx.x & 511u;
     uint32_t* row = sums + (size_t)half * Tp;
@@ -1027,14 +1193,15 @@ SG_D void block_sort_pass_global(const uint32_t* k, const uint32_t* v, uint32_t*
 }
 
 // Tiles too large for LDS (more than kLeafStage pairs, or a local key range
-// or top-pair count beyond the LDS sort's bit budget): one block per tile
-// emits the tile's pairs in emission order.  With self_sort, the grid has no
-// global leaf sort scheduled, so the block then sorts its accepted pairs
-// itself (stable LSD passes over the tile-local key, ping-ponging with
-// tk / tv) and writes their reference records -- correct but slow, for a
-// rebuild that meets an oversize tile the grid's build never met.  Without
-// self_sort the global pass sorts them (GridHeader::leaf_sort receives the
-// number of accepted pairs).  Either way GridHeader::oversize counts the tile.
+// or top-pair count beyond the LDS sort's bit budget) of a grid without the
+// parallel emission: one block emits such a tile's pairs in emission order,
+// sorts its accepted pairs (stable LSD passes over the tile-local key,
+// ping-ponging with tk / tv) and writes their reference records -- correct but
+// slow, for a rebuild that meets an oversize tile the grid's build never met.
+// A block looks after kOverTiles tiles: most rebuilds find none oversize, and
+// a block for each tile is then 8,000 blocks that only start and end.
+// GridHeader::oversize counts the tiles.
+constexpr uint32_t kOverTiles = 16;
 __global__ __launch_bounds__(kBlock) void k_leaf_emit_large(TriSoA t, GridHeader* h, BuildArgs a,
                                                             const uint32_t* __restrict__ top_keys,
                                                             const uint32_t* __restrict__ top_vals,
@@ -1043,80 +1210,112 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_large(TriSoA t, GridHeader
                                                             uint32_t* __restrict__ vals,
                                                             const uint32_t* __restrict__ sums,
                                                             const uint32_t* __restrict__ info, uint32_t T,
-                                                            int self_sort, uint32_t* __restrict__ tk,
-                                                            uint32_t* __restrict__ tv, float* __restrict__ refs,
+                                                            uint32_t* __restrict__ tk, uint32_t* __restrict__ tv, float* __restrict__ refs,
                                                             uint32_t* __restrict__ leaves) {
     __shared__ uint32_t s_scan[kBlock / 64];
     __shared__ uint32_t s_base[256], s_wc[256 * (kBlock / 64)];
+    __shared__ uint32_t s_wide[kBlock], s_wacc[kBlock], s_wrej[kBlock], s_wcnt[kBlock], s_nwide;
+    __shared__ float s_tab[3][kAxisMax];
+    __shared__ uint32_t s_over;
     LeafTilePlan q;
-    if (!leaf_tile_plan(a, sums, info, T, blockIdx.x, q) || q.staged) return;
+    if (threadIdx.x < 64) {   // which of the block's tiles are oversize
+        const uint32_t b = blockIdx.x * kOverTiles + threadIdx.x;
+        const uint64_t m = __ballot(threadIdx.x < kOverTiles && b < T && leaf_tile_plan(a, sums, info, T, b, q) && !q.staged);
+        if (threadIdx.x == 0) s_over = (uint32_t)m;
+    }
+    __syncthreads();
     const LeafParams L = read_leaf_params(h);
     const uint32_t cap = a.cap_P2;
-    const uint32_t rej_base = q.tot_acc + q.pre_rej;
-    if (threadIdx.x == 0) {
-        atomicAdd(&h->oversize, 1u);
-        if (!self_sort) h->leaf_sort = q.tot_acc;
-    }
-    uint32_t run_acc = 0, run_rej = 0;
-    for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBlock) {
-        const uint32_t i = c0 + threadIdx.x;
-        LeafSetup s;
-        uint32_t tri = 0, c = 0, ca = 0;
-        if (i < q.a1) {
-            tri = top_vals[i];
-            c = leaf_pair(t, L, h, top_keys[i], tri, cells, s);
-            if (c) leaf_visit(L, s, [&](uint32_t, bool ok) { ca += ok ? 1u : 0u; });
+    for (uint32_t todo = s_over; todo; todo &= todo - 1u) {
+        leaf_tile_plan(a, sums, info, T, blockIdx.x * kOverTiles + (uint32_t)__ffs((int)todo) - 1u, q);
+        const uint32_t rej_base = q.tot_acc + q.pre_rej;
+        if (threadIdx.x == 0) atomicAdd(&h->oversize, 1u);
+        uint32_t run_acc = 0, run_rej = 0;
+        for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBlock) {
+            const uint32_t i = c0 + threadIdx.x;
+            LeafSetup s;
+            uint32_t tri = 0, c = 0, ca = 0;
+            bool wide = false;
+            if (threadIdx.x == 0) s_nwide = 0;
+            __syncthreads();
+            if (i < q.a1) {
+                tri = top_vals[i];
+                c = leaf_pair(t, L, h, top_keys[i], tri, cells, s);
+                wide = wide_box(L, s, c);
+                if (wide) s_wide[atomicAdd(&s_nwide, 1u)] = threadIdx.x;
+                else if (c) leaf_visit(L, s, [&](uint32_t, bool ok) { ca += ok ? 1u : 0u; });
+            }
+            __syncthreads();
+            const uint32_t nwide = s_nwide;
+            for (uint32_t k = 0; k < nwide; ++k) {
+                LeafSetup ws;
+                const uint32_t pair = c0 + s_wide[k];
+                leaf_pair(t, L, h, top_keys[pair], top_vals[pair], cells, ws);
+                const uint32_t acc = wide_count<kBlock / 64>(L, ws, s_tab, s_scan);
+                if (threadIdx.x == s_wide[k]) ca = acc;
+            }
+            uint32_t agg_a, agg_r;
+            uint32_t pa = q.pre_acc + run_acc + block_excl_scan<kBlock / 64>(ca, &agg_a, s_scan);
+            uint32_t pr = rej_base + run_rej + block_excl_scan<kBlock / 64>(c - ca, &agg_r, s_scan);
+            if (wide) {
+                s_wacc[threadIdx.x] = pa;
+                s_wrej[threadIdx.x] = pr;
+                s_wcnt[threadIdx.x] = ca;
+            } else if (c) {
+                leaf_visit(L, s, [&](uint32_t key, bool ok) {
+                    const uint32_t idx = ok ? pa++ : pr++;
+                    if (idx < cap) {
+                        keys[idx] = ok ? key : L.C2;
+                        vals[idx] = tri;
+                    }
+                });
+            }
+            __syncthreads();
+            for (uint32_t k = 0; k < nwide; ++k) {
+                LeafSetup ws;
+                const uint32_t w = s_wide[k], pair = c0 + w, wtri = top_vals[pair];
+                const uint32_t wc = leaf_pair(t, L, h, top_keys[pair], wtri, cells, ws);
+                wide_emit(L, ws, s_tab, s_scan, wtri, s_wacc[w], s_wrej[w], wc - s_wcnt[w], cap, keys, vals);
+            }
+            __syncthreads();   // the lists are free for the next chunk
+            run_acc += agg_a;
+            run_rej += agg_r;
         }
-        uint32_t agg_a, agg_r;
-        uint32_t pa = q.pre_acc + run_acc + block_excl_scan<kBlock / 64>(ca, &agg_a, s_scan);
-        uint32_t pr = rej_base + run_rej + block_excl_scan<kBlock / 64>(c - ca, &agg_r, s_scan);
-        if (c)
-            leaf_visit(L, s, [&](uint32_t key, bool ok) {
-                const uint32_t idx = ok ? pa++ : pr++;
-                if (idx < cap) {
-                    keys[idx] = ok ? key : L.C2;
-                    vals[idx] = tri;
-                }
-            });
-        run_acc += agg_a;
-        run_rej += agg_r;
-    }
-    if (!self_sort) return;
-    // the accepted pairs of this tile: [pre_acc, pre_acc + run_acc), keys in
-    // [kbase, kbase + span) (leaf_tile_plan guarantees pre_acc + run_acc <= cap)
-    __threadfence_block();
-    __syncthreads();
-    const uint32_t n = run_acc;
-    uint32_t* k0 = keys + q.pre_acc;
-    uint32_t* v0 = vals + q.pre_acc;
-    uint32_t* k1 = tk + q.pre_acc;
-    uint32_t* v1 = tv + q.pre_acc;
-    const uint32_t span = q.span == 0xFFFFFFFFu ? 0xFFFFFFFFu : q.span;
-    const int bits = 32 - __builtin_clz(span | 1u);
-    const int passes = (bits + 7) / 8;
-    const int db = (bits + passes - 1) / passes;
-    for (int p = 0, lo = 0; p < passes; ++p, lo += db) {
-        if (p & 1) block_sort_pass_global(k1, v1, k0, v0, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
-        else block_sort_pass_global(k0, v0, k1, v1, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
+        // the accepted pairs of this tile: [pre_acc, pre_acc + run_acc), keys in
+        // [kbase, kbase + span) (leaf_tile_plan guarantees pre_acc + run_acc <= cap)
         __threadfence_block();
         __syncthreads();
-    }
-    if (passes & 1) {
-        for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
-            k0[i] = k1[i];
-            v0[i] = v1[i];
+        const uint32_t n = run_acc;
+        uint32_t* k0 = keys + q.pre_acc;
+        uint32_t* v0 = vals + q.pre_acc;
+        uint32_t* k1 = tk + q.pre_acc;
+        uint32_t* v1 = tv + q.pre_acc;
+        const uint32_t span = q.span == 0xFFFFFFFFu ? 0xFFFFFFFFu : q.span;
+        const int bits = 32 - __builtin_clz(span | 1u);
+        const int passes = (bits + 7) / 8;
+        const int db = (bits + passes - 1) / passes;
+        for (int p = 0, lo = 0; p < passes; ++p, lo += db) {
+            if (p & 1) block_sort_pass_global(k1, v1, k0, v0, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
+            else block_sort_pass_global(k0, v0, k1, v1, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
+            __threadfence_block();
+            __syncthreads();
         }
-    }
-    for (uint32_t i = threadIdx.x; i < n; i += kBlock)
-        write_ref_record(refs, q.pre_acc + i, t.rec, (passes & 1) ? v1[i] : v0[i], L.n_tris);
-    if (!leaves) return;
-    // the ranges of the tile's leaf cells from its sorted keys (as k_leaf_emit)
-    __threadfence_block();
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
-        const uint32_t key = k0[i];
-        if (i == 0 || k0[i - 1] != key) leaves[2 * (size_t)key] = q.pre_acc + i;
-        if (i + 1 == n || k0[i + 1] != key) leaves[2 * (size_t)key + 1] = q.pre_acc + i + 1u;
+        if (passes & 1) {
+            for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
+                k0[i] = k1[i];
+                v0[i] = v1[i];
+            }
+        }
+        for (uint32_t i = threadIdx.x; i < n; i += kBlock)
+            write_ref_record(refs, q.pre_acc + i, t.rec, (passes & 1) ? v1[i] : v0[i], L.n_tris);
+        // the ranges of the tile's leaf cells from its sorted keys (as k_leaf_emit)
+        __threadfence_block();
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
+            const uint32_t key = k0[i];
+            if (i == 0 || k0[i - 1] != key) leaves[2 * (size_t)key] = q.pre_acc + i;
+            if (i + 1 == n || k0[i + 1] != key) leaves[2 * (size_t)key + 1] = q.pre_acc + i + 1u;
+        }
     }
 }
 
@@ -1133,33 +1332,57 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
                                                           uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
                                                           const uint32_t* __restrict__ sums,
                                                           const uint32_t* __restrict__ info, uint32_t T,
+                                                          const uint32_t* __restrict__ prej,
                                                           const uint32_t* __restrict__ sacc,
                                                           const uint32_t* __restrict__ srej) {
+    __shared__ uint32_t s_scan[kBlock / 64], s_wide[kBlock], s_nwide;
+    __shared__ float s_tab[3][kAxisMax];
     const LeafParams L = read_leaf_params(h);
     const uint32_t P1v = min(h->P1_valid, a.cap_P1);
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < P1v; i += gridDim.x * kBlock) {
-        const uint32_t key = top_keys[i];
-        if (key >= L.C1) continue;
-        const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
+    for (uint32_t base = blockIdx.x * kBlock; base < P1v; base += gridDim.x * kBlock) {
+        if (threadIdx.x == 0) s_nwide = 0;
+        __syncthreads();
+        // the tile plan of pair i, when its tile is this kernel's
         LeafTilePlan q;
-        if (tile >= T || !leaf_tile_plan(a, sums, info, T, tile, q) || q.staged) continue;
-        if (i == q.a0) {
-            h->leaf_sort = q.tot_acc;
-            atomicAdd(&h->oversize, 1u);
+        auto mine = [&](uint32_t key) {
+            if (key >= L.C1) return false;
+            const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
+            return tile < T && leaf_tile_plan(a, sums, info, T, tile, q) && !q.staged;
+        };
+        auto acc_slot = [&](uint32_t i) { return q.pre_acc + (sacc[i] - sacc[q.a0]); };
+        auto rej_slot = [&](uint32_t i) { return q.tot_acc + q.pre_rej + (srej[i] - srej[q.a0]); };
+        const uint32_t i = base + threadIdx.x;
+        const uint32_t key = i < P1v ? top_keys[i] : L.C1;
+        if (mine(key)) {
+            if (i == q.a0) {
+                h->leaf_sort = q.tot_acc;
+                atomicAdd(&h->oversize, 1u);
+            }
+            const uint32_t tri = top_vals[i];
+            LeafSetup s;
+            const uint32_t c = leaf_pair(t, L, h, key, tri, cells, s);
+            if (wide_box(L, s, c)) {
+                s_wide[atomicAdd(&s_nwide, 1u)] = i;
+            } else if (c) {
+                uint32_t pa = acc_slot(i), pr = rej_slot(i);
+                leaf_visit(L, s, [&](uint32_t k2, bool ok) {
+                    const uint32_t idx = ok ? pa++ : pr++;
+                    if (idx < a.cap_P2) {
+                        keys[idx] = ok ? k2 : L.C2;
+                        vals[idx] = tri;
+                    }
+                });
+            }
         }
-        uint32_t pa = q.pre_acc + (sacc[i] - sacc[q.a0]);
-        uint32_t pr = q.tot_acc + q.pre_rej + (srej[i] - srej[q.a0]);
-        const uint32_t tri = top_vals[i];
-        LeafSetup s;
-        const uint32_t c = leaf_pair(t, L, h, key, tri, cells, s);
-        if (c)
-            leaf_visit(L, s, [&](uint32_t k2, bool ok) {
-                const uint32_t idx = ok ? pa++ : pr++;
-                if (idx < a.cap_P2) {
-                    keys[idx] = ok ? k2 : L.C2;
-                    vals[idx] = tri;
-                }
-            });
+        __syncthreads();
+        for (uint32_t k = 0; k < s_nwide; ++k) {
+            const uint32_t w = s_wide[k], wkey = top_keys[w], wtri = top_vals[w];
+            LeafSetup s;
+            leaf_pair(t, L, h, wkey, wtri, cells, s);
+            mine(wkey);
+            wide_emit(L, s, s_tab, s_scan, wtri, acc_slot(w), rej_slot(w), prej[w], a.cap_P2, keys, vals);
+        }
+        __syncthreads();   // the list is free for the next chunk
     }
 }
 
@@ -1244,7 +1467,8 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
                            sums, info, T, dbg, large ? large->pacc : nullptr, large ? large->prej : nullptr);
-    hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, h, a, sums, T);
+    hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges, cells, sums, T,
+                       large ? large->pacc : nullptr, large ? large->prej : nullptr);
     // with `large`, the global sort and k_ranges need every key; without it
     // the tiles write the leaf ranges and the keys are kept for keep_debug
     uint32_t* lv = large ? nullptr : leaves;
@@ -1257,10 +1481,10 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
         uint32_t pb = (a.cap_P1 + kBlock - 1) / kBlock;
         pb = pb < 1 ? 1 : (pb > 4096 ? 4096 : pb);
         hipLaunchKernelGGL(k_leaf_emit_par, dim3(pb), dim3(kBlock), 0, st, t, h, a, top_keys, top_vals, ranges, cells,
-                           keys, vals, sums, info, T, large->sacc, large->srej);
+                           keys, vals, sums, info, T, large->prej, large->sacc, large->srej);
     } else {
-        hipLaunchKernelGGL(k_leaf_emit_large, dim3(T), dim3(kBlock), 0, st, t, h, a, top_keys, top_vals, cells, keys,
-                           vals, sums, info, T, 1, tmp_keys, tmp_vals, refs, lv);
+        hipLaunchKernelGGL(k_leaf_emit_large, dim3((T + kOverTiles - 1) / kOverTiles), dim3(kBlock), 0, st, t, h, a,
+                           top_keys, top_vals, cells, keys, vals, sums, info, T, tmp_keys, tmp_vals, refs, lv);
     }
 }
 
@@ -1390,7 +1614,10 @@ size_t leaf_tiles(uint32_t n) {
     const size_t t = ((size_t)n + kLeafTile - 1) / kLeafTile;
     return t ? t : 1;
 }
-size_t leaf_sums_words(uint32_t n) { return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4; }
+// accepted and rejected totals, their grand totals, the list of wide boxes
+size_t leaf_sums_words(uint32_t n) {
+    return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap;
+}
 size_t leaf_info_words(uint32_t n) { return 4 * leaf_tiles(n); }
 
 

@@ -148,6 +148,60 @@ def test_rebuild_into_an_oversize_tile(ctx, oracle):
     np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
 
 
+def _dense_cell_with_wide_boxes(n_small):
+    """n_small tiny triangles in a sphere of radius 0.02 (one finely divided
+    top cell) and 300 large ones, ten of which cross it: seven at random
+    angles, one on a coordinate plane, one collinear, one almost a point"""
+    a = sa.gen_cluster(11, n_small, 300)
+    rng = np.random.default_rng(12)
+    big = (0.5 + rng.uniform(-0.4, 0.4, (7, 3, 3))).astype(np.float32)
+    big[:, 0] = 1.5 - big[:, 1] / 2 - big[:, 2] / 2 - 0.5   # around the cell
+    flat = [[0.2, 0.2, 0.5], [0.9, 0.3, 0.5], [0.4, 0.8, 0.5]]
+    line = [[0.25, 0.25, 0.25], [0.5, 0.5, 0.5], [0.75, 0.75, 0.75]]
+    dot = [[0.5, 0.5, 0.5], [0.5, 0.5, 0.5000001], [0.5, 0.5000001, 0.5]]
+    for k, t in enumerate(list(big) + [flat, line, dot]):
+        a[:, n_small + 5 + k] = np.asarray(t, np.float32).reshape(9)
+    return a
+
+
+@pytest.mark.parametrize("n_small", [3_000, 30_000, 200_000])
+def test_wide_leaf_boxes_bit_exact(ctx, oracle, n_small):
+    """large triangles across a finely divided top cell: leaf boxes below and
+    far above the size from which a block visits a box together"""
+    a = _dense_cell_with_wide_boxes(n_small)
+    kw = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16)
+    og = oracle.build_twolevel(a, **kw)
+    assert og.status == 0
+    assert og.pair_counts.max() > n_small // 25
+    _, g = _gpu_build(ctx, a, 1, **kw)
+    for _ in range(2):
+        _assert_same_params(g.info(), og)
+        _assert_top_level(g, og)
+        _assert_leaf_level(g, og)
+        g.rebuild()
+
+
+@pytest.mark.parametrize("n_small", [3_000, 30_000])
+def test_rebuild_into_wide_leaf_boxes(ctx, oracle, n_small):
+    """the same meshes met first by a rebuild: the grid is built while the
+    small triangles are spread over the scene, so one block emits and sorts
+    the dense cell's tile"""
+    b = _dense_cell_with_wide_boxes(n_small)
+    a = b.copy()
+    rng = np.random.default_rng(13)
+    a[:, :n_small] += np.tile(rng.uniform(0, 9, (3, n_small)), (3, 1)).astype(np.float32)
+    scene, g = _gpu_build(ctx, a, 1, lam=5.0, lambda_leaf=2.0, capacity_slack=4.0)
+    res = tuple(g.info().res)
+    scene.upload_vertices(b)
+    g.rebuild()
+    og = oracle.build_twolevel(b, lam=5.0, top_divisor=6, lambda_leaf=2.0, res_override=res)
+    info = g.info()
+    assert info.status == og.status == 0
+    assert og.pair_counts.max() >= (1024 if n_small > 10_000 else 64)
+    _assert_top_level(g, og)
+    _assert_leaf_level(g, og)
+
+
 def test_twolevel_reference_leaf_lambda(ctx, oracle):
     """lambda_leaf = 1.2 (TwoLevelBuildKernels.h:49) on the 10k soup"""
     w = W.soup10k()

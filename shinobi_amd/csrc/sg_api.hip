@@ -251,6 +251,7 @@ static size_t grid_layout(sg_grid* g, char* pool) {
         g->leaves = (uint32_t*)take((size_t)g->cap_C2 * 8 + 16);
     }
     g->refs = (float*)take((size_t)(two ? g->cap_P2 : g->cap_P1) * 36 + 16);
+    g->words = two ? nullptr : (uint4*)take(cell_words(g->cap_C1) * sizeof(uint4));
     if (two && g->large_path) {
         g->large.pacc = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
         g->large.prej = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
@@ -373,6 +374,7 @@ bool uni_job_of(sg_grid* g, UniJob* j) {
     j->rb = g->rb;
     j->ranges = g->ranges1;
     j->refs = g->refs;
+    j->words = g->words;
     return true;
 }
 
@@ -399,7 +401,9 @@ static void enqueue_build(sg_grid* g, bool fixed_res, hipStream_t st, void* cons
     mark(3);
     const int f1 = g->passes1 & 1;
     launch_ranges(g->k1[f1], &g->hdr->P1, g->cap_P1, &g->hdr->C1, g->ranges1, &g->hdr->P1_valid, st);
-    if (!two) launch_ref_records(g->v1[f1], &g->hdr->P1_valid, nullptr, g->cap_P1, g->scene->rec, N, g->refs, st);
+    if (!two)
+        launch_uniform_records(g->v1[f1], g->hdr, g->cap_P1, g->scene->rec, N, g->refs, g->ranges1, g->cap_C1, g->words,
+                               st);
     mark(4);
     if (!two) return;
     launch_leaf_cells(g->hdr, a, g->ranges1, g->cells1, g->dbg_leafc, g->sums_cells, st);

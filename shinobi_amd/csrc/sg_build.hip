@@ -1523,6 +1523,44 @@ void launch_ref_records(const uint32_t* indices, const uint32_t* d_valid, const 
                        rec, n_tris, refs);
 }
 
+// cell words from the cell ranges: a wave reads 64 neighbouring ranges and
+// writes their two words
+SG_D void cell_words_body(const uint32_t* __restrict__ ranges, uint32_t C, uint4* __restrict__ words, uint32_t bid,
+                          uint32_t nb) {
+    if (C < kWordCells) return;   // never read
+    const uint32_t pairs = (C + 63u) / 64u;
+    for (uint32_t w = bid * (kBlock / 64) + (uint32_t)wave_id(); w < pairs; w += nb * (kBlock / 64)) {
+        const uint32_t k = 64u * w + (uint32_t)lane_id();
+        const uint2 rg = k < C ? reinterpret_cast<const uint2*>(ranges)[k] : make_uint2(0u, 0u);
+        const uint32_t n = rg.y - rg.x;
+        const uint64_t m1 = __ballot(n >= 1u), m2 = __ballot(n >= 2u), m3 = __ballot(n >= 3u), m4 = __ballot(n >= 4u);
+        const int sh = lane_id() & 32;
+        const uint32_t h1 = (uint32_t)(m1 >> sh);
+        const uint32_t first = (uint32_t)__shfl((int)rg.x, sh + (h1 ? __ffs((int)h1) - 1 : 0), 64);
+        if ((lane_id() & 31) == 0)
+            words[2u * w + (sh ? 1u : 0u)] = make_uint4(h1, (uint32_t)(m2 >> sh), (uint32_t)(m3 >> sh),
+                                                        (uint32_t)(m4 >> sh) ? first | kWordFull : first);
+    }
+}
+
+// the last launch of a uniform build: reference records and cell words
+__global__ __launch_bounds__(kBlock) void k_uniform_records(const uint32_t* __restrict__ indices,
+                                                            const GridHeader* h, uint32_t cap,
+                                                            const float* __restrict__ rec, uint32_t n_tris,
+                                                            float* __restrict__ refs,
+                                                            const uint32_t* __restrict__ ranges, uint32_t cap_C,
+                                                            uint4* __restrict__ words) {
+    cell_words_body(ranges, min(h->C1, cap_C), words, blockIdx.x, gridDim.x);
+    ref_records_body(indices, &h->P1_valid, nullptr, cap, rec, n_tris, refs, blockIdx.x, gridDim.x);
+}
+
+void launch_uniform_records(const uint32_t* indices, const GridHeader* h, uint32_t cap, const float* rec,
+                            uint32_t n_tris, float* refs, const uint32_t* ranges, uint32_t cap_C, uint4* words,
+                            hipStream_t st) {
+    hipLaunchKernelGGL(k_uniform_records, dim3(refs_blocks(cap)), dim3(kBlock), 0, st, indices, h, cap, rec, n_tris,
+                       refs, ranges, cap_C, words);
+}
+
 // ------------------------------------------------ many uniform grids, one launch
 // k_multi_*: one launch of a phase for every job of an entry table; each
 // block runs the phase's body for its job (see UniJob)
@@ -1576,6 +1614,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_refs(const UniJob* __restrict_
     uint32_t bid, nb;
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
     const int f = j.passes & 1;
+    cell_words_body(j.ranges, min(j.h->C1, j.a.cap_C1), j.words, bid, nb);
     ref_records_body(j.v[f], &j.h->P1_valid, nullptr, j.cap_P, j.t.rec, j.n, j.refs, bid, nb);
 }
 

@@ -65,6 +65,7 @@ struct sg_grid {
     uint32_t *k2[2] = {nullptr, nullptr}, *v2[2] = {nullptr, nullptr};
     uint32_t* leaves = nullptr;
     float* refs = nullptr;    // per-reference records (write_ref_record)
+    uint4* words = nullptr;   // uniform: cell words (GridView::words)
     // parallel emission of oversize leaf tiles, laid out once a build of this
     // grid has met one (GridHeader::leaf_sort > 0)
     bool large_path = false;
@@ -137,6 +138,7 @@ inline GridView grid_view(const sg_grid* g) {
     v.indices = two ? g->v2[f2] : g->v1[f1];
     v.rec = g->scene->rec;
     v.refs = g->refs;
+    v.words = g->words;
     v.kind = g->kind;
     return v;
 }

@@ -325,3 +325,49 @@ def test_paths_with_ordered_bounces_equal_oracle(ctx, oracle):
             rays_o, _ = oracle.bounce(w.scene, rays_o, po, to, w.bounce_seed + d, order="exit", box=box)
     g.close()
     scene.close()
+
+
+def _clumped_soup(shift):
+    """20,000 small triangles, a quarter of them in clumps so that cells hold
+    from none to dozens of references"""
+    a = sa.gen_soup(81, 20_000, 0.01)
+    rng = np.random.default_rng(82)
+    at = rng.uniform(0.1, 0.9, (3, 50)).astype(np.float32)
+    k = np.arange(5_000)
+    mid = a[0:3, :5_000].copy()
+    for v in range(3):
+        a[3 * v:3 * v + 3, :5_000] += -mid + at[:, k % 50] + (0.02 * (mid - 0.5)).astype(np.float32)
+    return (a + np.float32(shift)).astype(np.float32)
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("shift", [0.0, 1000.0])
+@pytest.mark.parametrize("res", [(40, 41, 39), (64, 64, 32), (51, 53, 52), (131, 1, 1009)])
+def test_uniform_cell_words(ctx, oracle, res, shift, shadow):
+    """uniform walks below, at and above the size from which the cell ranges
+    are read from the packed words, with cells of more references than a word
+    can hold, rays that start inside, outside and on the faces, rays along the
+    axes and short ones; at +1000 the entry points round onto or past the far
+    faces.  Ids, t and the walk's counters equal the oracle's."""
+    a = _clumped_soup(shift)
+    og = oracle.build_uniform(a, lam=5.0, top_divisor=1, res_override=res)
+    assert og.status == 0
+    b = sa.FastSimpleGridBuilder(ctx, res_override=res)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    rays = sa.gen_random_rays(83, 20_000, -0.3, 1.3)
+    n = rays.shape[1] // 8
+    rays[3, :n] = 0.0                                  # in a plane across x
+    rays[4, n // 2:n] = 0.0                            # along z
+    rays[0, n:2 * n] = np.where(np.arange(n) % 2, og.bmin[0] - np.float32(shift), og.bmax[0] - np.float32(shift))
+    rays[2, 2 * n:3 * n] = og.bmax[2] - np.float32(shift)
+    rays[6, 3 * n:4 * n] = 0.2                         # short segments
+    rays[0:3] += np.float32(shift)
+    if shadow:
+        rays[6] = 1.0
+    pg, tg, sg = g.trace_host(rays, with_stats=True, shadow=shadow)
+    po, to, so = og.trace(rays, with_stats=True, shadow=shadow)
+    np.testing.assert_array_equal(pg, po)
+    np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+    np.testing.assert_array_equal(sg, so)
+    assert (po != sa.MISS).sum() > 100

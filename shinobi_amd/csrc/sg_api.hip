@@ -269,8 +269,9 @@ static size_t grid_layout(sg_grid* g, char* pool) {
     g->bpart = (uint32_t*)take(bounds_blocks(N) * 6 * 4 + 16);
     g->sums_top = (uint32_t*)take(emit_tiles(N) * 4 + 16);
     g->sums_cells = two ? (uint32_t*)take(cell_tiles(g->cap_C1) * 4 + 16) : nullptr;
-    g->sums_leaf = two ? (uint32_t*)take(leaf_sums_words(g->cap_P1) * 4) : nullptr;
+    g->sums_leaf = two ? (uint32_t*)take((leaf_sums_words(g->cap_P1) + leaf_item_words(g->cap_P1)) * 4) : nullptr;
     g->leaf_info = two ? (uint32_t*)take(leaf_info_words(g->cap_P1) * 4) : nullptr;
+    g->boxes = two ? (uint2*)take((size_t)g->cap_P1 * 8 + 16) : nullptr;
     g->key_bits1 = bit_length(g->cap_C1);
     g->passes1 = sort_passes(g->key_bits1, g->rb);
     g->sort1_words = sort_scratch_words(g->cap_P1, g->key_bits1, g->rb);
@@ -340,7 +341,8 @@ static ZeroSegs zero_segs(const sg_grid* g) {
     };
     seg(g->ranges1, (size_t)g->cap_C1 * 8);
     if (two) {
-        seg(g->leaves, (size_t)g->cap_C2 * 8);
+        // without the global leaf sort the emission writes every leaf range
+        if (g->large_path) seg(g->leaves, (size_t)g->cap_C2 * 8);
         seg(g->sums_leaf, leaf_sums_words(g->cap_P1) * 4);
         seg(g->leaf_info, leaf_info_words(g->cap_P1) * 4);
     }
@@ -406,11 +408,12 @@ static void enqueue_build(sg_grid* g, bool fixed_res, hipStream_t st, void* cons
                                st);
     mark(4);
     if (!two) return;
-    launch_leaf_cells(g->hdr, a, g->ranges1, g->cells1, g->dbg_leafc, g->sums_cells, st);
+    launch_leaf_cells(g->hdr, a, g->ranges1, g->cells1, g->dbg_leafc, g->sums_cells, g->large_path ? nullptr : g->leaves,
+                      st);
     mark(5);
     launch_leaf_emit(t, g->hdr, a, g->k1[f1], g->v1[f1], g->ranges1, g->cells1, g->k2[0], g->v2[0], g->k2[1],
-                     g->v2[1], g->refs, g->dbg_pair, g->sums_leaf, g->leaf_info, g->large_path ? &g->large : nullptr,
-                     g->leaves, st);
+                     g->v2[1], g->refs, g->dbg_pair, g->sums_leaf, g->leaf_info, g->boxes,
+                     g->large_path ? &g->large : nullptr, g->leaves, st);
     mark(6);
     // Only a grid whose build met leaf tiles too large for the LDS sort has
     // the parallel emission of such tiles and needs the global sort after

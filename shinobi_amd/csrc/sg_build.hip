@@ -471,7 +471,8 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_count(GridHeader* h, Buil
 __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, BuildArgs a,
                                                              const uint32_t* __restrict__ ranges,
                                                              uint32_t* __restrict__ cells,
-                                                             const uint32_t* __restrict__ sums) {
+                                                             const uint32_t* __restrict__ sums,
+                                                         uint32_t* __restrict__ leaves) {
     __shared__ uint32_t s_scan[kBlock / 64];
     const uint32_t C1 = h->C1;
     const uint32_t base = blockIdx.x * kBlock;
@@ -482,7 +483,13 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
     if (k < C1) cnt = leaf_cell(h, a, ranges, k, &bits);
     uint32_t agg;
     const uint32_t local = block_excl_scan<kBlock / 64>(cnt, &agg, s_scan);
-    if (k < C1) reinterpret_cast<uint2*>(cells)[k] = make_uint2(prefix + local, bits);
+    if (k < C1) {
+        reinterpret_cast<uint2*>(cells)[k] = make_uint2(prefix + local, bits);
+        // an empty top cell's one leaf cell; the others' are written by the
+        // tiles that emit their pairs, so nothing else clears them
+        if (leaves && !(bits & kNotEmpty) && prefix + local < a.cap_C2)
+            reinterpret_cast<uint2*>(leaves)[prefix + local] = make_uint2(0u, 0u);
+    }
     if (base + kBlock >= C1 && threadIdx.x == 0) {
         const uint32_t C2 = prefix + agg;
         h->need_C2 = C2;
@@ -508,19 +515,33 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
 // order.  Leaf tiles hold whole top cells: tile t covers the sorted top pairs
 // from the first top-cell start at or after t*kLeafTile to the first one at
 // or after (t+1)*kLeafTile.  The count kernel runs the plane test and leaves
-// the tile's accepted and rejected totals; the emit kernel builds the tile's
-// pairs in LDS as (tile-local key << 12 | index of the top pair within the
-// tile), sorts them by key there and writes accepted pairs to their final
+// the tile's accepted and rejected totals, and for each pair where its box
+// begins and which cells of it were accepted (PairBox); the emit kernel
+// counts the tile's pairs per leaf cell in LDS, scans the counts, puts each
+// pair's index into its cells' lists and writes accepted pairs to their final
 // slots and rejected ones to the tail.  A tile too large for LDS writes
 // its pairs in emission order and raises GridHeader::leaf_sort, which enables
 // a global stable radix sort of the accepted pairs (a no-op otherwise).
 constexpr uint32_t kLeafTile = 512;                   // nominal sorted top pairs per leaf tile
 constexpr int kLeafBlock = 512;                       // threads of the leaf emission kernel
-constexpr uint32_t kLeafStage = 4096;                 // leaf pairs a tile sorts in LDS
-constexpr int kPayBits = 12;                          // payload: top pair index within the tile
-constexpr int kLocalBits = 16;                        // tile-local key bits the LDS sort handles
-constexpr int kDigitBits = 6;                         // widest digit of an LDS sort pass
-constexpr int kLeafRounds = kLeafStage / kLeafBlock;  // LDS sort rounds per pass
+constexpr int kBigBlock = 1024;                       // threads of its form for larger tiles
+// What a tile may hold in LDS: accepted pairs, leaf cells, top pairs.  A tile
+// beyond LeafSmall goes to the larger kernel, one beyond LeafBig is oversize.
+struct LeafSmall {
+    static constexpr uint32_t pairs = 4096, span = 4096, tops = 1536;
+};
+struct LeafBig {
+    static constexpr uint32_t pairs = 65024, span = 16384, tops = 8192;
+};
+// A tile of the larger kernel is taken by several blocks: slice s holds the
+// leaf cells whose lists begin in [s * kLeafSlice, (s+1) * kLeafSlice) of the
+// tile's accepted pairs.  Every block counts the whole tile, then lists, sorts
+// and writes its slice only.
+constexpr uint32_t kLeafSlice = 4096;
+constexpr uint32_t kSliceShift = 24, kSlicesMax = (LeafBig::pairs + kLeafSlice - 1) / kLeafSlice;
+constexpr int kTopBits = 13;                          // a list entry's top pair bits
+static_assert(LeafBig::tops <= 1u << kTopBits && LeafBig::pairs < 65536u, "list entries and 16-bit counts");
+static_assert(kSlicesMax <= 256u, "slice bits of a work item");
 
 struct LeafParams {
     v3 gmin, cs;
@@ -737,12 +758,13 @@ SG_D uint32_t wide_count(const LeafParams& L, const LeafSetup& s, float (*tab)[k
 
 // The leaf pairs of a wide box: accepted ones from slot pa in z/y/x order,
 // the `rej` rejected ones from slot pr (all alike: key C2).
+template <int NW>
 SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], uint32_t* s_scan, uint32_t tri,
                     uint32_t pa, uint32_t pr, uint32_t rej, uint32_t cap, uint32_t* __restrict__ keys,
                     uint32_t* __restrict__ vals) {
     wide_visit(L, s, tab, [&](bool, uint32_t key0, int xa, int xb) {
         uint32_t agg;
-        uint32_t p = pa + block_excl_scan<kBlock / 64>((uint32_t)(xb - xa), &agg, s_scan);
+        uint32_t p = pa + block_excl_scan<NW>((uint32_t)(xb - xa), &agg, s_scan);
         for (int x = xa; x < xb; ++x, ++p)
             if (p < cap) {
                 keys[p] = key0 + (uint32_t)x;
@@ -750,11 +772,55 @@ SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisM
             }
         pa += agg;
     });
-    for (uint32_t j = threadIdx.x; j < rej; j += kBlock)
+    for (uint32_t j = threadIdx.x; j < rej; j += NW * 64)
         if (pr + j < cap) {
             keys[pr + j] = L.C2;
             vals[pr + j] = tri;
         }
+}
+
+// PairBox: what the emission needs of a top pair, so that it neither gathers
+// the triangle nor forms its box and plane again.  x: the leaf cell of the
+// box's corner within its top cell (16 bits) and the box's extents less one
+// (5 bits each); y: the accepted cells, bit k for the k-th in z/y/x order.
+// Boxes of up to 32 cells with a corner below 2^16 have this form; others
+// are open (kBoxOpen: the emission visits the box again), pairs without leaf
+// cells empty.
+constexpr uint32_t kBoxOpen = 0x80000000u, kBoxEmpty = 0x7FFFFFFFu;
+
+SG_D uint2 pair_box(const LeafSetup& s, uint32_t c, uint32_t mask) {
+    if (c == 0) return make_uint2(kBoxEmpty, 0u);
+    const uint32_t crx = f2u(s.cres.x), crxy = f2u(s.cres.x * s.cres.y);
+    const uint32_t corner = (uint32_t)s.lo[0] + (uint32_t)s.lo[1] * crx + (uint32_t)s.lo[2] * crxy;
+    if (c > 32u || corner >= 65536u) return make_uint2(kBoxOpen, 0u);
+    return make_uint2(corner | (uint32_t)(s.hp[0] - s.lo[0] - 1) << 16 | (uint32_t)(s.hp[1] - s.lo[1] - 1) << 21 |
+                          (uint32_t)(s.hp[2] - s.lo[2] - 1) << 26,
+                      mask);
+}
+
+// cells of the box (0: empty)
+SG_D uint32_t box_cells(uint32_t x) {
+    if (x >= kBoxEmpty) return 0u;
+    return (((x >> 16) & 31u) + 1u) * (((x >> 21) & 31u) + 1u) * (((x >> 26) & 31u) + 1u);
+}
+
+// f(leaf cell) for every accepted cell of a box that is not open, `first` the
+// tile's index of the top cell's leaf cell 0, res its packed resolution
+template <class F>
+SG_D void box_visit(uint2 box, uint32_t first, uint32_t res, F&& f) {
+    const uint32_t ex = ((box.x >> 16) & 31u) + 1u, ey = ((box.x >> 21) & 31u) + 1u;
+    const uint32_t crx = res & 0xFFu, crxy = crx * ((res >> 8) & 0xFFu);
+    uint32_t row = first + (box.x & 0xFFFFu), y = 0, x = 0;
+    const uint32_t next = crxy - (ey - 1u) * crx;   // from a slice's last row to the next slice's first
+    for (uint32_t m = box.y; m; m >>= 1) {
+        if (m & 1u) f(row + x);
+        if (++x == ex) {
+            x = 0;
+            const bool last = ++y == ey;
+            row += last ? next : crx;
+            y = last ? 0u : y;
+        }
+    }
 }
 
 // Leaf tile of a sorted top pair: tile t holds the top cells that start in
@@ -763,6 +829,7 @@ SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisM
 // records (zero-initialised words, combined with atomicMax):
 //   info[4t+0] = ~first pair   info[4t+1] = end pair
 //   info[4t+2] = ~first leaf key   info[4t+3] = last leaf key + 1
+//   info[4T+t] = 1 when a pair of the tile has an open box
 // and its accepted / rejected leaf-pair totals in sums[t] / sums[Tp + t].
 SG_HD uint32_t leaf_sums_stride(uint32_t T) { return (T + 15u) & ~15u; }
 
@@ -777,7 +844,8 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                                        const uint32_t* __restrict__ cells,
                                                        uint32_t* __restrict__ sums, uint32_t* __restrict__ info,
                                                        uint32_t T, uint32_t* __restrict__ dbg_counts,
-                                                       uint32_t* __restrict__ pacc, uint32_t* __restrict__ prej) {
+                                                       uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
+                                                       uint32_t* __restrict__ prej) {
     constexpr int kSlots = 4;
     __shared__ uint32_t s_acc[kSlots], s_rej[kSlots];
     const uint32_t P1v = h->P1_valid;
@@ -801,7 +869,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
         LeafSetup st;
         const uint32_t c = leaf_pair(t, L, h, key, tri, cells, st);
         if (dbg_counts) dbg_counts[i] = c;
-        uint32_t acc = 0;
+        uint32_t acc = 0, mask = 0;
         bool counted = true;
         if (c) {
             // a box of one leaf cell on some axis has no plane test: every
@@ -812,15 +880,26 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                   (uint32_t)(st.hp[2] - 1) * crxy + st.px;
             if (!plane_tested(st) && kmax < L.C2) {
                 acc = c;
+                mask = c >= 32u ? 0xFFFFFFFFu : (1u << c) - 1u;
             } else {
                 if (wide_box(L, st, c)) {   // k_leaf_scan counts it
                     const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
                     counted = w >= kWideCap;
                     if (!counted) sums[2 * (size_t)Tp + 4 + w] = i;
                 }
-                if (counted) leaf_visit(L, st, [&](uint32_t, bool ok) { acc += ok ? 1u : 0u; });
+                if (counted) {
+                    uint32_t bit = 0;
+                    leaf_visit(L, st, [&](uint32_t, bool ok) {
+                        acc += ok ? 1u : 0u;
+                        mask |= ok && bit < 32u ? 1u << bit : 0u;
+                        ++bit;
+                    });
+                }
             }
         }
+        const uint2 box = pair_box(st, c, mask);
+        boxes[i] = box;
+        if (box.x == kBoxOpen && tile < T) info[4 * (size_t)T + tile] = 1u;
         if (counted && pacc) {   // per-pair totals for the parallel emission of oversize tiles
             pacc[i] = acc;
             prej[i] = c - acc;
@@ -933,8 +1012,14 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
         uint32_t p = run + pre + inc - sum;
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
-            if (i0 + k < T) row[i0 + k] = p;
-            p += v[k];
+            const uint32_t x = v[k];
+            v[k] = p;
+            p += x;
+        }
+        if (i0 + kPer <= Tp) {   // rows are padded to whole groups of kPer
+#pragma unroll
+            for (int q = 0; q < kPer / 4; ++q)
+                reinterpret_cast<uint4*>(row + i0)[q] = make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
         }
         run += tot;
     }
@@ -957,204 +1042,276 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
     }
 }
 
-// One stable LSD pass over n <= kLeafStage words: digit (x >> shift) & (2^db - 1),
-// db <= kDigitBits, in -> out, by a block of kLeafBlock threads.  Ranks within
-// a wave come from ballots over the digit bits (computed once for the digit
-// histogram and again for the scatter, which keeps registers low); waves are
-// ordered through per-wave digit counts, rounds through running bases.
-SG_D void lds_sort_pass(const uint32_t* in, uint32_t* out, uint32_t n, int shift, int db, uint32_t* s_base,
-                        uint32_t* s_wc, uint32_t* s_scan) {
-    constexpr int NW = kLeafBlock / 64;
-    constexpr int RM = 1 << kDigitBits;
-    static_assert(RM * NW <= kLeafBlock, "one zeroing store per thread");
-    const uint32_t R = 1u << db, mask = R - 1u;
-    const int w = wave_id();
-    const uint64_t lt = lanemask_lt();
-    if (threadIdx.x < RM * NW) s_wc[threadIdx.x] = 0;
-    if (threadIdx.x < RM) s_base[threadIdx.x] = 0;
-    __syncthreads();
-    for (uint32_t r0 = 0; r0 < n; r0 += kLeafBlock) {
-        const uint32_t i = r0 + threadIdx.x;
-        const bool ok = i < n;
-        const uint32_t d = ok ? (in[i] >> shift) & mask : 0u;
-        const uint64_t peers = digit_peers(ok, d, db);
-        if (ok && (peers & lt) == 0) atomicAdd(&s_base[d], (uint32_t)__popcll(peers));
-    }
-    __syncthreads();
-    {
-        const uint32_t v = threadIdx.x < R ? s_base[threadIdx.x] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_excl_scan<NW>(v, &tot, s_scan);
-        if (threadIdx.x < R) s_base[threadIdx.x] = ex;
-        __syncthreads();
-    }
-    for (uint32_t r0 = 0; r0 < n; r0 += kLeafBlock) {
-        const uint32_t i = r0 + threadIdx.x;
-        const bool ok = i < n;
-        const uint32_t x = ok ? in[i] : 0u;
-        const uint32_t d = (x >> shift) & mask;
-        const uint64_t peers = digit_peers(ok, d, db);
-        const uint32_t rk = (uint32_t)__popcll(peers & lt);
-        if (ok && rk == 0) s_wc[w * RM + d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (ok) {
-            uint32_t pos = s_base[d] + rk;
-            for (int v = 0; v < w; ++v) pos += s_wc[v * RM + d];
-            out[pos] = x;
-        }
-        __syncthreads();
-        if (threadIdx.x < R) {
-            uint32_t s = 0;
-#pragma unroll
-            for (int v = 0; v < NW; ++v) {
-                s += s_wc[v * RM + threadIdx.x];
-                s_wc[v * RM + threadIdx.x] = 0;
-            }
-            s_base[threadIdx.x] += s;
-        }
-        __syncthreads();
-    }
-}
-
 // Where tile b's pairs go: prefixes from k_leaf_scan, tile bounds and leaf
-// key range from k_leaf_count; `staged` when the tile fits the LDS sort.
+// key range from k_leaf_count, and who emits it.
+enum LeafMode : uint32_t { LEAF_NONE, LEAF_SMALL, LEAF_BIG, LEAF_OVERSIZE };
 struct LeafTilePlan {
-    uint32_t a0, a1, pre_acc, pre_rej, tot_acc, kbase, span;
-    bool staged;
+    uint32_t a0, a1, pre_acc, pre_rej, acc, rej, tot_acc, kbase, span;
+    LeafMode mode;
 };
 
-SG_D bool leaf_tile_plan(const BuildArgs& a, const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info,
+SG_D void leaf_tile_plan(const BuildArgs& a, const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info,
                          uint32_t T, uint32_t b, LeafTilePlan& q) {
     const uint32_t Tp = leaf_sums_stride(T);
     const uint32_t tot_acc = sums[2 * (size_t)Tp], tot_rej = sums[2 * (size_t)Tp + 1];
-    if ((uint64_t)tot_acc + tot_rej > a.cap_P2) return false;   // flagged by k_leaf_scan
+    q.mode = LEAF_NONE;
+    if ((uint64_t)tot_acc + tot_rej > a.cap_P2) return;   // flagged by k_leaf_scan
     const uint4 inf = reinterpret_cast<const uint4*>(info)[b];
-    if (inf.x == 0) return false;   // no top cell starts in this tile
+    if (inf.x == 0) return;   // no top cell starts in this tile
     q.a0 = ~inf.x;
     q.a1 = inf.y > q.a0 ? inf.y : q.a0;
-    if (q.a0 >= q.a1) return false;
+    if (q.a0 >= q.a1) return;
     q.tot_acc = tot_acc;
     q.pre_acc = sums[b];
     q.pre_rej = sums[Tp + b];
-    const uint32_t n_tile = ((b + 1 < T ? sums[b + 1] : tot_acc) - q.pre_acc) +
-                            ((b + 1 < T ? sums[Tp + b + 1] : tot_rej) - q.pre_rej);
+    q.acc = (b + 1 < T ? sums[b + 1] : tot_acc) - q.pre_acc;
+    q.rej = (b + 1 < T ? sums[Tp + b + 1] : tot_rej) - q.pre_rej;
     q.kbase = ~inf.z;
     q.span = inf.w >= q.kbase ? inf.w - q.kbase : 0xFFFFFFFFu;
-    q.staged = n_tile <= kLeafStage && q.span < (1u << kLocalBits) && q.a1 - q.a0 <= (1u << kPayBits);
-    return true;
+    const uint32_t tops = q.a1 - q.a0;
+    if (q.acc <= LeafSmall::pairs && q.span <= LeafSmall::span && tops <= LeafSmall::tops &&
+        info[4 * (size_t)T + b] == 0u)
+        q.mode = LEAF_SMALL;
+    else if (q.acc <= LeafBig::pairs && q.span <= LeafBig::span && tops <= LeafBig::tops)
+        q.mode = LEAF_BIG;
+    else
+        q.mode = LEAF_OVERSIZE;
 }
 
-// tiles that fit the LDS sort
-__global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_leaf_emit(TriSoA t, GridHeader* h, BuildArgs a,
-                                                         const uint32_t* __restrict__ top_keys,
-                                                         const uint32_t* __restrict__ top_vals,
-                                                         const uint32_t* __restrict__ cells,
-                                                         uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                         float* __restrict__ refs,
-                                                         const uint32_t* __restrict__ sums,
-                                                         const uint32_t* __restrict__ info, uint32_t T,
-                                                         uint32_t* __restrict__ leaves, int write_keys) {
-    constexpr int NW = kLeafBlock / 64;
-    __shared__ uint32_t s_scan[NW];
-    __shared__ uint32_t s_a[kLeafStage], s_b[kLeafStage];
-    __shared__ uint32_t s_base[1 << kDigitBits], s_wc[(1 << kDigitBits) * NW];
-    static_assert(kLeafStage >= (1u << kPayBits), "the spare sort buffer holds the tile's triangle ids");
-    LeafTilePlan q;
-    if (!leaf_tile_plan(a, sums, info, T, blockIdx.x, q) || !q.staged) return;
-    const LeafParams L = read_leaf_params(h);
-    const uint32_t a0 = q.a0, a1 = q.a1, kbase = q.kbase, span = q.span;
-    const uint32_t cap = a.cap_P2;
-    const uint32_t rej_base = q.tot_acc + q.pre_rej;
+// 16-bit counters in LDS, two to a word: add one, return the old value
+SG_D uint32_t count_add(uint16_t* s_cnt, uint32_t k) {
+    const uint32_t sh = (k & 1u) * 16u;
+    return (atomicAdd(reinterpret_cast<uint32_t*>(s_cnt) + (k >> 1), 1u << sh) >> sh) & 0xFFFFu;
+}
 
-    // pairs in emission order as (local key << kPayBits | top pair); a
-    // rejected pair takes the local key `span`, after every accepted one
-    uint32_t run = 0, n_acc = 0;
-    for (uint32_t c0 = a0; c0 < a1; c0 += kLeafBlock) {
-        const uint32_t i = c0 + threadIdx.x;
-        LeafSetup s;
-        uint32_t c = 0;
-        if (i < a1) c = leaf_pair(t, L, h, top_keys[i], top_vals[i], cells, s);
+// Exclusive scan of s_cnt[0..span) in place by a block of NW waves, and the
+// ranges of the tile's leaf cells, which no other tile holds: {first, last+1}
+// of its references, {0, 0} without (the leaf cells of empty top cells between
+// the tile's are zero as well); n_ranges of them lie below C2.
+template <int NW>
+SG_D void leaf_scan_counts(uint16_t* s_cnt, uint32_t span, uint32_t first, uint32_t* s_scan,
+                           uint2* __restrict__ ranges, uint32_t n_ranges) {
+    uint32_t run = 0;
+    for (uint32_t k0 = 0; k0 < span; k0 += NW * 128) {   // two cells, one word, per thread
+        const uint32_t k = k0 + 2u * threadIdx.x;
+        const uint32_t w = k < span ? reinterpret_cast<uint32_t*>(s_cnt)[k >> 1] : 0u;
+        const uint32_t n0 = w & 0xFFFFu, n1 = w >> 16;
         uint32_t agg;
-        uint32_t p = run + block_excl_scan<NW>(c, &agg, s_scan);
-        const uint32_t pay = i - a0;
-        if (c)
-            leaf_visit(L, s, [&](uint32_t key, bool ok) {
-                const uint32_t lk = (ok && key >= kbase && key - kbase < span) ? key - kbase : span;
-                n_acc += lk < span ? 1u : 0u;
-                if (p < kLeafStage) s_a[p] = (lk << kPayBits) | pay;
-                ++p;
-            });
+        const uint32_t p = run + block_excl_scan<NW>(n0 + n1, &agg, s_scan);
+        if (k < span) reinterpret_cast<uint32_t*>(s_cnt)[k >> 1] = p | (p + n0) << 16;
+        const uint32_t f = first + p;
+        if (k < n_ranges && k < span) ranges[k] = n0 ? make_uint2(f, f + n0) : make_uint2(0u, 0u);
+        if (k + 1u < n_ranges && k + 1u < span)
+            ranges[k + 1u] = n1 ? make_uint2(f + n0, f + n0 + n1) : make_uint2(0u, 0u);
         run += agg;
     }
-    const uint32_t acc_t = block_sum<NW>(n_acc, s_scan);   // syncs: staging complete
-    const uint32_t n = run < kLeafStage ? run : kLeafStage;
-    const int bits = 32 - __builtin_clz(span | 1u);   // local keys 0..span
-    const int passes = (bits + kDigitBits - 1) / kDigitBits;
-    const int db = (bits + passes - 1) / passes;
-    uint32_t* src = s_a;
-    uint32_t* dst = s_b;
-    for (int k = 0, lo = 0; k < passes; ++k, lo += db) {
-        lds_sort_pass(src, dst, n, kPayBits + lo, min(db, bits - lo), s_base, s_wc, s_scan);
-        uint32_t* tmp = src;
-        src = dst;
-        dst = tmp;
-    }
-    // the triangle of each top pair of the tile, in the sort buffer the last
-    // pass read (free now): the write-out reads it there instead of gathering
-    // it from the sorted top pairs.  Sharing the buffer keeps the block's LDS
-    // at 35 KB, four blocks per CU.
-    uint32_t* s_tri = dst;
-    for (uint32_t j = threadIdx.x; j < a1 - a0; j += kLeafBlock) s_tri[j] = top_vals[a0 + j];
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < n; j += kLeafBlock) {
-        const uint32_t x = src[j];
-        const uint32_t v = s_tri[x & ((1u << kPayBits) - 1u)];
-        const uint32_t lk = x >> kPayBits;
-        uint32_t idx, key;
-        if (j < acc_t) {
-            idx = q.pre_acc + j;
-            key = kbase + lk;
-        } else {
-            idx = rej_base + (j - acc_t);
-            key = L.C2;
+}
+
+// The lists of the tile's leaf cells, s_ord[end of cell k-1 .. end of cell k)
+// with the ends in s_end (s_ord begins with cell k0, at place `base`), were
+// filled by LDS atomics, so their order is any;
+// the canonical order is top pairs ascending.  Entry j of the lists holds x =
+// (leaf cell << kTopBits | top pair); its place among the tile's accepted pairs
+// is the start of its cell's list and the number of smaller entries in it:
+// as many LDS reads as the list is long, U in flight, all lanes at once (a
+// height field's lists hold 10 on average; sorting them in place, a lane or a
+// wave to a list, left the other lanes waiting: 27 % of the kernel).  Lists
+// beyond kLongList are sorted first, by leaf_sort_long.
+constexpr uint32_t kLongList = 192;
+template <uint32_t U>
+SG_D uint32_t leaf_place(const uint32_t* s_ord, const uint16_t* s_end, uint32_t x, uint32_t j, uint32_t k0,
+                         uint32_t base) {
+    const uint32_t k = x >> kTopBits;
+    const uint32_t st = k > k0 ? s_end[k - 1] - base : 0u, en = s_end[k] - base;
+    if (en - st > kLongList) return j;
+    uint32_t rank = 0;
+    for (uint32_t i = st; i < en; i += U) {
+        uint32_t v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) v[u] = s_ord[min(i + u, en - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) rank += i + u < en && v[u] < x ? 1u : 0u;
+    }
+    return st + rank;
+}
+
+// a wave sorts each long list of the leaf cells [k0, k1) with a bitmap over the tile's top pairs (bm, the
+// wave's own `words` words)
+template <int NW>
+SG_D void leaf_sort_long(uint32_t* s_ord, const uint16_t* s_end, uint32_t k0, uint32_t k1, uint32_t base, uint32_t* bm,
+                         uint32_t words) {
+    const uint32_t l = (uint32_t)lane_id();
+    for (uint32_t c0 = k0; c0 < k1; c0 += NW * 64) {
+        const uint32_t k = c0 + threadIdx.x;
+        const uint32_t st = k < k1 && k > k0 ? s_end[k - 1] - base : 0u, n = k < k1 ? s_end[k] - base - st : 0u;
+        for (uint64_t big = __ballot(n > kLongList); big; big &= big - 1) {
+            const int L = __ffsll((long long)big) - 1;
+            const uint32_t lst = (uint32_t)__builtin_amdgcn_readlane((int)st, L),
+                           ln = (uint32_t)__builtin_amdgcn_readlane((int)n, L),
+                           hi = (uint32_t)__builtin_amdgcn_readlane((int)k, L) << kTopBits;
+            for (uint32_t w = l; w < words; w += 64) bm[w] = 0;
+            __threadfence_block();
+            for (uint32_t i = l; i < ln; i += 64) {
+                const uint32_t v = s_ord[lst + i] & ((1u << kTopBits) - 1u);
+                if ((v >> 5) < words) atomicOr(&bm[v >> 5], 1u << (v & 31u));
+            }
+            __threadfence_block();
+            uint32_t run = lst;
+            for (uint32_t w0 = 0; w0 < words; w0 += 64) {
+                const uint32_t w = w0 + l;
+                uint32_t m = w < words ? bm[w] : 0u;
+                const uint32_t c = (uint32_t)__popc(m), inc = wave_incl_scan(c);
+                uint32_t p = run + inc - c;
+                for (; m; m &= m - 1u) s_ord[p++] = hi | (32u * w + (uint32_t)__ffs((int)m) - 1u);
+                run += (uint32_t)__shfl((int)inc, 63, 64);
+            }
+            __threadfence_block();
         }
-        if (idx < cap) {
-            if (write_keys) keys[idx] = key;
-            vals[idx] = v;
-            if (j < acc_t) {
-                // accepted pairs are at their final slots: their reference
-                // records too (the tile's triangles were read while staging)
-                write_ref_record(refs, idx, t.rec, v, L.n_tris);
-                // and the ranges of the tile's leaf cells, which no other
-                // tile holds: {first, last + 1} of each key, as k_ranges
-                // writes them from the sorted keys
-                if (leaves) {
-                    if (j == 0 || (src[j - 1] >> kPayBits) != lk) leaves[2 * (size_t)key] = idx;
-                    if (j + 1 == acc_t || (src[j + 1] >> kPayBits) != lk) leaves[2 * (size_t)key + 1] = idx + 1u;
-                }
+    }
+    __syncthreads();
+}
+
+// the rejected pairs of one top pair, from slot r of the tail
+SG_D void leaf_reject(uint32_t r, uint32_t n, uint32_t tri, uint32_t cap, uint32_t C2, uint32_t* __restrict__ keys,
+                      uint32_t* __restrict__ vals, int write_keys) {
+    for (; n && r < cap; --n, ++r) {
+        if (write_keys) keys[r] = C2;
+        vals[r] = tri;
+    }
+}
+
+// Tiles that fit LeafSmall.  Each pair's box comes from k_leaf_count, so a
+// tile is a counting sort of its accepted cells: LDS counts, one scan, LDS
+// lists.  2,093,058-triangle height field, 6.6 M references: 139 us for 433 MB
+// (3.1 TB/s; the reference records alone are 239 MB), VALU busy for half of
+// it, the rest waiting for memory in the first loads (36 % of a block's time)
+// and the write-out (40 %).  The form before it, a stable two-pass LDS radix
+// sort of staged pairs with the boxes formed again from the gathered
+// triangles, took 174 us.  Two pairs per lane in the write-out, so that their
+// gathers overlap, changed nothing.
+SG_D void leaf_emit_small(const LeafTilePlan& q, const uint2* __restrict__ boxes, const TriSoA& t, uint32_t n_tris,
+                          uint32_t C1, uint32_t C2, uint32_t cap, const uint32_t* __restrict__ top_keys,
+                          const uint32_t* __restrict__ top_vals, const uint32_t* __restrict__ cells,
+                          uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
+                          uint32_t* __restrict__ leaves, int write_keys, uint16_t* s_cnt, uint32_t* s_ord,
+                          uint32_t* s_tri, uint32_t* s_bm, uint32_t* s_scan) {
+    constexpr int NW = kLeafBlock / 64;
+    constexpr int R = LeafSmall::tops / kLeafBlock;   // rounds; a tile rarely needs more than two
+    for (uint32_t k = threadIdx.x; 2u * k < q.span; k += kLeafBlock) reinterpret_cast<uint32_t*>(s_cnt)[k] = 0;
+    const uint32_t tops = q.a1 - q.a0;
+    uint2 box[R];
+    uint32_t first[R], res[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const uint32_t i = q.a0 + (uint32_t)j * kLeafBlock + threadIdx.x;
+        box[j] = make_uint2(kBoxEmpty, 0u);
+        first[j] = res[j] = 0;
+        if (i < q.a1) {
+            const uint32_t key = top_keys[i];
+            const uint2 bx = boxes[i];
+            s_tri[i - q.a0] = top_vals[i];
+            if (key < C1) {
+                const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
+                box[j] = bx;
+                first[j] = cl.x - q.kbase;
+                res[j] = cl.y;
             }
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if ((uint32_t)j * kLeafBlock >= tops) break;
+        box_visit(box[j], first[j], res[j], [&](uint32_t k) {
+            if (k < q.span) count_add(s_cnt, k);
+        });
+    }
+    if (q.rej) {
+        uint32_t run = q.tot_acc + q.pre_rej;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            if ((uint32_t)j * kLeafBlock >= tops) break;
+            const uint32_t n = box_cells(box[j].x) - (uint32_t)__popc(box[j].y);
+            uint32_t agg;
+            const uint32_t r = run + block_excl_scan<NW>(n, &agg, s_scan);
+            if (n) leaf_reject(r, n, s_tri[(uint32_t)j * kLeafBlock + threadIdx.x], cap, C2, keys, vals, write_keys);
+            run += agg;
+        }
+    }
+    __syncthreads();
+    leaf_scan_counts<NW>(s_cnt, q.span, q.pre_acc, s_scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
+                         leaves && C2 > q.kbase ? C2 - q.kbase : 0u);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if ((uint32_t)j * kLeafBlock >= tops) break;
+        box_visit(box[j], first[j], res[j], [&](uint32_t k) {
+            if (k < q.span) {
+                const uint32_t p = count_add(s_cnt, k);
+                if (p < LeafSmall::pairs) s_ord[p] = k << kTopBits | ((uint32_t)j * kLeafBlock + threadIdx.x);
+            }
+        });
+    }
+    __syncthreads();
+    leaf_sort_long<NW>(s_ord, s_cnt, 0, q.span, 0, s_bm + LeafSmall::tops / 32 * wave_id(), LeafSmall::tops / 32);
+    // [0, acc) of s_ord is filled: every accepted cell was counted and listed
+    for (uint32_t j = threadIdx.x; j < q.acc; j += kLeafBlock) {
+        const uint32_t x = s_ord[j];
+        if ((x >> kTopBits) >= q.span) continue;
+        const uint32_t idx = q.pre_acc + leaf_place<4>(s_ord, s_cnt, x, j, 0, 0);
+        const uint32_t tri = s_tri[min(x & ((1u << kTopBits) - 1u), tops - 1u)];
+        if (idx >= cap) continue;
+        if (write_keys) keys[idx] = q.kbase + (x >> kTopBits);
+        vals[idx] = tri;
+        write_ref_record(refs, idx, t.rec, tri, n_tris);
+    }
 }
 
-// One stable LSD pass by a block of kBlock threads over n (key, value)
+// items receives the work of the larger kernel (tile | slice << kSliceShift),
+// *todo its number
+__global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_leaf_emit(
+    TriSoA t, GridHeader* h, BuildArgs a, const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
+    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, uint32_t* __restrict__ keys,
+    uint32_t* __restrict__ vals, float* __restrict__ refs, const uint32_t* __restrict__ sums,
+    const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves, int write_keys, int large,
+    uint32_t* __restrict__ todo, uint32_t* __restrict__ items) {
+    constexpr int NW = kLeafBlock / 64;
+    __shared__ uint32_t s_scan[NW], s_ord[LeafSmall::pairs], s_tri[LeafSmall::tops];
+    __shared__ uint32_t s_bm[LeafSmall::tops / 32 * NW];
+    __shared__ __align__(4) uint16_t s_cnt[LeafSmall::span];
+    LeafTilePlan q;
+    leaf_tile_plan(a, sums, info, T, blockIdx.x, q);
+    if (q.mode != LEAF_SMALL) {
+        // oversize tiles of a grid with the parallel emission are its
+        const uint32_t n = q.mode == LEAF_BIG ? max(1u, (q.acc + kLeafSlice - 1u) / kLeafSlice)
+                                              : (q.mode == LEAF_OVERSIZE && !large ? 1u : 0u);
+        if (threadIdx.x == 0 && n) {
+            const uint32_t at = atomicAdd(todo, n);
+            for (uint32_t j = 0; j < n; ++j) items[at + j] = blockIdx.x | j << kSliceShift;
+        }
+        return;
+    }
+    leaf_emit_small(q, boxes, t, h->n_tris, h->C1, h->C2, a.cap_P2, top_keys, top_vals, cells, keys, vals, refs, leaves,
+                    write_keys, s_cnt, s_ord, s_tri, s_bm, s_scan);
+}
+
+// One stable LSD pass by a block of kBigBlock threads over n (key, value)
 // pairs in global memory: digit ((k - kbase) >> shift) & (2^db - 1), db <= 8,
 // (k, v) -> (ko, vo).  Ranks as lds_sort_pass: a digit histogram, its scan,
-// then rounds of kBlock pairs ranked by wave ballots and ordered across
+// then rounds of kBigBlock pairs ranked by wave ballots and ordered across
 // waves by per-wave digit counts.
-static_assert(kBlock == 256, "one digit bin per thread");
 SG_D void block_sort_pass_global(const uint32_t* k, const uint32_t* v, uint32_t* ko, uint32_t* vo, uint32_t n,
                                  uint32_t kbase, int shift, int db, uint32_t* s_base, uint32_t* s_wc,
                                  uint32_t* s_scan) {
-    constexpr int NW = kBlock / 64;
+    constexpr int NW = kBigBlock / 64;
     constexpr int RM = 256;
     const uint32_t R = 1u << db, mask = R - 1u;
     const int w = wave_id();
     const uint64_t lt = lanemask_lt();
-    for (uint32_t j = threadIdx.x; j < RM * NW; j += kBlock) s_wc[j] = 0;
-    s_base[threadIdx.x] = 0;   // kBlock == RM
+    for (uint32_t j = threadIdx.x; j < RM * NW; j += kBigBlock) s_wc[j] = 0;
+    if (threadIdx.x < RM) s_base[threadIdx.x] = 0;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += kBlock) atomicAdd(&s_base[((k[i] - kbase) >> shift) & mask], 1u);
+    for (uint32_t i = threadIdx.x; i < n; i += kBigBlock) atomicAdd(&s_base[((k[i] - kbase) >> shift) & mask], 1u);
     __syncthreads();
     {
         const uint32_t c = threadIdx.x < R ? s_base[threadIdx.x] : 0u;
@@ -1163,7 +1320,7 @@ SG_D void block_sort_pass_global(const uint32_t* k, const uint32_t* v, uint32_t*
         if (threadIdx.x < R) s_base[threadIdx.x] = ex;
         __syncthreads();
     }
-    for (uint32_t r0 = 0; r0 < n; r0 += kBlock) {
+    for (uint32_t r0 = 0; r0 < n; r0 += kBigBlock) {
         const uint32_t i = r0 + threadIdx.x;
         const bool ok = i < n;
         const uint32_t x = ok ? k[i] : 0u, y = ok ? v[i] : 0u;
@@ -1192,130 +1349,279 @@ SG_D void block_sort_pass_global(const uint32_t* k, const uint32_t* v, uint32_t*
     }
 }
 
-// Tiles too large for LDS (more than kLeafStage pairs, or a local key range
-// or top-pair count beyond the LDS sort's bit budget) of a grid without the
-// parallel emission: one block emits such a tile's pairs in emission order,
-// sorts its accepted pairs (stable LSD passes over the tile-local key,
-// ping-ponging with tk / tv) and writes their reference records -- correct but
-// slow, for a rebuild that meets an oversize tile the grid's build never met.
-// A block looks after kOverTiles tiles: most rebuilds find none oversize, and
-// a block for each tile is then 8,000 blocks that only start and end.
-// GridHeader::oversize counts the tiles.
-constexpr uint32_t kOverTiles = 16;
-__global__ __launch_bounds__(kBlock) void k_leaf_emit_large(TriSoA t, GridHeader* h, BuildArgs a,
-                                                            const uint32_t* __restrict__ top_keys,
-                                                            const uint32_t* __restrict__ top_vals,
-                                                            const uint32_t* __restrict__ cells,
-                                                            uint32_t* __restrict__ keys,
-                                                            uint32_t* __restrict__ vals,
-                                                            const uint32_t* __restrict__ sums,
-                                                            const uint32_t* __restrict__ info, uint32_t T,
-                                                            uint32_t* __restrict__ tk, uint32_t* __restrict__ tv, float* __restrict__ refs,
-                                                            uint32_t* __restrict__ leaves) {
-    __shared__ uint32_t s_scan[kBlock / 64];
-    __shared__ uint32_t s_base[256], s_wc[256 * (kBlock / 64)];
-    __shared__ uint32_t s_wide[kBlock], s_wacc[kBlock], s_wrej[kBlock], s_wcnt[kBlock], s_nwide;
-    __shared__ float s_tab[3][kAxisMax];
-    __shared__ uint32_t s_over;
-    LeafTilePlan q;
-    if (threadIdx.x < 64) {   // which of the block's tiles are oversize
-        const uint32_t b = blockIdx.x * kOverTiles + threadIdx.x;
-        const uint64_t m = __ballot(threadIdx.x < kOverTiles && b < T && leaf_tile_plan(a, sums, info, T, b, q) && !q.staged);
-        if (threadIdx.x == 0) s_over = (uint32_t)m;
+// LDS of k_leaf_emit_big: a tile's counts and lists, or the digit counts of a
+// tile sorted in global memory
+struct BigLds {
+    union {
+        struct {
+            uint32_t ord[kLeafSlice + LeafBig::tops];   // a list is no longer than the tile's top pairs
+            uint16_t cnt[LeafBig::span];
+        };
+        struct {
+            uint32_t base[256], wc[256 * (kBigBlock / 64)];
+        };
+    };
+    union {
+        uint32_t bm[LeafBig::tops / 32 * (kBigBlock / 64)];   // leaf_sort_long, after the lists are filled
+        struct {
+            uint32_t wide[kBigBlock], wacc[kBigBlock], wrej[kBigBlock], wcnt[kBigBlock];
+        };
+    };
+    float tab[3][kAxisMax];
+    uint32_t scan[kBigBlock / 64];
+    uint32_t n_wide, k0, k1;
+};
+
+// A slice of a tile that fits LeafBig: as leaf_emit_small, its top pairs in
+// rounds, open boxes visited again, wide ones by the block.  Slice 0 also
+// writes the rejected pairs and the leaf ranges.  200,000-triangle sphere (12
+// such tiles, the largest of 20,456 accepted pairs): one block per tile 147
+// us, in slices 84 us (two fifths counting, one fifth listing); the global
+// sort and range passes that such tiles needed before took 130 us.
+SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams& L, GridHeader* h, const uint2* __restrict__ boxes,
+                        const TriSoA& t, uint32_t cap, const uint32_t* __restrict__ top_keys,
+                        const uint32_t* __restrict__ top_vals, const uint32_t* __restrict__ cells,
+                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
+                        uint32_t* __restrict__ leaves, int write_keys, BigLds& s) {
+    constexpr int NW = kBigBlock / 64;
+    for (uint32_t k = threadIdx.x; 2u * k < q.span; k += kBigBlock) reinterpret_cast<uint32_t*>(s.cnt)[k] = 0;
+    uint32_t run = q.tot_acc + q.pre_rej, k0 = 0, k1 = q.span, base = 0;
+    if (threadIdx.x == 0) s.k0 = s.k1 = q.span;
+    // pass 0 counts and writes the rejected pairs, pass 1 fills the lists
+    for (int pass = 0; pass < 2; ++pass) {
+        for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBigBlock) {
+            __syncthreads();
+            if (threadIdx.x == 0) s.n_wide = 0;
+            __syncthreads();
+            const uint32_t i = c0 + threadIdx.x;
+            uint32_t rej = 0, tri = 0;
+            // a leaf cell of the tile that pair p lies in
+            auto add = [&](uint32_t k, uint32_t p) {
+                if (k < k0 || k >= k1) return;
+                const uint32_t at = count_add(s.cnt, k) - base;
+                if (pass && at < kLeafSlice + LeafBig::tops) s.ord[at] = k << kTopBits | (p - q.a0);
+            };
+            if (i < q.a1) {
+                const uint32_t key = top_keys[i];
+                tri = top_vals[i];
+                const uint2 box = key < L.C1 ? boxes[i] : make_uint2(kBoxEmpty, 0u);
+                if (box.x == kBoxOpen) {
+                    LeafSetup st;
+                    const uint32_t c = leaf_pair(t, L, h, key, tri, cells, st);
+                    if (wide_box(L, st, c)) {
+                        s.wide[atomicAdd(&s.n_wide, 1u)] = threadIdx.x;
+                    } else if (c) {
+                        leaf_visit(L, st, [&](uint32_t k, bool ok) {
+                            if (ok) add(k - q.kbase, i);
+                            else ++rej;
+                        });
+                    }
+                } else if (box.x != kBoxEmpty) {
+                    const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
+                    box_visit(box, cl.x - q.kbase, cl.y, [&](uint32_t k) { add(k, i); });
+                    rej = box_cells(box.x) - (uint32_t)__popc(box.y);
+                }
+            }
+            __syncthreads();
+            const uint32_t n_wide = s.n_wide;
+            for (uint32_t w = 0; w < n_wide; ++w) {
+                const uint32_t p = c0 + s.wide[w];
+                LeafSetup st;
+                const uint32_t c = leaf_pair(t, L, h, top_keys[p], top_vals[p], cells, st);
+                uint32_t acc = 0;
+                wide_visit(L, st, s.tab, [&](bool, uint32_t key0, int xa, int xb) {
+                    for (int x = xa; x < xb; ++x) add(key0 + (uint32_t)x - q.kbase, p);
+                    acc += (uint32_t)(xb - xa);
+                });
+                acc = block_sum<NW>(acc, s.scan);
+                if (threadIdx.x == s.wide[w]) rej = c - acc;
+            }
+            if (pass || slice || !q.rej) continue;
+            uint32_t agg;
+            const uint32_t r = run + block_excl_scan<NW>(rej, &agg, s.scan);
+            run += agg;
+            if (rej < kWideBox / 2) {
+                leaf_reject(r, rej, tri, cap, L.C2, keys, vals, write_keys);
+            } else {
+                s.wacc[threadIdx.x] = r;
+                s.wrej[threadIdx.x] = rej;
+                s.wcnt[threadIdx.x] = tri;
+            }
+            // long runs of rejected pairs by the whole block
+            __syncthreads();
+            if (threadIdx.x == 0) s.n_wide = 0;
+            __syncthreads();
+            if (rej >= kWideBox / 2) s.wide[atomicAdd(&s.n_wide, 1u)] = threadIdx.x;
+            __syncthreads();
+            for (uint32_t w = 0; w < s.n_wide; ++w) {
+                const uint32_t o = s.wide[w];
+                for (uint32_t j = threadIdx.x; j < s.wrej[o]; j += kBigBlock)
+                    leaf_reject(s.wacc[o] + j, 1u, s.wcnt[o], cap, L.C2, keys, vals, write_keys);
+            }
+        }
+        __syncthreads();
+        if (pass == 0) {
+            leaf_scan_counts<NW>(s.cnt, q.span, q.pre_acc, s.scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
+                                 leaves && slice == 0 && L.C2 > q.kbase ? L.C2 - q.kbase : 0u);
+            // the slice's leaf cells [k0, k1) and the place of its first pair
+            for (uint32_t k = threadIdx.x; k < q.span; k += kBigBlock) {
+                const uint32_t at = s.cnt[k], lo = slice * kLeafSlice, hi = lo + kLeafSlice;
+                const bool start = k == 0u;
+                const uint32_t before = start ? 0u : s.cnt[k - 1u];
+                if (at >= lo && (start || before < lo)) s.k0 = k;
+                if (at >= hi && (start || before < hi)) s.k1 = k;
+            }
+            __syncthreads();
+            k0 = s.k0;
+            k1 = s.k1;
+            base = k0 < q.span ? s.cnt[k0] : q.acc;
+        }
     }
     __syncthreads();
+    if (k0 >= k1) return;
+    leaf_sort_long<NW>(s.ord, s.cnt, k0, k1, base, s.bm + LeafBig::tops / 32 * wave_id(), (q.a1 - q.a0 + 31u) / 32u);
+    const uint32_t n = min((uint32_t)s.cnt[k1 - 1u] - base, kLeafSlice + LeafBig::tops);
+    for (uint32_t j = threadIdx.x; j < n; j += kBigBlock) {
+        const uint32_t x = s.ord[j];
+        if ((x >> kTopBits) >= q.span) continue;
+        const uint32_t idx = q.pre_acc + base + leaf_place<8>(s.ord, s.cnt, x, j, k0, base);
+        const uint32_t tri = top_vals[min(q.a0 + (x & (LeafBig::tops - 1u)), q.a1 - 1u)];
+        if (idx >= cap) continue;
+        if (write_keys) keys[idx] = q.kbase + (x >> kTopBits);
+        vals[idx] = tri;
+        write_ref_record(refs, idx, t.rec, tri, L.n_tris);
+    }
+}
+
+// An oversize tile of a grid without the parallel emission: the block emits
+// the tile's pairs in emission order, sorts its accepted pairs (stable LSD
+// passes over the tile-local key, ping-ponging with tk / tv) and writes their
+// reference records and leaf ranges -- correct but slow, for a rebuild that
+// meets an oversize tile the grid's build never met.
+SG_D void leaf_emit_oversize(const LeafTilePlan& q, const LeafParams& L, GridHeader* h, const TriSoA& t, uint32_t cap,
+                             const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
+                             const uint32_t* __restrict__ cells, uint32_t* __restrict__ keys,
+                             uint32_t* __restrict__ vals, uint32_t* __restrict__ tk, uint32_t* __restrict__ tv,
+                             float* __restrict__ refs, uint32_t* __restrict__ leaves, BigLds& s_) {
+    uint32_t *s_scan = s_.scan, *s_base = s_.base, *s_wc = s_.wc, *s_wide = s_.wide, *s_wacc = s_.wacc,
+             *s_wrej = s_.wrej, *s_wcnt = s_.wcnt;
+    uint32_t& s_nwide = s_.n_wide;
+    float(*s_tab)[kAxisMax] = s_.tab;
+    const uint32_t rej_base = q.tot_acc + q.pre_rej;
+    if (threadIdx.x == 0) atomicAdd(&h->oversize, 1u);
+    for (uint32_t k = threadIdx.x; k < q.span && q.span != 0xFFFFFFFFu; k += kBigBlock)
+        if (q.kbase + k < L.C2) reinterpret_cast<uint2*>(leaves)[q.kbase + k] = make_uint2(0u, 0u);
+    uint32_t run_acc = 0, run_rej = 0;
+    for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBigBlock) {
+        const uint32_t i = c0 + threadIdx.x;
+        LeafSetup s;
+        uint32_t tri = 0, c = 0, ca = 0;
+        bool wide = false;
+        if (threadIdx.x == 0) s_nwide = 0;
+        __syncthreads();
+        if (i < q.a1) {
+            tri = top_vals[i];
+            c = leaf_pair(t, L, h, top_keys[i], tri, cells, s);
+            wide = wide_box(L, s, c);
+            if (wide) s_wide[atomicAdd(&s_nwide, 1u)] = threadIdx.x;
+            else if (c) leaf_visit(L, s, [&](uint32_t, bool ok) { ca += ok ? 1u : 0u; });
+        }
+        __syncthreads();
+        const uint32_t nwide = s_nwide;
+        for (uint32_t k = 0; k < nwide; ++k) {
+            LeafSetup ws;
+            const uint32_t pair = c0 + s_wide[k];
+            leaf_pair(t, L, h, top_keys[pair], top_vals[pair], cells, ws);
+            const uint32_t acc = wide_count<kBigBlock / 64>(L, ws, s_tab, s_scan);
+            if (threadIdx.x == s_wide[k]) ca = acc;
+        }
+        uint32_t agg_a, agg_r;
+        uint32_t pa = q.pre_acc + run_acc + block_excl_scan<kBigBlock / 64>(ca, &agg_a, s_scan);
+        uint32_t pr = rej_base + run_rej + block_excl_scan<kBigBlock / 64>(c - ca, &agg_r, s_scan);
+        if (wide) {
+            s_wacc[threadIdx.x] = pa;
+            s_wrej[threadIdx.x] = pr;
+            s_wcnt[threadIdx.x] = ca;
+        } else if (c) {
+            leaf_visit(L, s, [&](uint32_t key, bool ok) {
+                const uint32_t idx = ok ? pa++ : pr++;
+                if (idx < cap) {
+                    keys[idx] = ok ? key : L.C2;
+                    vals[idx] = tri;
+                }
+            });
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < nwide; ++k) {
+            LeafSetup ws;
+            const uint32_t w = s_wide[k], pair = c0 + w, wtri = top_vals[pair];
+            const uint32_t wc = leaf_pair(t, L, h, top_keys[pair], wtri, cells, ws);
+            wide_emit<kBigBlock / 64>(L, ws, s_tab, s_scan, wtri, s_wacc[w], s_wrej[w], wc - s_wcnt[w], cap, keys, vals);
+        }
+        __syncthreads();   // the lists are free for the next chunk
+        run_acc += agg_a;
+        run_rej += agg_r;
+    }
+    // the accepted pairs of this tile: [pre_acc, pre_acc + run_acc), keys in
+    // [kbase, kbase + span) (leaf_tile_plan guarantees pre_acc + run_acc <= cap)
+    __threadfence_block();
+    __syncthreads();
+    const uint32_t n = run_acc;
+    uint32_t* k0 = keys + q.pre_acc;
+    uint32_t* v0 = vals + q.pre_acc;
+    uint32_t* k1 = tk + q.pre_acc;
+    uint32_t* v1 = tv + q.pre_acc;
+    const uint32_t span = q.span == 0xFFFFFFFFu ? 0xFFFFFFFFu : q.span;
+    const int bits = 32 - __builtin_clz(span | 1u);
+    const int passes = (bits + 7) / 8;
+    const int db = (bits + passes - 1) / passes;
+    for (int p = 0, lo = 0; p < passes; ++p, lo += db) {
+        if (p & 1) block_sort_pass_global(k1, v1, k0, v0, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
+        else block_sort_pass_global(k0, v0, k1, v1, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
+        __threadfence_block();
+        __syncthreads();
+    }
+    if (passes & 1) {
+        for (uint32_t i = threadIdx.x; i < n; i += kBigBlock) {
+            k0[i] = k1[i];
+            v0[i] = v1[i];
+        }
+    }
+    for (uint32_t i = threadIdx.x; i < n; i += kBigBlock)
+        write_ref_record(refs, q.pre_acc + i, t.rec, (passes & 1) ? v1[i] : v0[i], L.n_tris);
+    // the ranges of the tile's leaf cells from its sorted keys (as k_leaf_emit)
+    __threadfence_block();
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += kBigBlock) {
+        const uint32_t key = k0[i];
+        if (i == 0 || k0[i - 1] != key) leaves[2 * (size_t)key] = q.pre_acc + i;
+        if (i + 1 == n || k0[i + 1] != key) leaves[2 * (size_t)key + 1] = q.pre_acc + i + 1u;
+    }
+}
+
+// the work k_leaf_emit left, an item per block; most builds have none
+constexpr uint32_t kBigBlocks = 256;
+__global__ __launch_bounds__(kBigBlock) void k_leaf_emit_big(
+    TriSoA t, GridHeader* h, BuildArgs a, const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
+    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, uint32_t* __restrict__ keys,
+    uint32_t* __restrict__ vals, float* __restrict__ refs, const uint32_t* __restrict__ sums,
+    const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves, int write_keys,
+    const uint32_t* __restrict__ todo, const uint32_t* __restrict__ items, uint32_t* __restrict__ tk,
+    uint32_t* __restrict__ tv) {
+    __shared__ BigLds s;
+    const uint32_t n = min(*todo, kSlicesMax * T);
+    if (blockIdx.x >= n) return;
     const LeafParams L = read_leaf_params(h);
-    const uint32_t cap = a.cap_P2;
-    for (uint32_t todo = s_over; todo; todo &= todo - 1u) {
-        leaf_tile_plan(a, sums, info, T, blockIdx.x * kOverTiles + (uint32_t)__ffs((int)todo) - 1u, q);
-        const uint32_t rej_base = q.tot_acc + q.pre_rej;
-        if (threadIdx.x == 0) atomicAdd(&h->oversize, 1u);
-        uint32_t run_acc = 0, run_rej = 0;
-        for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBlock) {
-            const uint32_t i = c0 + threadIdx.x;
-            LeafSetup s;
-            uint32_t tri = 0, c = 0, ca = 0;
-            bool wide = false;
-            if (threadIdx.x == 0) s_nwide = 0;
-            __syncthreads();
-            if (i < q.a1) {
-                tri = top_vals[i];
-                c = leaf_pair(t, L, h, top_keys[i], tri, cells, s);
-                wide = wide_box(L, s, c);
-                if (wide) s_wide[atomicAdd(&s_nwide, 1u)] = threadIdx.x;
-                else if (c) leaf_visit(L, s, [&](uint32_t, bool ok) { ca += ok ? 1u : 0u; });
-            }
-            __syncthreads();
-            const uint32_t nwide = s_nwide;
-            for (uint32_t k = 0; k < nwide; ++k) {
-                LeafSetup ws;
-                const uint32_t pair = c0 + s_wide[k];
-                leaf_pair(t, L, h, top_keys[pair], top_vals[pair], cells, ws);
-                const uint32_t acc = wide_count<kBlock / 64>(L, ws, s_tab, s_scan);
-                if (threadIdx.x == s_wide[k]) ca = acc;
-            }
-            uint32_t agg_a, agg_r;
-            uint32_t pa = q.pre_acc + run_acc + block_excl_scan<kBlock / 64>(ca, &agg_a, s_scan);
-            uint32_t pr = rej_base + run_rej + block_excl_scan<kBlock / 64>(c - ca, &agg_r, s_scan);
-            if (wide) {
-                s_wacc[threadIdx.x] = pa;
-                s_wrej[threadIdx.x] = pr;
-                s_wcnt[threadIdx.x] = ca;
-            } else if (c) {
-                leaf_visit(L, s, [&](uint32_t key, bool ok) {
-                    const uint32_t idx = ok ? pa++ : pr++;
-                    if (idx < cap) {
-                        keys[idx] = ok ? key : L.C2;
-                        vals[idx] = tri;
-                    }
-                });
-            }
-            __syncthreads();
-            for (uint32_t k = 0; k < nwide; ++k) {
-                LeafSetup ws;
-                const uint32_t w = s_wide[k], pair = c0 + w, wtri = top_vals[pair];
-                const uint32_t wc = leaf_pair(t, L, h, top_keys[pair], wtri, cells, ws);
-                wide_emit(L, ws, s_tab, s_scan, wtri, s_wacc[w], s_wrej[w], wc - s_wcnt[w], cap, keys, vals);
-            }
-            __syncthreads();   // the lists are free for the next chunk
-            run_acc += agg_a;
-            run_rej += agg_r;
-        }
-        // the accepted pairs of this tile: [pre_acc, pre_acc + run_acc), keys in
-        // [kbase, kbase + span) (leaf_tile_plan guarantees pre_acc + run_acc <= cap)
-        __threadfence_block();
-        __syncthreads();
-        const uint32_t n = run_acc;
-        uint32_t* k0 = keys + q.pre_acc;
-        uint32_t* v0 = vals + q.pre_acc;
-        uint32_t* k1 = tk + q.pre_acc;
-        uint32_t* v1 = tv + q.pre_acc;
-        const uint32_t span = q.span == 0xFFFFFFFFu ? 0xFFFFFFFFu : q.span;
-        const int bits = 32 - __builtin_clz(span | 1u);
-        const int passes = (bits + 7) / 8;
-        const int db = (bits + passes - 1) / passes;
-        for (int p = 0, lo = 0; p < passes; ++p, lo += db) {
-            if (p & 1) block_sort_pass_global(k1, v1, k0, v0, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
-            else block_sort_pass_global(k0, v0, k1, v1, n, q.kbase, lo, min(db, bits - lo), s_base, s_wc, s_scan);
-            __threadfence_block();
-            __syncthreads();
-        }
-        if (passes & 1) {
-            for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
-                k0[i] = k1[i];
-                v0[i] = v1[i];
-            }
-        }
-        for (uint32_t i = threadIdx.x; i < n; i += kBlock)
-            write_ref_record(refs, q.pre_acc + i, t.rec, (passes & 1) ? v1[i] : v0[i], L.n_tris);
-        // the ranges of the tile's leaf cells from its sorted keys (as k_leaf_emit)
-        __threadfence_block();
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
-            const uint32_t key = k0[i];
-            if (i == 0 || k0[i - 1] != key) leaves[2 * (size_t)key] = q.pre_acc + i;
-            if (i + 1 == n || k0[i + 1] != key) leaves[2 * (size_t)key + 1] = q.pre_acc + i + 1u;
-        }
+    for (uint32_t o = blockIdx.x; o < n; o += gridDim.x) {
+        LeafTilePlan q;
+        const uint32_t item = items[o];
+        leaf_tile_plan(a, sums, info, T, item & ((1u << kSliceShift) - 1u), q);
+        __syncthreads();   // s is free again
+        if (q.mode == LEAF_BIG)
+            leaf_emit_big(q, item >> kSliceShift, L, h, boxes, t, a.cap_P2, top_keys, top_vals, cells, keys, vals, refs,
+                          leaves, write_keys, s);
+        else if (q.mode == LEAF_OVERSIZE)
+            leaf_emit_oversize(q, L, h, t, a.cap_P2, top_keys, top_vals, cells, keys, vals, tk, tv, refs, leaves, s);
     }
 }
 
@@ -1347,7 +1653,9 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
         auto mine = [&](uint32_t key) {
             if (key >= L.C1) return false;
             const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
-            return tile < T && leaf_tile_plan(a, sums, info, T, tile, q) && !q.staged;
+            if (tile >= T) return false;
+            leaf_tile_plan(a, sums, info, T, tile, q);
+            return q.mode == LEAF_OVERSIZE;
         };
         auto acc_slot = [&](uint32_t i) { return q.pre_acc + (sacc[i] - sacc[q.a0]); };
         auto rej_slot = [&](uint32_t i) { return q.tot_acc + q.pre_rej + (srej[i] - srej[q.a0]); };
@@ -1380,7 +1688,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
             LeafSetup s;
             leaf_pair(t, L, h, wkey, wtri, cells, s);
             mine(wkey);
-            wide_emit(L, s, s_tab, s_scan, wtri, acc_slot(w), rej_slot(w), prej[w], a.cap_P2, keys, vals);
+            wide_emit<kBlock / 64>(L, s, s_tab, s_scan, wtri, acc_slot(w), rej_slot(w), prej[w], a.cap_P2, keys, vals);
         }
         __syncthreads();   // the list is free for the next chunk
     }
@@ -1451,30 +1759,35 @@ void launch_ranges(const uint32_t* keys, const uint32_t* d_n, uint32_t cap, cons
 }
 
 void launch_leaf_cells(GridHeader* h, const BuildArgs& a, const uint32_t* ranges, uint32_t* cells,
-                       uint32_t* dbg, uint32_t* sums, hipStream_t st) {
+                       uint32_t* dbg, uint32_t* sums, uint32_t* leaves, hipStream_t st) {
     const uint32_t blocks = (a.cap_C1 + kBlock - 1) / kBlock;
     if (blocks == 0) return;
     hipLaunchKernelGGL(k_leaf_cells_count, dim3(blocks), dim3(kBlock), 0, st, h, a, ranges, sums, dbg);
-    hipLaunchKernelGGL(k_leaf_cells_write, dim3(blocks), dim3(kBlock), 0, st, h, a, ranges, cells, sums);
+    hipLaunchKernelGGL(k_leaf_cells_write, dim3(blocks), dim3(kBlock), 0, st, h, a, ranges, cells, sums,
+                       leaves);
 }
 
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
                       const uint32_t* top_vals, const uint32_t* ranges, const uint32_t* cells, uint32_t* keys,
                       uint32_t* vals, uint32_t* tmp_keys, uint32_t* tmp_vals, float* refs, uint32_t* dbg,
-                      uint32_t* sums, uint32_t* info, const LeafLarge* large, uint32_t* leaves, hipStream_t st) {
+                      uint32_t* sums, uint32_t* info, uint2* boxes, const LeafLarge* large, uint32_t* leaves, hipStream_t st) {
     const uint32_t T = (uint32_t)leaf_tiles(a.cap_P1);
     const uint32_t blocks = (a.cap_P1 + kBlock - 1) / kBlock;
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
-                           sums, info, T, dbg, large ? large->pacc : nullptr, large ? large->prej : nullptr);
+                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr);
     hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges, cells, sums, T,
                        large ? large->pacc : nullptr, large ? large->prej : nullptr);
     // with `large`, the global sort and k_ranges need every key; without it
     // the tiles write the leaf ranges and the keys are kept for keep_debug
     uint32_t* lv = large ? nullptr : leaves;
+    uint32_t* todo = sums + 2 * (size_t)leaf_sums_stride(T) + 4 + kWideCap;   // see leaf_sums_words
     const int write_keys = (large || a.keep_debug) ? 1 : 0;
-    hipLaunchKernelGGL(k_leaf_emit, dim3(T), dim3(kLeafBlock), 0, st, t, h, a, top_keys, top_vals, cells, keys, vals,
-                       refs, sums, info, T, lv, write_keys);
+    hipLaunchKernelGGL(k_leaf_emit, dim3(T), dim3(kLeafBlock), 0, st, t, h, a, top_keys, top_vals, cells, boxes, keys,
+                       vals, refs, sums, info, T, lv, write_keys, large ? 1 : 0, todo, todo + 1);
+    hipLaunchKernelGGL(k_leaf_emit_big, dim3(kBigBlocks), dim3(kBigBlock), 0, st, t, h, a,
+                       top_keys, top_vals, cells, boxes, keys, vals, refs, sums, info, T, lv, write_keys, todo, todo + 1,
+                       tmp_keys, tmp_vals);
     if (large) {
         launch_scan(large->pacc, large->sacc, a.cap_P1, false, large->scan_scratch, st);
         launch_scan(large->prej, large->srej, a.cap_P1, false, large->scan_scratch, st);
@@ -1482,9 +1795,6 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
         pb = pb < 1 ? 1 : (pb > 4096 ? 4096 : pb);
         hipLaunchKernelGGL(k_leaf_emit_par, dim3(pb), dim3(kBlock), 0, st, t, h, a, top_keys, top_vals, ranges, cells,
                            keys, vals, sums, info, T, large->prej, large->sacc, large->srej);
-    } else {
-        hipLaunchKernelGGL(k_leaf_emit_large, dim3((T + kOverTiles - 1) / kOverTiles), dim3(kBlock), 0, st, t, h, a,
-                           top_keys, top_vals, cells, keys, vals, sums, info, T, tmp_keys, tmp_vals, refs, lv);
     }
 }
 
@@ -1653,11 +1963,14 @@ size_t leaf_tiles(uint32_t n) {
     const size_t t = ((size_t)n + kLeafTile - 1) / kLeafTile;
     return t ? t : 1;
 }
-// accepted and rejected totals, their grand totals, the list of wide boxes
+// accepted and rejected totals, their grand totals, the list of wide boxes, the
+// number of work items of k_leaf_emit_big (all cleared before each build), then
+// the items
 size_t leaf_sums_words(uint32_t n) {
-    return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap;
+    return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap + 1;
 }
-size_t leaf_info_words(uint32_t n) { return 4 * leaf_tiles(n); }
+size_t leaf_item_words(uint32_t n) { return kSlicesMax * leaf_tiles(n); }
+size_t leaf_info_words(uint32_t n) { return 5 * leaf_tiles(n); }
 
 
 }  // namespace sg

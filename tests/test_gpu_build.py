@@ -202,6 +202,60 @@ def test_rebuild_into_wide_leaf_boxes(ctx, oracle, n_small):
     _assert_leaf_level(g, og)
 
 
+def _clumps(n_clump, spread):
+    """20,000 small triangles, n_clump of them moved into one top cell:
+    spread 0 puts them all on one place (every leaf list as long as the
+    clump), otherwise over spread times the cell"""
+    a = sa.gen_soup(71, 20_000, 0.01)
+    at = np.float32(0.301)
+    for j in range(3):
+        own = a[3 * j:3 * j + 3, :n_clump].copy()
+        if spread == 0.0:
+            own = np.repeat(own[:, :1], n_clump, axis=1)
+        a[3 * j:3 * j + 3, :n_clump] = at + (own - np.float32(0.5)) * np.float32(max(spread, 0.004))
+    return a
+
+
+@pytest.mark.parametrize("keep", [0, 1])
+@pytest.mark.parametrize("case", [
+    ("clump", 400, 0.05), ("clump", 2_000, 0.05), ("clump", 2_200, 0.05), ("clump", 11_200, 0.05),
+    ("clump", 11_600, 0.05), ("clump", 190, 0.0), ("clump", 200, 0.0), ("clump", 1_700, 0.0), ("clump", 9_000, 0.0),
+    ("sphere", 30_000, 0.0), ("sphere", 200_000, 0.0), ("coarse", 4_000, 0.0)], ids=lambda c: f"{c[0]}{c[1]}-{c[2]}")
+def test_leaf_tile_forms_bit_exact(ctx, oracle, case, keep):
+    """leaf tiles at the edges of the emission's forms: more top pairs than a
+    small and than a sliced tile holds, lists on both sides of the length from
+    which a wave sorts them, boxes of more than 32 cells (large triangles over
+    a finely divided cell), tiles in several slices"""
+    name, n, spread = case
+    kw = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0)
+    if name == "clump":
+        a = _clumps(n, spread)
+    elif name == "sphere":
+        a = W.sphere_mesh(n)
+    else:   # few large triangles over a grid of few, finely divided top cells
+        a = sa.gen_soup(73, n, 0.3)
+        kw = dict(res_override=(2, 2, 3), lambda_leaf=4.0)
+    og = oracle.build_twolevel(a, **kw)
+    assert og.status == 0
+    scene = sa.FaceSoup(ctx, a)
+    b = sa.FastTwoLevelGridBuilder(ctx, keep_debug=keep, **kw)
+    b.init(scene)
+    g = b.build()
+    rays = sa.gen_random_rays(72, 20_000, 0.0, 1.0)
+    po, to = og.trace(rays)
+    for _ in range(2):
+        info = g.info()
+        assert info.status == 0
+        assert (info.C2, info.P2, info.P2_valid) == (og.C2, og.P2, og.P2_valid)
+        names = ["top_keys", "top_vals", "top_cells", "leaf_vals", "leaves", "indices"]
+        for k in names + (["leaf_keys", "pair_counts"] if keep else []):
+            np.testing.assert_array_equal(g.download(k), getattr(og, k), err_msg=k)
+        pg, tg = g.trace_host(rays)   # reads the reference records
+        np.testing.assert_array_equal(pg, po)
+        np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+        g.rebuild()
+
+
 def test_twolevel_reference_leaf_lambda(ctx, oracle):
     """lambda_leaf = 1.2 (TwoLevelBuildKernels.h:49) on the 10k soup"""
     w = W.soup10k()

@@ -371,3 +371,45 @@ def test_uniform_cell_words(ctx, oracle, res, shift, shadow):
     np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
     np.testing.assert_array_equal(sg, so)
     assert (po != sa.MISS).sum() > 100
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("shift", [0.0, 1000.0])
+@pytest.mark.parametrize("res,scale_z,flagged", [
+    ((13, 14, 12), 1.0, False), ((2, 1, 1), 1.0, False),
+    ((1, 1, 1), 19.9, False),          # one top cell, near 255 leaf cells along z
+    ((1, 1, 1), 22.0, True),           # beyond 255: the packed byte wraps
+    ((64, 64, 1), 1.0, True), ((2, 90, 3), 1.0, True), ((1, 1, 40), 1.0, True)])   # leaf resolutions of 0
+def test_leaf_walk_forms(ctx, oracle, res, scale_z, flagged, shift, shadow):
+    """the leaf walk of grids whose leaf resolutions lie in 1..255 and of those
+    flagged otherwise: ids, t and the walk's counters equal the oracle's, for
+    rays from inside, outside and on the faces, along the axes and short ones"""
+    a = _clumped_soup(0.0)
+    a[2::3] *= np.float32(scale_z)
+    a += np.float32(shift)
+    opt = dict(lam=5.0, top_divisor=1, lambda_leaf=2.0, leaf_min_refs=16, res_override=res)
+    og = oracle.build_twolevel(a, **opt)
+    assert (og.status != 0) == flagged
+    b = sa.FastTwoLevelGridBuilder(ctx, **opt)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    rays = sa.gen_random_rays(83, 20_000, -0.3, 1.3)
+    n = rays.shape[1] // 8
+    rays[3, :n] = 0.0                                  # in a plane across x
+    rays[4, n // 2:n] = 0.0                            # along z
+    rays[0, n:2 * n] = np.where(np.arange(n) % 2, og.bmin[0] - np.float32(shift), og.bmax[0] - np.float32(shift))
+    rays[2] *= np.float32(scale_z)
+    rays[5] *= np.float32(scale_z)
+    rays[2, 2 * n:3 * n] = og.bmax[2] - np.float32(shift)
+    rays[6, 3 * n:4 * n] = 0.2                         # short segments
+    rays[0:3] += np.float32(shift)
+    if shadow:
+        rays[6] = 1.0
+    pg, tg, sg = g.trace_host(rays, with_stats=True, shadow=shadow)
+    po, to, so = og.trace(rays, with_stats=True, shadow=shadow)
+    np.testing.assert_array_equal(pg, po)
+    np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+    np.testing.assert_array_equal(sg, so)
+    p2, t2 = g.trace_host(rays, shadow=shadow)         # without counters
+    np.testing.assert_array_equal(p2, po)
+    np.testing.assert_array_equal(t2.view(np.uint32), to.view(np.uint32))

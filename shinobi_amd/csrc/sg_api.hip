@@ -371,7 +371,7 @@ bool uni_job_of(sg_grid* g, UniJob* j) {
     }
     j->sort = g->sort1;
     j->cap_P = g->cap_P1;
-    j->T = (uint32_t)((g->cap_P1 + 4095u) / 4096u);
+    j->T = multi_sort_tiles(g->cap_P1);
     j->passes = g->passes1;
     j->rb = g->rb;
     j->ranges = g->ranges1;

@@ -13,9 +13,16 @@
 
 namespace sg {
 
-constexpr int kItems = 4;                      // items per thread in the emission kernels
-constexpr int kTile = kBlock * kItems;         // 1024 items per tile
-constexpr uint32_t kStage = 4096;              // top pairs a tile stages in LDS before writing them out
+// Triangles per thread in the top-level count and emission: four (16-byte
+// loads), or one for scenes too small to give every CU a block that way, whose
+// time is the longest lane's emission.
+// (k_top_emit with one: 10,000-triangle soup 17.2 -> 6.8 us; with one or two
+// on the 2,093,058-triangle height field the rebuild was 4 % slower or equal.)
+constexpr int kItems = 4;
+constexpr uint32_t kSmallTop = 1u << 19;       // triangles up to which a thread takes one
+constexpr uint32_t kStage = 1024;              // top pairs a tile stages in LDS, for each of a thread's triangles
+static int top_items(uint32_t n) { return n <= kSmallTop ? 1 : kItems; }
+static size_t top_tiles(uint32_t n, int items) { return ((size_t)n + kBlock * items - 1) / (kBlock * items); }
 
 // --------------------------------------------------------------- init
 // Zero the cell ranges and leaves; reset the header.
@@ -276,31 +283,32 @@ SG_D void top_emit_one(const Params& P, const v3& v0, const v3& v1, const v3& v2
 // ------------------------------------------------------ top level emission
 // countRefs + InclusiveScan + buildUnsortedGrid of
 // src/Control/Algorithm/FastBuildKernels.h:31-215 as reduce-then-scan: a
-// count kernel leaves one sum per 1024-triangle tile, the emit kernel folds
+// count kernel leaves one sum per tile of 1024 or 256 triangles, the emit kernel folds
 // the sums of the tiles before it, rescans its own counts and writes every
-// triangle's pairs at its slot.  Four consecutive triangles per lane (one
+// triangle's pairs at its slot.  kItems consecutive triangles per lane (one
 // 16-byte load per SoA array); the emit kernel keeps the lane's vertices in
 // registers from the count to the emission (reloading them after the scans
 // fetched the arrays 2.3 times: a wave of blocks touches more than an XCD's
 // L2 holds).
-SG_D void top_counts(const Params& P, const TriSoA& t, uint32_t n, uint32_t i0, uint32_t cnt[kItems],
-                     float f[9][kItems]) {
-    cnt[0] = cnt[1] = cnt[2] = cnt[3] = 0;
+template <int ITEMS>
+SG_D void top_counts(const Params& P, const TriSoA& t, uint32_t n, uint32_t i0, uint32_t cnt[ITEMS],
+                     float f[9][ITEMS]) {
+    for (int j = 0; j < ITEMS; ++j) cnt[j] = 0;
     if (!P.ok || i0 >= n) return;
-    if (i0 + kItems <= n) {
+    if (ITEMS == 4 && i0 + 4 <= n) {
 #pragma unroll
         for (int c = 0; c < 9; ++c) {
             const float4 q = reinterpret_cast<const float4*>(t.v[c])[i0 / 4];
-            f[c][0] = q.x; f[c][1] = q.y; f[c][2] = q.z; f[c][3] = q.w;
+            f[c][0] = q.x; f[c][1 % ITEMS] = q.y; f[c][2 % ITEMS] = q.z; f[c][3 % ITEMS] = q.w;
         }
     } else {
 #pragma unroll
         for (int c = 0; c < 9; ++c)
 #pragma unroll
-            for (int j = 0; j < kItems; ++j) f[c][j] = i0 + j < n ? t.v[c][i0 + j] : 0.f;
+            for (int j = 0; j < ITEMS; ++j) f[c][j] = i0 + j < n ? t.v[c][i0 + j] : 0.f;
     }
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
         if (i0 + j < n) {
             v3 mn, mx;
             uint32_t lo[3], hi[3];
@@ -311,38 +319,46 @@ SG_D void top_counts(const Params& P, const TriSoA& t, uint32_t n, uint32_t i0, 
     }
 }
 
+template <int ITEMS>
 SG_D void top_count_body(const TriSoA& t, uint32_t n, const GridHeader* h, uint32_t* __restrict__ sums,
                          uint32_t* __restrict__ dbg_counts, uint32_t bid) {
     __shared__ uint32_t s_red[kBlock / 64];
     const Params P = read_params(h);
-    const uint32_t i0 = bid * kTile + threadIdx.x * kItems;
-    uint32_t cnt[kItems];
-    float f[9][kItems];
-    top_counts(P, t, n, i0, cnt, f);
+    const uint32_t i0 = bid * (kBlock * ITEMS) + threadIdx.x * ITEMS;
+    uint32_t cnt[ITEMS];
+    float f[9][ITEMS];
+    top_counts<ITEMS>(P, t, n, i0, cnt, f);
     if (dbg_counts)
-        for (int j = 0; j < kItems; ++j)
+        for (int j = 0; j < ITEMS; ++j)
             if (i0 + j < n) dbg_counts[i0 + j] = cnt[j];
-    const uint32_t s = block_sum<kBlock / 64>(cnt[0] + cnt[1] + cnt[2] + cnt[3], s_red);
+    uint32_t sum = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) sum += cnt[j];
+    const uint32_t s = block_sum<kBlock / 64>(sum, s_red);
     if (threadIdx.x == 0) sums[bid] = s;
 }
 
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_top_count(TriSoA t, uint32_t n, GridHeader* h,
                                                       uint32_t* __restrict__ sums,
                                                       uint32_t* __restrict__ dbg_counts) {
-    top_count_body(t, n, h, sums, dbg_counts, blockIdx.x);
+    top_count_body<ITEMS>(t, n, h, sums, dbg_counts, blockIdx.x);
 }
 
+template <int ITEMS>
 SG_D void top_emit_body(const TriSoA& t, uint32_t n, GridHeader* h, const BuildArgs& a, uint32_t* __restrict__ keys,
                         uint32_t* __restrict__ vals, const uint32_t* __restrict__ sums, uint32_t bid, uint32_t nb) {
     __shared__ uint32_t s_scan[kBlock / 64];
-    __shared__ uint32_t s_k[kStage], s_v[kStage];
+    __shared__ uint32_t s_k[(kStage * ITEMS)], s_v[(kStage * ITEMS)];
     const Params P = read_params(h);
     const uint32_t prefix = block_prefix_of<kBlock / 64>(sums, bid, s_scan);
-    const uint32_t i0 = bid * kTile + threadIdx.x * kItems;
-    uint32_t cnt[kItems];
-    float f[9][kItems];
-    top_counts(P, t, n, i0, cnt, f);
-    const uint32_t sum = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    const uint32_t i0 = bid * (kBlock * ITEMS) + threadIdx.x * ITEMS;
+    uint32_t cnt[ITEMS];
+    float f[9][ITEMS];
+    top_counts<ITEMS>(P, t, n, i0, cnt, f);
+    uint32_t sum = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) sum += cnt[j];
     uint32_t agg;
     const uint32_t local = block_excl_scan<kBlock / 64>(sum, &agg, s_scan);
     if (bid == nb - 1 && threadIdx.x == 0) {
@@ -352,12 +368,12 @@ SG_D void top_emit_body(const TriSoA& t, uint32_t n, GridHeader* h, const BuildA
         if (P1 > a.cap_P1) atomicOr(&h->status, ST_CAP_P1);
     }
     if ((uint64_t)prefix + agg > a.cap_P1) return;   // flagged by the last tile
-    if (agg <= kStage) {
+    if (agg <= (kStage * ITEMS)) {
         // the tile's pairs are one contiguous run: build it in LDS, then
         // write it out with full cache lines
         uint32_t ls = local;
 #pragma unroll
-        for (int j = 0; j < kItems; ++j) {
+        for (int j = 0; j < ITEMS; ++j) {
             if (cnt[j])
                 top_emit_one(P, mk(f[0][j], f[1][j], f[2][j]), mk(f[3][j], f[4][j], f[5][j]),
                              mk(f[6][j], f[7][j], f[8][j]), i0 + j, ls, s_k, s_v);
@@ -372,7 +388,7 @@ SG_D void top_emit_body(const TriSoA& t, uint32_t n, GridHeader* h, const BuildA
     }
     uint32_t slot = prefix + local;
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
         if (cnt[j])
             top_emit_one(P, mk(f[0][j], f[1][j], f[2][j]), mk(f[3][j], f[4][j], f[5][j]),
                          mk(f[6][j], f[7][j], f[8][j]), i0 + j, slot, keys, vals);
@@ -380,11 +396,12 @@ SG_D void top_emit_body(const TriSoA& t, uint32_t n, GridHeader* h, const BuildA
     }
 }
 
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_top_emit(TriSoA t, uint32_t n, GridHeader* h, BuildArgs a,
                                                      uint32_t* __restrict__ keys,
                                                      uint32_t* __restrict__ vals,
                                                      const uint32_t* __restrict__ sums) {
-    top_emit_body(t, n, h, a, keys, vals, sums, blockIdx.x, gridDim.x);
+    top_emit_body<ITEMS>(t, n, h, a, keys, vals, sums, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------- ranges
@@ -1746,10 +1763,16 @@ void launch_params(GridHeader* h, const BuildArgs& a, const uint32_t* part, uint
 
 void launch_top_emit(const TriSoA& t, uint32_t n, GridHeader* h, const BuildArgs& a, uint32_t* keys,
                      uint32_t* vals, uint32_t* dbg, uint32_t* sums, hipStream_t st) {
-    const uint32_t blocks = (n + kTile - 1) / kTile;
-    if (blocks == 0) return;
-    hipLaunchKernelGGL(k_top_count, dim3(blocks), dim3(kBlock), 0, st, t, n, h, sums, dbg);
-    hipLaunchKernelGGL(k_top_emit, dim3(blocks), dim3(kBlock), 0, st, t, n, h, a, keys, vals, sums);
+    const int items = top_items(n);
+    const dim3 blocks((uint32_t)top_tiles(n, items)), tb(kBlock);
+    if (n == 0) return;
+    if (items == 1) {
+        hipLaunchKernelGGL(k_top_count<1>, blocks, tb, 0, st, t, n, h, sums, dbg);
+        hipLaunchKernelGGL(k_top_emit<1>, blocks, tb, 0, st, t, n, h, a, keys, vals, sums);
+    } else {
+        hipLaunchKernelGGL(k_top_count<kItems>, blocks, tb, 0, st, t, n, h, sums, dbg);
+        hipLaunchKernelGGL(k_top_emit<kItems>, blocks, tb, 0, st, t, n, h, a, keys, vals, sums);
+    }
 }
 
 void launch_ranges(const uint32_t* keys, const uint32_t* d_n, uint32_t cap, const uint32_t* d_C,
@@ -1899,7 +1922,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_top_count(const UniJob* __rest
     uint32_t bid, nb;
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
     const TriSoA t = j.t;
-    top_count_body(t, j.n, j.h, j.sums, j.dbg, bid);
+    top_count_body<kItems>(t, j.n, j.h, j.sums, j.dbg, bid);
 }
 
 __global__ __launch_bounds__(kBlock) void k_multi_top_emit(const UniJob* __restrict__ jobs,
@@ -1908,7 +1931,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_top_emit(const UniJob* __restr
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
     const TriSoA t = j.t;
     const BuildArgs a = j.a;
-    top_emit_body(t, j.n, j.h, a, j.k[0], j.v[0], j.sums, bid, nb);
+    top_emit_body<kItems>(t, j.n, j.h, a, j.k[0], j.v[0], j.sums, bid, nb);
 }
 
 __global__ __launch_bounds__(kBlock) void k_multi_ranges(const UniJob* __restrict__ jobs,
@@ -1933,7 +1956,7 @@ uint32_t multi_blocks(const UniJob& j, MultiPhase ph) {
         case MP_INIT: return init_blocks(j.z) > j.nb_bounds ? init_blocks(j.z) : j.nb_bounds;
         case MP_PARAMS: return 1;
         case MP_TOP_COUNT:
-        case MP_TOP_EMIT: return (j.n + kTile - 1) / kTile;
+        case MP_TOP_EMIT: return (uint32_t)top_tiles(j.n, kItems);
         case MP_RANGES: return ranges_blocks(j.cap_P);
         case MP_REFS: return refs_blocks(j.cap_P);
         default: return 0;
@@ -1956,7 +1979,7 @@ void launch_multi(MultiPhase ph, const UniJob* jobs, const MultiEntry* e, uint32
 }
 
 // number of per-tile sums the emission kernels need for n items
-size_t emit_tiles(uint32_t n) { return ((size_t)n + kTile - 1) / kTile; }
+size_t emit_tiles(uint32_t n) { return top_tiles(n, top_items(n)); }
 size_t cell_tiles(uint32_t n) { return ((size_t)n + kBlock - 1) / kBlock; }
 // leaf tiles over n sorted top pairs
 size_t leaf_tiles(uint32_t n) {

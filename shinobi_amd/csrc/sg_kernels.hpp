@@ -227,6 +227,7 @@ enum MultiSortStep { MS_UP, MS_SCAN, MS_DOWN };
 // blocks a grid's own launch of the phase uses (0: no launch)
 uint32_t multi_blocks(const UniJob& j, MultiPhase ph);
 uint32_t multi_sort_blocks(const UniJob& j, MultiSortStep step);
+uint32_t multi_sort_tiles(uint32_t cap);   // UniJob::T
 void launch_multi(MultiPhase ph, const UniJob* jobs, const MultiEntry* e, uint32_t ne, uint32_t blocks,
                   hipStream_t st);
 // pass `pass` of every listed job, all of radix width rb

@@ -2,7 +2,7 @@
 // scan for gfx950, both reduce-then-scan (no inter-block waiting).
 //
 // Sort (semantics of chag::pp::sort as driven by src/Utils/Sort.cu:28-56),
-// per pass over 4096-key tiles:
+// per pass over tiles of 4096 or 1024 keys:
 //   up     per-tile digit counts -> counts[digit][tile]
 //   scan   one block per digit: exclusive scan of its row, and its total
 //   down   scans the digit totals into bases, ranks the tile's keys per digit
@@ -19,55 +19,71 @@
 
 namespace sg {
 
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kBlock * kSortItems;   // 4096 keys
+// Keys per thread.  A tile of 16 x 256 keys writes its digit runs in whole
+// cache lines; a small sort then has few tiles, and each waits for 16 ranking
+// rounds in a row, so sorts of up to kSmallSort pairs take 4 keys per thread.
+// (26,000 pairs: k_sort_down 11.4 -> 6.5 us a pass, k_sort_up 4.1 -> 2.4; at
+// 2.46 M pairs the smaller tiles were 10 us slower.)
+constexpr int kSortItems = 16, kSmallItems = 4;
+constexpr uint32_t kSmallSort = 1u << 20;
+// Up to this many tiles a tile's digit offsets are folded by the downsweep
+// itself from counts stored [tile][digit] (one row of them per tile before
+// it), and the scan launch between the sweeps, 3 us and a gap, falls away.
+constexpr uint32_t kFoldTiles = 64;
+
+static int sort_items(uint32_t cap) { return cap <= kSmallSort ? kSmallItems : kSortItems; }
 
 int sort_passes(int key_bits, int radix_bits) {
     if (key_bits < 1) key_bits = 1;
     return (key_bits + radix_bits - 1) / radix_bits;
 }
 
-static size_t sort_tiles(uint32_t cap) { return ((size_t)cap + kSortTile - 1) / kSortTile; }
+static size_t sort_tiles(uint32_t cap, int items) {
+    const size_t tile = (size_t)kBlock * items;
+    return ((size_t)cap + tile - 1) / tile;
+}
+
+uint32_t multi_sort_tiles(uint32_t cap) { return (uint32_t)sort_tiles(cap, kSortItems); }
 
 size_t sort_scratch_words(uint32_t cap, int key_bits, int radix_bits) {
     const size_t R = (size_t)1 << radix_bits;
     const size_t passes = (size_t)sort_passes(key_bits, radix_bits);
-    size_t w = passes * R + R * (sort_tiles(cap) + 1);
+    size_t w = passes * R + R * (sort_tiles(cap, sort_items(cap)) + 1);
     return (w + 3) & ~(size_t)3;   // 16-byte multiple
 }
 
-// per-tile digit counts of one pass -> counts[d * T + tile].  Each thread
-// counts 16 consecutive keys and adds runs of equal digits with one LDS
+// per-tile digit counts of one pass -> counts[d * T + tile], with FOLD
+// counts[tile * R + d].  Each thread counts ITEMS consecutive keys and adds runs of equal digits with one LDS
 // atomic, so runs of equal keys (cell-ordered emission) do not serialise.
 // (the kernels are bodies taking the tile / digit index `bid`, called by
 // the single-sort kernels with blockIdx.x and by the multi-grid kernels
 // with the block's index within its grid)
-template <int RB>
+template <int RB, int ITEMS, bool FOLD>
 SG_D void sort_up_body(const uint32_t* __restrict__ keys, const uint32_t* d_n, uint32_t cap, int shift,
                        uint32_t* __restrict__ counts, uint32_t T, uint32_t bid) {
     constexpr int R = 1 << RB;
     __shared__ uint32_t s[R];
     const uint32_t n = min(*d_n, cap);
-    const uint32_t base = bid * kSortTile;
+    const uint32_t base = bid * (kBlock * ITEMS);
     if (base >= n) return;
     for (int i = threadIdx.x; i < R; i += kBlock) s[i] = 0;
     __syncthreads();
-    const uint32_t i0 = base + threadIdx.x * kSortItems;
-    uint32_t k[kSortItems];
-    if (i0 + kSortItems <= n) {
+    const uint32_t i0 = base + threadIdx.x * ITEMS;
+    uint32_t k[ITEMS];
+    if (i0 + ITEMS <= n) {
 #pragma unroll
-        for (int q = 0; q < kSortItems / 4; ++q) {
+        for (int q = 0; q < ITEMS / 4; ++q) {
             const uint4 v = reinterpret_cast<const uint4*>(keys + i0)[q];
             k[4 * q] = v.x; k[4 * q + 1] = v.y; k[4 * q + 2] = v.z; k[4 * q + 3] = v.w;
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < kSortItems; ++j) k[j] = i0 + j < n ? keys[i0 + j] : 0u;
+        for (int j = 0; j < ITEMS; ++j) k[j] = i0 + j < n ? keys[i0 + j] : 0u;
     }
-    const uint32_t m = i0 < n ? min((uint32_t)kSortItems, n - i0) : 0u;
+    const uint32_t m = i0 < n ? min((uint32_t)ITEMS, n - i0) : 0u;
     uint32_t rd = 0, rc = 0;
 #pragma unroll
-    for (int j = 0; j < kSortItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
         if ((uint32_t)j < m) {
             const uint32_t d = (k[j] >> shift) & (R - 1);
             if (rc && d != rd) {
@@ -80,24 +96,24 @@ SG_D void sort_up_body(const uint32_t* __restrict__ keys, const uint32_t* d_n, u
     }
     if (rc) atomicAdd(&s[rd], rc);
     __syncthreads();
-    for (int d = threadIdx.x; d < R; d += kBlock) counts[(size_t)d * T + bid] = s[d];
+    for (int d = threadIdx.x; d < R; d += kBlock) counts[FOLD ? (size_t)bid * R + d : (size_t)d * T + bid] = s[d];
 }
 
-template <int RB>
+template <int RB, int ITEMS, bool FOLD>
 __global__ __launch_bounds__(kBlock) void k_sort_up(const uint32_t* __restrict__ keys, const uint32_t* d_n,
                                                     uint32_t cap, int shift, uint32_t* __restrict__ counts,
                                                     uint32_t T) {
-    sort_up_body<RB>(keys, d_n, cap, shift, counts, T, blockIdx.x);
+    sort_up_body<RB, ITEMS, FOLD>(keys, d_n, cap, shift, counts, T, blockIdx.x);
 }
 
 // one block per digit d: counts[d][t] -> sum over t' < t (in place), and
 // totals[d] = the digit's count over all tiles
-template <int RB>
+template <int RB, int ITEMS>
 SG_D void sort_scan_body(const uint32_t* d_n, uint32_t cap, uint32_t* __restrict__ totals,
                          uint32_t* __restrict__ counts, uint32_t T, uint32_t bid) {
     __shared__ uint32_t s_scan[kBlock / 64];
     const uint32_t n = min(*d_n, cap);
-    const uint32_t tiles = (n + kSortTile - 1) / kSortTile;
+    const uint32_t tiles = (n + kBlock * ITEMS - 1) / (kBlock * ITEMS);
     const uint32_t d = bid;
     uint32_t run = 0;
     uint32_t* row = counts + (size_t)d * T;
@@ -122,37 +138,38 @@ SG_D void sort_scan_body(const uint32_t* d_n, uint32_t cap, uint32_t* __restrict
     if (threadIdx.x == 0) totals[d] = run;
 }
 
-template <int RB>
+template <int RB, int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_sort_scan(const uint32_t* d_n, uint32_t cap,
                                                       uint32_t* __restrict__ totals,
                                                       uint32_t* __restrict__ counts, uint32_t T) {
-    sort_scan_body<RB>(d_n, cap, totals, counts, T, blockIdx.x);
+    sort_scan_body<RB, ITEMS>(d_n, cap, totals, counts, T, blockIdx.x);
 }
 
-template <int RB>
+template <int RB, int ITEMS, bool FOLD>
 SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                          uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, const uint32_t* d_n,
                          uint32_t cap, int shift, const uint32_t* __restrict__ totals,
                          const uint32_t* __restrict__ offsets, uint32_t T, uint32_t bid) {
     constexpr int R = 1 << RB;
+    constexpr uint32_t kTileKeys = kBlock * ITEMS;
     __shared__ uint32_t s_cnt[4][R];
     __shared__ uint32_t s_goff[R];
     __shared__ uint32_t s_tdo[R];
-    __shared__ uint32_t s_k[kSortTile];
-    __shared__ uint32_t s_v[kSortTile];
+    __shared__ uint32_t s_k[kTileKeys];
+    __shared__ uint32_t s_v[kTileKeys];
     __shared__ uint32_t s_scan[4];
     const uint32_t n = min(*d_n, cap);
     const uint32_t tile = bid;
-    const uint32_t base = tile * kSortTile;
+    const uint32_t base = tile * kTileKeys;
     if (base >= n) return;
     for (int i = threadIdx.x; i < 4 * R; i += kBlock) (&s_cnt[0][0])[i] = 0u;
     __syncthreads();
 
     const int w = wave_id(), l = lane_id();
-    const uint32_t wbase = base + (uint32_t)w * (kSortItems * 64);
-    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
+    const uint32_t wbase = base + (uint32_t)w * (ITEMS * 64);
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kSortItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const uint32_t pos = wbase + k * 64 + l;
         const bool ok = pos < n;
         key[k] = ok ? kin[pos] : 0u;
@@ -162,7 +179,7 @@ SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __res
     // RB ballots; items processed in tile order
     const uint64_t lt = lanemask_lt();
 #pragma unroll
-    for (int k = 0; k < kSortItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const uint32_t pos = wbase + k * 64 + l;
         const bool ok = pos < n;
         const uint32_t d = (key[k] >> shift) & (R - 1);
@@ -180,6 +197,27 @@ SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __res
         if (ok && l == __ffsll((long long)m) - 1) s_cnt[w][d] = cur + cnt;
     }
     __syncthreads();
+    // the digit's count in the tiles before this one, and in all
+    uint32_t before = 0, all = 0;
+    if (threadIdx.x < R) {
+        if (FOLD) {
+            const uint32_t tiles = (n + kTileKeys - 1u) / kTileKeys;
+            for (uint32_t t0 = 0; t0 < tiles; t0 += 16u) {
+                uint32_t c[16];
+#pragma unroll
+                for (uint32_t u = 0; u < 16u; ++u)
+                    c[u] = t0 + u < tiles ? offsets[(size_t)(t0 + u) * R + threadIdx.x] : 0u;
+#pragma unroll
+                for (uint32_t u = 0; u < 16u; ++u) {
+                    before += t0 + u < tile ? c[u] : 0u;
+                    all += c[u];
+                }
+            }
+        } else {
+            before = offsets[(size_t)threadIdx.x * T + tile];
+            all = totals[threadIdx.x];
+        }
+    }
     uint32_t total = 0;
     if (threadIdx.x < R) {
         const int d = threadIdx.x;
@@ -193,14 +231,14 @@ SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __res
     uint32_t tsum;
     const uint32_t tdo = block_excl_scan<kBlock / 64>(total, &tsum, s_scan);
     // digit bases: exclusive scan of the digit totals
-    const uint32_t dbase = block_excl_scan<kBlock / 64>(threadIdx.x < R ? totals[threadIdx.x] : 0u, &tsum, s_scan);
+    const uint32_t dbase = block_excl_scan<kBlock / 64>(all, &tsum, s_scan);
     if (threadIdx.x < R) {
         s_tdo[threadIdx.x] = tdo;
-        s_goff[threadIdx.x] = dbase + offsets[(size_t)threadIdx.x * T + tile] - tdo;
+        s_goff[threadIdx.x] = dbase + before - tdo;
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kSortItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const uint32_t pos = wbase + k * 64 + l;
         if (pos < n) {
             const uint32_t d = (key[k] >> shift) & (R - 1);
@@ -210,7 +248,7 @@ SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __res
         }
     }
     __syncthreads();
-    const uint32_t cnt_tile = min((uint32_t)kSortTile, n - base);
+    const uint32_t cnt_tile = min(kTileKeys, n - base);
     for (uint32_t j = threadIdx.x; j < cnt_tile; j += kBlock) {
         const uint32_t k = s_k[j];
         const uint32_t g = s_goff[(k >> shift) & (R - 1)] + j;
@@ -219,14 +257,14 @@ SG_D void sort_down_body(const uint32_t* __restrict__ kin, const uint32_t* __res
     }
 }
 
-template <int RB>
+template <int RB, int ITEMS, bool FOLD>
 __global__ __launch_bounds__(kBlock) void k_sort_down(const uint32_t* __restrict__ kin,
                                                       const uint32_t* __restrict__ vin,
                                                       uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                       const uint32_t* d_n, uint32_t cap, int shift,
                                                       const uint32_t* __restrict__ totals,
                                                       const uint32_t* __restrict__ offsets, uint32_t T) {
-    sort_down_body<RB>(kin, vin, kout, vout, d_n, cap, shift, totals, offsets, T, blockIdx.x);
+    sort_down_body<RB, ITEMS, FOLD>(kin, vin, kout, vout, d_n, cap, shift, totals, offsets, T, blockIdx.x);
 }
 
 // pass `pass` of the sorts of many grids (UniJob): scratch layout as
@@ -236,7 +274,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_sort_up(const UniJob* __restri
                                                           const MultiEntry* __restrict__ e, uint32_t ne, int pass) {
     uint32_t bid, nb;
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
-    sort_up_body<RB>(j.k[pass & 1], &j.h->P1, j.cap_P, pass * RB, j.sort + (size_t)j.passes * (1 << RB), j.T, bid);
+    sort_up_body<RB, kSortItems, false>(j.k[pass & 1], &j.h->P1, j.cap_P, pass * RB, j.sort + (size_t)j.passes * (1 << RB), j.T, bid);
 }
 
 template <int RB>
@@ -244,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_sort_scan(const UniJob* __rest
                                                             const MultiEntry* __restrict__ e, uint32_t ne, int pass) {
     uint32_t bid, nb;
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
-    sort_scan_body<RB>(&j.h->P1, j.cap_P, j.sort + (size_t)pass * (1 << RB), j.sort + (size_t)j.passes * (1 << RB),
+    sort_scan_body<RB, kSortItems>(&j.h->P1, j.cap_P, j.sort + (size_t)pass * (1 << RB), j.sort + (size_t)j.passes * (1 << RB),
                        j.T, bid);
 }
 
@@ -254,29 +292,40 @@ __global__ __launch_bounds__(kBlock) void k_multi_sort_down(const UniJob* __rest
     uint32_t bid, nb;
     const UniJob& j = jobs[multi_entry(e, ne, blockIdx.x, gridDim.x, bid, nb)];
     const int i = pass & 1, o = i ^ 1;
-    sort_down_body<RB>(j.k[i], j.v[i], j.k[o], j.v[o], &j.h->P1, j.cap_P, pass * RB,
+    sort_down_body<RB, kSortItems, false>(j.k[i], j.v[i], j.k[o], j.v[o], &j.h->P1, j.cap_P, pass * RB,
                        j.sort + (size_t)pass * (1 << RB), j.sort + (size_t)j.passes * (1 << RB), j.T, bid);
 }
 
-template <int RB>
+template <int RB, int ITEMS, bool FOLD>
 static void sort_impl(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, const uint32_t* d_n, uint32_t cap,
                       int key_bits, uint32_t* scratch, hipStream_t st) {
     constexpr int R = 1 << RB;
     const int passes = sort_passes(key_bits, RB);
-    const uint32_t T = (uint32_t)sort_tiles(cap);
+    const uint32_t T = (uint32_t)sort_tiles(cap, ITEMS);
     if (T == 0) return;
     uint32_t* totals = scratch;
     uint32_t* counts = scratch + (size_t)passes * R;
     uint32_t *ki = k0, *vi = v0, *ko = k1, *vo = v1;
+    const dim3 tiles(T), tb(kBlock);
     for (int p = 0; p < passes; ++p) {
         uint32_t* tot = totals + (size_t)p * R;
-        hipLaunchKernelGGL(k_sort_up<RB>, dim3(T), dim3(kBlock), 0, st, ki, d_n, cap, p * RB, counts, T);
-        hipLaunchKernelGGL(k_sort_scan<RB>, dim3(R), dim3(kBlock), 0, st, d_n, cap, tot, counts, T);
-        hipLaunchKernelGGL(k_sort_down<RB>, dim3(T), dim3(kBlock), 0, st, ki, vi, ko, vo, d_n, cap, p * RB, tot,
+        hipLaunchKernelGGL((k_sort_up<RB, ITEMS, FOLD>), tiles, tb, 0, st, ki, d_n, cap, p * RB, counts, T);
+        if (!FOLD) hipLaunchKernelGGL((k_sort_scan<RB, ITEMS>), dim3(R), tb, 0, st, d_n, cap, tot, counts, T);
+        hipLaunchKernelGGL((k_sort_down<RB, ITEMS, FOLD>), tiles, tb, 0, st, ki, vi, ko, vo, d_n, cap, p * RB, tot,
                            counts, T);
         uint32_t* t = ki; ki = ko; ko = t;
         t = vi; vi = vo; vo = t;
     }
+}
+
+template <int RB>
+static void sort_size(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, const uint32_t* d_n, uint32_t cap,
+                      int key_bits, uint32_t* scratch, hipStream_t st) {
+    if (sort_items(cap) == kSortItems) sort_impl<RB, kSortItems, false>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st);
+    else if (sort_tiles(cap, kSmallItems) > kFoldTiles)
+        sort_impl<RB, kSmallItems, false>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st);
+    else
+        sort_impl<RB, kSmallItems, true>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st);
 }
 
 uint32_t multi_sort_blocks(const UniJob& j, MultiSortStep step) {
@@ -305,9 +354,9 @@ void launch_multi_sort(MultiSortStep step, int rb, int pass, const UniJob* jobs,
 void launch_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, const uint32_t* d_n, uint32_t cap,
                        int key_bits, int radix_bits, uint32_t* scratch, hipStream_t st) {
     switch (radix_bits) {
-        case 4: sort_impl<4>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
-        case 6: sort_impl<6>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
-        default: sort_impl<8>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
+        case 4: sort_size<4>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
+        case 6: sort_size<6>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
+        default: sort_size<8>(k0, v0, k1, v1, d_n, cap, key_bits, scratch, st); break;
     }
 }
 

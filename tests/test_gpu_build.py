@@ -436,3 +436,18 @@ def test_rebuild_many_graph_matches_oracle(ctx, oracle):
     _assert_top_level(g, og)
     np.testing.assert_array_equal(g.download("indices"), og.indices)
     batch.clear()
+
+
+@pytest.mark.parametrize("n,size", [
+    (1, 0.1), (255, 0.05), (256, 0.05), (257, 0.05),
+    (1_000, 0.4),                                  # more pairs in a tile than it stages
+    (2**19 - 1, 0.002), (2**19, 0.002), (2**19 + 1, 0.002)])   # one triangle or four per thread
+def test_top_emission_forms_at_their_edges(ctx, oracle, n, size):
+    a = sa.gen_soup(91, n, size)
+    og = oracle.build_uniform(a, lam=5.0, top_divisor=1)
+    assert og.status == 0
+    _, g = _gpu_build(ctx, a, 0, lam=5.0)
+    _assert_same_params(g.info(), og)
+    _assert_top_level(g, og)
+    g.rebuild()
+    _assert_top_level(g, og)

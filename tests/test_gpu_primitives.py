@@ -39,3 +39,18 @@ def test_sort_is_stable_and_matches_numpy(ctx, radix_bits, n, key_bits, dup):
     order = np.argsort(keys, kind="stable")
     np.testing.assert_array_equal(k, keys[order])
     np.testing.assert_array_equal(v, vals[order])
+
+
+@pytest.mark.parametrize("radix_bits", [4, 6, 8])
+@pytest.mark.parametrize("n", [255, 1023, 1025, 65_535, 65_536, 65_537, 2**20 - 1, 2**20, 2**20 + 1])
+def test_sort_forms_at_their_edges(ctx, radix_bits, n):
+    """tiles of 1024 and 4096 keys, digit offsets folded in the downsweep (up
+    to 64 tiles) or scanned by a launch of their own: either side of each edge"""
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 2**18, n, dtype=np.uint64).astype(np.uint32)
+    keys[: n // 3] = 5
+    vals = np.arange(n, dtype=np.uint32)
+    k, v = sa.sort_pairs(ctx, keys, vals, key_bits=18, radix_bits=radix_bits)
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k, keys[order])
+    np.testing.assert_array_equal(v, vals[order])

@@ -413,3 +413,68 @@ def test_leaf_walk_forms(ctx, oracle, res, scale_z, flagged, shift, shadow):
     p2, t2 = g.trace_host(rays, shadow=shadow)         # without counters
     np.testing.assert_array_equal(p2, po)
     np.testing.assert_array_equal(t2.view(np.uint32), to.view(np.uint32))
+
+
+def _ahead_scene(name):
+    if name == "soup":
+        return _clumped_soup(0.0)
+    if name == "shifted":                      # entry points round onto or past the far faces
+        return _clumped_soup(1000.0)
+    if name == "cluster":                      # cells of hundreds of references, long leaf walks
+        return sa.gen_cluster(4, 30_000, 120)
+    return sa.gen_heightfield(2, 121, 0.2)
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("scene", ["soup", "shifted", "cluster", "heightfield"])
+def test_small_batches_walk_ahead(ctx, oracle, scene, kind, shadow):
+    """batches on either side of every count of rays per wave (a device of 256
+    CUs holds 6,144 waves): ids and t equal the oracle's bit for bit, with the
+    count on the host and on the device"""
+    a = _ahead_scene(scene)
+    opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)
+    og = oracle.build_twolevel(a, **opt) if kind else oracle.build_uniform(a, top_divisor=1, **opt)
+    b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    sizes = [1, 63, 1_000, 12_288, 12_289, 24_576, 24_577, 49_152, 49_153, 98_304, 98_305]
+    rays = sa.gen_random_rays(95, max(sizes), -0.2, 1.2)
+    n = rays.shape[1]
+    rays[3, ::11] = 0.0
+    rays[4, ::22] = 0.0
+    rays[0, 3::13] = og.bmax[0] if scene != "shifted" else og.bmax[0] - np.float32(1000.0)
+    rays[6, 5::17] = 0.3
+    if scene == "shifted":
+        rays[0:3] += np.float32(1000.0)
+    if shadow:
+        rays[6] = 1.0
+    rays = rays[:, np.random.default_rng(96).permutation(n)]
+    po, to = og.trace(np.ascontiguousarray(rays), shadow=shadow)[:2]
+    assert (po != sa.MISS).sum() > 50
+    cap = sa.RayBatch(ctx, np.ascontiguousarray(rays))
+    count = sa.DeviceBuffer(ctx, 4)
+    for m in sizes:
+        p, t = g.trace_host(np.ascontiguousarray(rays[:, :m]), shadow=shadow)
+        np.testing.assert_array_equal(p, po[:m])
+        np.testing.assert_array_equal(t.view(np.uint32), to[:m].view(np.uint32))
+        count.upload(np.array([m], np.uint32))
+        pd, td = g.trace(cap, d_count=count.ptr, n=n, shadow=shadow)
+        np.testing.assert_array_equal(pd.download(np.uint32, m), po[:m])
+        np.testing.assert_array_equal(td.download(np.float32, m).view(np.uint32), to[:m].view(np.uint32))
+
+
+def test_rays_that_never_leave_walk_ahead(ctx, oracle):
+    """NaN and infinite rays end with the guard, in both grid kinds"""
+    a = _clumped_soup(0.0)
+    rays = sa.gen_random_rays(97, 640, -0.2, 1.2)
+    rays[0, ::7], rays[3, 1::7], rays[6, 2::7], rays[4, 3::7], rays[5, 4::7] = np.nan, np.nan, np.nan, np.inf, -np.inf
+    for kind in (0, 1):
+        opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)
+        b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
+        b.init(sa.FaceSoup(ctx, a))
+        g = b.build()
+        ps, ts, _ = g.trace_host(rays, with_stats=True)     # the general walk
+        p, t = g.trace_host(rays)
+        np.testing.assert_array_equal(p, ps)
+        np.testing.assert_array_equal(t.view(np.uint32), ts.view(np.uint32))

@@ -1041,13 +1041,7 @@ SG_D void trace_one(const GView& g, const GRays& rays, uint32_t i, gptr<uint32_t
 
 // one ray per G lanes (see cells_ahead); lanes without one (valid false) take part
 template <int KIND, bool SHADOW>
-SG_D void trace_ahead(const GView& g, const GRays& rays, uint32_t i, gptr<uint32_t> prim, gptr<float> tout,
-                      bool valid, uint32_t G) {
-    const GParams p = load_gparams(g.hdr);
-    const uint32_t j = valid ? i : 0u;
-    Ray r;
-    ray_begin(r, mk(rays.a[0][j], rays.a[1][j], rays.a[2][j]), mk(rays.a[3][j], rays.a[4][j], rays.a[5][j]),
-              valid ? rays.a[6][j] : 0.f);
+SG_D void ray_walk_ahead(const GView& g, const GParams& p, Ray& r, bool valid, uint32_t G) {
     Walk w;
     if (KIND == 0) {
         walk_init_uniform<SHADOW>(p, r, w);
@@ -1058,6 +1052,17 @@ SG_D void trace_ahead(const GView& g, const GRays& rays, uint32_t i, gptr<uint32
         w.active = w.active && valid;
         walk_twolevel_ahead<SHADOW>(g, p, r, w, G);
     }
+}
+
+template <int KIND, bool SHADOW>
+SG_D void trace_ahead(const GView& g, const GRays& rays, uint32_t i, gptr<uint32_t> prim, gptr<float> tout,
+                      bool valid, uint32_t G) {
+    const GParams p = load_gparams(g.hdr);
+    const uint32_t j = valid ? i : 0u;
+    Ray r;
+    ray_begin(r, mk(rays.a[0][j], rays.a[1][j], rays.a[2][j]), mk(rays.a[3][j], rays.a[4][j], rays.a[5][j]),
+              valid ? rays.a[6][j] : 0.f);
+    ray_walk_ahead<KIND, SHADOW>(g, p, r, valid, G);
     if (valid && ((uint32_t)lane_id() & (G - 1u)) == 0u) {
         prim[i] = r.best == kMiss ? kMiss : g.indices[r.best];
         tout[i] = r.t;
@@ -1215,35 +1220,51 @@ SG_D uint32_t xcd_group_block(uint32_t b, uint32_t nb) {
 // (src/Engine/RayBuffers.h:52-77) with the direction the trace kernel
 // restores, 1 / rcp (src/Engine/RayTracingKernels.h:128-130), and bestHit =
 // the reference index the traverser returns (0xFFFFFFFF on a miss).
-template <int KIND, bool CAM>
-__global__ __launch_bounds__(kBlock) SG_TRACE_OCCUPANCY void k_trace_gen(GridView g, RaySoA rays, CamArgs cam,
-                                                                        uint32_t cap, const uint32_t* d_n,
-                                                                        TraceOut out) {
+// AHEAD: a small batch, walked ahead of as by k_trace's sparse form
+// (256 x 256 camera rays, 10,000 triangles, uniform: 38.8 -> 30.3 us; 24,000
+// camera rays, 500,000-triangle height field, two-level: 162 -> 58 us).
+template <int KIND, bool CAM, bool AHEAD>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(AHEAD ? 4 : 5))) void k_trace_gen(
+    GridView g, RaySoA rays, CamArgs cam, uint32_t cap, const uint32_t* d_n, uint32_t fill, TraceOut out) {
     const uint32_t n = (!CAM && d_n) ? min(*d_n, cap) : cap;
-    const uint32_t i = (CAM ? xcd_group_block(blockIdx.x, gridDim.x) : blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
     const GView gv = gview(g);
+    const uint32_t block = CAM ? xcd_group_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    uint32_t i = block * blockDim.x + threadIdx.x, G = 1;
+    bool valid = i < n;
+    if (AHEAD) {   // one-wave blocks
+        const uint32_t R = rays_per_wave(n, fill), l = (uint32_t)lane_id();
+        if (block * R >= n) return;
+        // failed builds and irregular leaf levels go the general way
+        if (!__builtin_amdgcn_readfirstlane((int)(gv.hdr->status & ~ST_NEG_EXTENT))) G = 64u / R;
+        i = block * R + l / G;
+        valid = i < n && l / G < R;
+    } else if (!valid) {
+        return;
+    }
     const bool failed = grid_failed(gv);
     const GParams p = load_gparams(gv.hdr);
-    uint32_t slot = i;
+    uint32_t slot = valid ? i : 0u;
     Ray r;
     if (CAM) {
-        slot = tile_pixel(cam, i);
+        slot = tile_pixel(cam, slot);
         const v3 o = mk(cam.pos[0], cam.pos[1], cam.pos[2]);
         const v3 d = camera_dir(cam, slot);
-        if (out.rays[0]) {
+        if (out.rays[0] && valid) {
             const float v[7] = {o.x, o.y, o.z, d.x, d.y, d.z, 3.402823466e+38f};
             for (int k = 0; k < 7; ++k) out.rays[k][slot] = v[k];
         }
-        ray_begin(r, o, d, 3.402823466e+38f);
+        ray_begin(r, o, d, !AHEAD || valid ? 3.402823466e+38f : 0.f);
     } else {
         const GRays gr = grays(rays);
-        ray_begin(r, mk(gr.a[0][i], gr.a[1][i], gr.a[2][i]), mk(gr.a[3][i], gr.a[4][i], gr.a[5][i]), gr.a[6][i]);
+        ray_begin(r, mk(gr.a[0][slot], gr.a[1][slot], gr.a[2][slot]), mk(gr.a[3][slot], gr.a[4][slot], gr.a[5][slot]),
+                  !AHEAD || valid ? gr.a[6][slot] : 0.f);
     }
     if (!failed) {
         uint32_t s1 = 0, s2 = 0, s3 = 0;
-        ray_walk<KIND, false>(gv, p, r, s1, s2, s3);
+        if (AHEAD && G > 1u) ray_walk_ahead<KIND, false>(gv, p, r, valid, G);
+        else ray_walk<KIND, false>(gv, p, r, s1, s2, s3);
     }
+    if (AHEAD && !(valid && ((uint32_t)lane_id() & (G - 1u)) == 0u)) return;
     if (out.prim) out.prim[slot] = r.best == kMiss ? kMiss : gv.indices[r.best];
     if (out.t) out.t[slot] = r.t;
     if (out.raybuf) {
@@ -1266,16 +1287,24 @@ void launch_trace_gen(const GridView& g, const RaySoA& r, const CamArgs* cam, ui
                       const TraceOut& out, hipStream_t st) {
     if (n == 0) return;
     constexpr int B = 64;   // one-wave blocks, as launch_trace
-    const dim3 grid((n + B - 1) / B), tb(B);
     CamArgs c{};
     if (cam) c = *cam;
+    const uint32_t fill = device_fill();
+    // a count in device memory takes the dense form
+    const uint32_t R = d_n ? 64u : rays_per_wave(n, fill);
+    const bool ahead = R <= kAheadRays;
+    const dim3 grid((n + (ahead ? R : B) - 1) / (ahead ? R : B)), tb(B);
+#define SG_GEN(K, C)                                                                                               \
+    do {                                                                                                           \
+        if (ahead) hipLaunchKernelGGL((k_trace_gen<K, C, true>), grid, tb, 0, st, g, r, c, n, d_n, fill, out);     \
+        else hipLaunchKernelGGL((k_trace_gen<K, C, false>), grid, tb, 0, st, g, r, c, n, d_n, fill, out);          \
+    } while (0)
     if (g.kind == 0) {
-        if (cam) hipLaunchKernelGGL((k_trace_gen<0, true>), grid, tb, 0, st, g, r, c, n, d_n, out);
-        else hipLaunchKernelGGL((k_trace_gen<0, false>), grid, tb, 0, st, g, r, c, n, d_n, out);
+        if (cam) SG_GEN(0, true); else SG_GEN(0, false);
     } else {
-        if (cam) hipLaunchKernelGGL((k_trace_gen<1, true>), grid, tb, 0, st, g, r, c, n, d_n, out);
-        else hipLaunchKernelGGL((k_trace_gen<1, false>), grid, tb, 0, st, g, r, c, n, d_n, out);
+        if (cam) SG_GEN(1, true); else SG_GEN(1, false);
     }
+#undef SG_GEN
 }
 
 // ------------------------------------------------- many batches, one launch

@@ -118,3 +118,30 @@ def test_trace_store_equals_oracle(ctx, oracle, kind):
     assert np.isnan(got[:, m:]).all()
     g.close()
     scene.close()
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("res", [(1, 1), (3, 5), (96, 128), (97, 127), (256, 192), (257, 192), (256, 384), (257, 384)])
+def test_small_images_walk_ahead(ctx, oracle, kind, res):
+    """images on either side of every count of rays per wave, with every output"""
+    opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)
+    a = sa.gen_heightfield(2, 81, 0.2)
+    b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    og = oracle.build_twolevel(a, **opt) if kind else oracle.build_uniform(a, top_divisor=1, **opt)
+    camera = W.heightfield_pinhole(2, *res)
+    rays = sa.gen_camera_rays(*camera)
+    n = res[0] * res[1]
+    prim, t, raybuf = _nan_buffer(ctx, n), _nan_buffer(ctx, n), _nan_buffer(ctx, 8 * n)
+    rays_out = sa.RayBatch(ctx, np.full((7, n), np.nan, np.float32))
+    g.trace_camera(sa.pinhole(*camera), (2, 32), prim=prim, t=t, raybuf=raybuf, rays_out=rays_out)
+    ctx.sync()
+    po, to = og.trace(rays)
+    np.testing.assert_array_equal(rays_out.download().view(np.uint32), rays.view(np.uint32))
+    np.testing.assert_array_equal(prim.download(np.uint32, n), po)
+    np.testing.assert_array_equal(t.download(np.uint32, n), to.view(np.uint32))
+    np.testing.assert_array_equal(raybuf.download(np.uint32, 8 * n).reshape(8, n), og.trace_store(rays).view(np.uint32))
+    buf = _nan_buffer(ctx, 8 * n)
+    g.trace_store(sa.RayBatch(ctx, rays), raybuf=buf)
+    np.testing.assert_array_equal(buf.download(np.uint32, 8 * n).reshape(8, n), og.trace_store(rays).view(np.uint32))

@@ -547,207 +547,6 @@ SG_D void uniform_start(const GView& g, const GParams& p, Ray& r, Walk& w, RemBi
     }
 }
 
-template <bool SHADOW>
-SG_D void walk_uniform(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t& steps) {
-    RemBits b;
-    UWalk u;
-    uniform_start<SHADOW>(g, p, r, w, b, u, steps);
-    if ((uint32_t)p.res[0] * (uint32_t)p.res[1] * (uint32_t)p.res[2] >= kWordCells)
-        while (const uint64_t act = __ballot(u.active)) uniform_step<SHADOW, true>(g, b, r, u, act, steps);
-    else
-        while (const uint64_t act = __ballot(u.active)) uniform_step<SHADOW, false>(g, b, r, u, act, steps);
-}
-
-// TwoLevelGridTraverser::traverse, src/Control/Algorithm/TwoLevelGridTraverser.h:445-671;
-// SHADOW: TwoLevelGridShadowTraverser (:677-828) does not start a ray with
-// t < 0.9999, visits every leaf cell of an entered top cell and every top
-// cell up to the grid exit until t < 0.9999 (no t > tMax tests).  It ignores
-// a failed traverseInit and walks from an uninitialised cell; here such a
-// ray is not traversed.
-template <bool SHADOW>
-SG_D void walk_init_twolevel(const GParams& p, const Ray& r, Walk& w) {
-    w.guard = 0;
-    w.active = SHADOW ? !(r.t < kShadowT) : r.t > 0.f;
-    if (!traverse_init<true>(p, r, w.tEntry, w.cell, w.tMax)) w.active = false;
-}
-
-SG_D bool take_step(uint32_t& left) {
-    if (left == 0u) return false;
-    --left;
-    return true;
-}
-
-// the leaf walk of one top cell (TwoLevelGridTraverser.h:489-528 set-up)
-struct LeafEntry {
-    v3 sc, stMax, scs;      // entry leaf cell, exit distances, leaf cell size
-    uint32_t c0, c1, c2;    // the top cell's leaf resolution
-};
-
-SG_D LeafEntry leaf_entry(const GParams& p, const GView& g, const Ray& r, const Walk& w, uint2 top) {
-    LeafEntry e;
-    const v3 ep = r.o + div_rcp(w.tEntry, r);
-    e.c0 = top.y & 0xFFu;
-    e.c1 = (top.y >> 8) & 0xFFu;
-    e.c2 = (top.y >> 16) & 0xFFu;
-    const v3 cres = mk((float)e.c0, (float)e.c1, (float)e.c2);
-    const v3 srcp = p.crcp * cres;
-    const v3 mb = w.cell * p.cs + p.bmin;
-    v3 sc = mk(floorf((ep.x - mb.x) * srcp.x), floorf((ep.y - mb.y) * srcp.y), floorf((ep.z - mb.z) * srcp.z));
-    e.scs = mk(g.hdr->leaf_size[0][e.c0], g.hdr->leaf_size[1][e.c1], g.hdr->leaf_size[2][e.c2]);
-    sc = vmin(cres - mk(1.f, 1.f, 1.f), vmax(sc, mk(0.f, 0.f, 0.f)));
-    e.sc = sc;
-    e.stMax.x = ((sc.x + (float)(r.rcp.x > 0.f ? 1 : 0)) * e.scs.x + mb.x - r.o.x) * r.rcp.x;
-    e.stMax.y = ((sc.y + (float)(r.rcp.y > 0.f ? 1 : 0)) * e.scs.y + mb.y - r.o.y) * r.rcp.y;
-    e.stMax.z = ((sc.z + (float)(r.rcp.z > 0.f ? 1 : 0)) * e.scs.z + mb.z - r.o.z) * r.rcp.z;
-    return e;
-}
-
-// Leaf levels whose resolutions all lie in 1..255 (every grid but those
-// flagged ST_LEAF_RES): the entry cell is then inside the leaf level and the
-// walk needs no guard, so it runs as Cells does in the uniform grid.  The
-// fields of rem have fixed widths here (8 bits and the top bit).  The walk is
-// bound by issue (VALU busy in 64-70 % of the cycles) and a step in LeafAny's
-// form is a third of an iteration's instructions: 300,007 any-hit segments
-// through 38,665 triangles 272 -> 256 us, 1,000 random rays through 225,615
-// triangles 218 -> 198 us, the height field's camera and bounce launches
-// together 1.14 -> 1.10 ms.
-constexpr RemBits kLeafRem = {9u, 18u, 1u << 8 | 1u << 17 | 1u << 26};
-struct LeafCells {
-    Cells c;
-
-    SG_D v3 tmax() const { return c.tMax; }
-    SG_D void enter(const LeafEntry& e, uint32_t base, const Ray& r) {
-        c.tMax = e.stMax;
-        c.dt = mk(e.scs.x * fabsf(r.rcp.x), e.scs.y * fabsf(r.rcp.y), e.scs.z * fabsf(r.rcp.z));
-        const uint32_t x = (uint32_t)e.sc.x, y = (uint32_t)e.sc.y, z = (uint32_t)e.sc.z, sz = e.c0 * e.c1;
-        const bool px = r.rcp.x > 0.f, py = r.rcp.y > 0.f, pz = r.rcp.z > 0.f;
-        c.incx = px ? 1u : 0u - 1u;
-        c.incy = py ? e.c0 : 0u - e.c0;
-        c.incz = pz ? sz : 0u - sz;
-        c.cell = base + x + y * e.c0 + z * sz;
-        c.rem = (256u - (px ? e.c0 - x : x + 1u)) | (256u - (py ? e.c1 - y : y + 1u)) << 9 |
-                (256u - (pz ? e.c2 - z : z + 1u)) << 18;
-    }
-    SG_D bool step(const Ray&) { return cells_step(c, kLeafRem); }
-    SG_D uint2 load(const GView& g, const GParams& p) const {
-        return c.cell < p.C2 ? ld2(g.leaves + 2 * (size_t)c.cell) : make_uint2(0u, 0u);
-    }
-};
-
-// Any leaf level: a resolution of 0 puts the entry cell at -1, and the guard
-// ends walks that never reach an exit.
-struct LeafAny {
-    v3 sc, stMax, scs, cres;
-    uint32_t base, left;        // left: steps the guard still admits
-
-    SG_D v3 tmax() const { return stMax; }
-    SG_D void enter(const LeafEntry& e, uint32_t first, const Ray&) {
-        sc = e.sc;
-        stMax = e.stMax;
-        scs = e.scs;
-        cres = mk((float)e.c0, (float)e.c1, (float)e.c2);
-        base = first;
-        // the guard admits 2 (c0 + c1 + c2) + 16 leaf cells, the entry cell one of them
-        left = 2u * (e.c0 + e.c1 + e.c2) + 15u;
-    }
-    SG_D bool step(const Ray& r) { return dda_step(min_axis(stMax), sc, stMax, r.rcp, scs, cres) && take_step(left); }
-    SG_D uint2 load(const GView& g, const GParams& p) const {
-        const uint32_t li = base + f2u(sc.x + cres.x * sc.y + cres.x * cres.y * sc.z);
-        return li < p.C2 ? ld2(g.leaves + 2 * (size_t)li) : make_uint2(0u, 0u);
-    }
-};
-
-template <bool SHADOW, class Leaf>
-SG_D void walk_twolevel(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t& lsteps, uint32_t& tsteps,
-                        uint32_t& entered) {
-    const uint32_t cap = step_cap(p);
-    Refs q;
-    q.it = q.e = 0;
-    Leaf L;
-    bool in_leaf = false;
-    // enter the top cell at w.cell: a non-empty one starts its leaf walk
-    auto top_cell = [&]() {
-        if (!(w.guard++ < cap)) {
-            w.active = false;
-            return;
-        }
-        const uint2 top = load_cell(g, p, w.cell);
-        if (top.y & kNotEmpty) {
-            ++entered;
-            L.enter(leaf_entry(p, g, r, w, top), top.x, r);
-            in_leaf = true;
-            refs_begin(g, q, L.load(g, p), r);
-        }
-    };
-    if (w.active) top_cell();
-    // A lane done with its top cell waits (top_wait) until the wave takes its
-    // top steps together: at least kTopBatch lanes waiting, a lane waiting
-    // kTopWaitMax iterations, or no lane with anything else to do.  The top
-    // step and the set-up of the next leaf walk are the longest code of the
-    // loop; batching them runs that code in fewer iterations.
-    bool top_wait = false;
-    uint32_t waited = 0;
-    while (__ballot(w.active)) {
-        refs_coop(g, q, r, coop_threshold(w.active));
-        const bool test = q.it < q.e;
-        RefRec x;
-        if (test) ref_load(g, q, x);
-        // a lane whose leaf cell ends in this iteration takes the leaf DDA
-        // step before its test, as in the uniform walk
-        const bool fin = w.active && !top_wait && q.it + 1u >= q.e;
-        float tm = 0.f;
-        bool stepped = false;
-        uint2 nr = make_uint2(0u, 0u);
-        if (fin && in_leaf) {
-            tm = tmin(L.tmax());
-            stepped = L.step(r);
-            if (stepped) nr = L.load(g, p);
-        }
-        if (test) {
-            mt_test(x.a, x.b, x.c, q.it, r);
-            ++q.it;
-        }
-        if (fin) {
-            bool top_next = !in_leaf;
-            if (in_leaf) {
-                // a leaf cell is done: t check, then the leaf step taken above
-                const bool go = SHADOW ? !(r.t < kShadowT) : r.t > tm;
-                if (go) ++lsteps;
-                if (go && stepped) {
-                    refs_begin(g, q, nr, r);
-                } else {
-                    in_leaf = false;
-                    top_next = true;
-                }
-            }
-            top_wait = top_next;
-        }
-        const uint64_t waiting = __ballot(w.active && top_wait);
-        if (waiting) {
-            const bool go = __popcll(waiting) >= kTopBatch || !__ballot(w.active && !top_wait) ||
-                            __ballot(w.active && top_wait && waited >= kTopWaitMax);
-            if (w.active && top_wait) {
-                if (!go) {
-                    ++waited;
-                } else {
-                    top_wait = false;
-                    waited = 0;
-                    // the top cell is done: t check, top DDA step, next top cell
-                    if (SHADOW ? r.t < kShadowT : !(r.t > w.tMax.x || r.t > w.tMax.y || r.t > w.tMax.z)) {
-                        w.active = false;
-                    } else {
-                        ++tsteps;
-                        const Step a = min_axis(w.tMax);
-                        w.tEntry = sel(a, w.tMax.x, w.tMax.y, w.tMax.z);
-                        w.active = dda_step(a, w.cell, w.tMax, r.rcp, p.cs, p.resf);
-                        if (w.active) top_cell();
-                    }
-                }
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------- walking ahead
 // Batches too small to fill the chip last as long as their longest ray: a
 // serial chain of one step and one memory round trip per cell.  Here G lanes
@@ -867,20 +666,200 @@ SG_D void cells_ahead(const GView& g, const RemBits& b, Ray& r, Cells c, bool ac
     }
 }
 
+// the cells of a uniform grid from c on
+template <bool SHADOW>
+SG_D void uniform_ahead(const GView& g, const GParams& p, const RemBits& b, Ray& r, const Cells& c, bool active,
+                        uint32_t G) {
+    auto stops = [](float t, float tm) { return SHADOW ? !(t >= kShadowT) : !(t > tm); };
+    if ((uint32_t)p.res[0] * (uint32_t)p.res[1] * (uint32_t)p.res[2] >= kWordCells)
+        cells_ahead(g, b, r, c, active, G, [&](uint32_t k) {
+            return word_range(g, *(gptr<const u4v>)(g.words + 4u * (size_t)(k >> 5)), k);
+        }, stops);
+    else
+        cells_ahead(g, b, r, c, active, G, [&](uint32_t k) { return ld2(g.cells + 2u * (size_t)k); }, stops);
+}
+
 template <bool SHADOW>
 SG_D void walk_uniform_ahead(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t G) {
     uint32_t steps = 0;
     RemBits b;
     UWalk u;
     uniform_start<SHADOW>(g, p, r, w, b, u, steps);
-    auto stops = [](float t, float tm) { return SHADOW ? !(t >= kShadowT) : !(t > tm); };
-    if ((uint32_t)p.res[0] * (uint32_t)p.res[1] * (uint32_t)p.res[2] >= kWordCells)
-        cells_ahead(g, b, r, u.c, u.active, G, [&](uint32_t k) {
-            return word_range(g, *(gptr<const u4v>)(g.words + 4u * (size_t)(k >> 5)), k);
-        }, stops);
-    else
-        cells_ahead(g, b, r, u.c, u.active, G, [&](uint32_t k) { return ld2(g.cells + 2u * (size_t)k); }, stops);
+    uniform_ahead<SHADOW>(g, p, b, r, u.c, u.active, G);
 }
+
+// The end of a full wave.  Once kFewRays rays of it still walk, their
+// lanes' share of an iteration is an eighth at most, and the wave lasts as
+// long as the longest of them: the wave's lanes then split over those rays and
+// walk ahead of them (cells_ahead).  `few` says how: lane l takes over the ray
+// of lane src, which its group of G lanes finishes; ray_back returns t and
+// best to the ray's own lane.  Only waves with all 64 lanes present do this.
+// The sparse kernels have the registers for it; in the dense ones it cost
+// more than it gained (spills or five waves per SIMD for eight: 1920 x 1080
+// camera rays 0.44 -> 0.63 ms two-level, 0.31 -> 0.38 uniform).  150,000 rays
+// at 32 per wave: two-level soup 535 -> 433 us, 2 M-triangle height field 269
+// -> 197, uniform soup 147 -> 119, dense cluster 555 -> 466.
+constexpr uint32_t kFewRays = 8;
+struct Few {
+    uint32_t src, G;
+    bool active;   // the lane's group has a ray
+};
+
+SG_D bool few_left(uint64_t act) { return (uint32_t)__popcll(act) <= kFewRays && __ballot(true) == ~0ull; }
+
+SG_D Few few_split(uint64_t act) {
+    const uint32_t n = (uint32_t)__popcll(act);
+    Few f;
+    f.G = n > 4u ? 8u : (n > 2u ? 16u : (n > 1u ? 32u : 64u));
+    const uint32_t k = (uint32_t)lane_id() / f.G;
+    uint64_t m = act;
+    for (uint32_t s = 0; s + 1u < kFewRays; ++s)
+        if (s < k) m &= m - 1ull;
+    f.active = m != 0ull;
+    f.src = min(first_lane(m), 63u);
+    return f;
+}
+
+SG_D Ray few_ray(const Few& f, const Ray& r) {
+    Ray x;
+    x.o = shfl_v(r.o, f.src);
+    x.D = shfl_v(r.D, f.src);
+    x.rcp = shfl_v(r.rcp, f.src);
+    x.t = shfl_f(r.t, f.src);
+    x.best = shfl_u(r.best, f.src);
+    x.fast = (__ballot(r.fast) >> f.src) & 1ull;
+    x.tests = 0;
+    return x;
+}
+
+SG_D void ray_back(const Few& f, uint64_t act, const Ray& x, Ray& r) {
+    const uint32_t rank = (uint32_t)__popcll(act & lanemask_lt());
+    const float t = shfl_f(x.t, (rank * f.G) & 63u);
+    const uint32_t best = shfl_u(x.best, (rank * f.G) & 63u);
+    if ((act >> lane_id()) & 1ull) {
+        r.t = t;
+        r.best = best;
+    }
+}
+
+template <bool SHADOW, bool FEW>
+SG_D void walk_uniform(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t& steps) {
+    RemBits b;
+    UWalk u;
+    uniform_start<SHADOW>(g, p, r, w, b, u, steps);
+    uint64_t act;
+    if ((uint32_t)p.res[0] * (uint32_t)p.res[1] * (uint32_t)p.res[2] >= kWordCells)
+        while ((act = __ballot(u.active)) && !(FEW && few_left(act)))
+            uniform_step<SHADOW, true>(g, b, r, u, act, steps);
+    else
+        while ((act = __ballot(u.active)) && !(FEW && few_left(act)))
+            uniform_step<SHADOW, false>(g, b, r, u, act, steps);
+    if (FEW && act) {
+        const Few f = few_split(act);
+        Ray x = few_ray(f, r);
+        uniform_ahead<SHADOW>(g, p, b, x, shfl_cells(u.c, f.src), f.active, f.G);
+        ray_back(f, act, x, r);
+    }
+}
+
+// TwoLevelGridTraverser::traverse, src/Control/Algorithm/TwoLevelGridTraverser.h:445-671;
+// SHADOW: TwoLevelGridShadowTraverser (:677-828) does not start a ray with
+// t < 0.9999, visits every leaf cell of an entered top cell and every top
+// cell up to the grid exit until t < 0.9999 (no t > tMax tests).  It ignores
+// a failed traverseInit and walks from an uninitialised cell; here such a
+// ray is not traversed.
+template <bool SHADOW>
+SG_D void walk_init_twolevel(const GParams& p, const Ray& r, Walk& w) {
+    w.guard = 0;
+    w.active = SHADOW ? !(r.t < kShadowT) : r.t > 0.f;
+    if (!traverse_init<true>(p, r, w.tEntry, w.cell, w.tMax)) w.active = false;
+}
+
+SG_D bool take_step(uint32_t& left) {
+    if (left == 0u) return false;
+    --left;
+    return true;
+}
+
+// the leaf walk of one top cell (TwoLevelGridTraverser.h:489-528 set-up)
+struct LeafEntry {
+    v3 sc, stMax, scs;      // entry leaf cell, exit distances, leaf cell size
+    uint32_t c0, c1, c2;    // the top cell's leaf resolution
+};
+
+SG_D LeafEntry leaf_entry(const GParams& p, const GView& g, const Ray& r, const Walk& w, uint2 top) {
+    LeafEntry e;
+    const v3 ep = r.o + div_rcp(w.tEntry, r);
+    e.c0 = top.y & 0xFFu;
+    e.c1 = (top.y >> 8) & 0xFFu;
+    e.c2 = (top.y >> 16) & 0xFFu;
+    const v3 cres = mk((float)e.c0, (float)e.c1, (float)e.c2);
+    const v3 srcp = p.crcp * cres;
+    const v3 mb = w.cell * p.cs + p.bmin;
+    v3 sc = mk(floorf((ep.x - mb.x) * srcp.x), floorf((ep.y - mb.y) * srcp.y), floorf((ep.z - mb.z) * srcp.z));
+    e.scs = mk(g.hdr->leaf_size[0][e.c0], g.hdr->leaf_size[1][e.c1], g.hdr->leaf_size[2][e.c2]);
+    sc = vmin(cres - mk(1.f, 1.f, 1.f), vmax(sc, mk(0.f, 0.f, 0.f)));
+    e.sc = sc;
+    e.stMax.x = ((sc.x + (float)(r.rcp.x > 0.f ? 1 : 0)) * e.scs.x + mb.x - r.o.x) * r.rcp.x;
+    e.stMax.y = ((sc.y + (float)(r.rcp.y > 0.f ? 1 : 0)) * e.scs.y + mb.y - r.o.y) * r.rcp.y;
+    e.stMax.z = ((sc.z + (float)(r.rcp.z > 0.f ? 1 : 0)) * e.scs.z + mb.z - r.o.z) * r.rcp.z;
+    return e;
+}
+
+// Leaf levels whose resolutions all lie in 1..255 (every grid but those
+// flagged ST_LEAF_RES): the entry cell is then inside the leaf level and the
+// walk needs no guard, so it runs as Cells does in the uniform grid.  The
+// fields of rem have fixed widths here (8 bits and the top bit).  The walk is
+// bound by issue (VALU busy in 64-70 % of the cycles) and a step in LeafAny's
+// form is a third of an iteration's instructions: 300,007 any-hit segments
+// through 38,665 triangles 272 -> 256 us, 1,000 random rays through 225,615
+// triangles 218 -> 198 us, the height field's camera and bounce launches
+// together 1.14 -> 1.10 ms.
+constexpr RemBits kLeafRem = {9u, 18u, 1u << 8 | 1u << 17 | 1u << 26};
+struct LeafCells {
+    Cells c;
+
+    SG_D v3 tmax() const { return c.tMax; }
+    SG_D void enter(const LeafEntry& e, uint32_t base, const Ray& r) {
+        c.tMax = e.stMax;
+        c.dt = mk(e.scs.x * fabsf(r.rcp.x), e.scs.y * fabsf(r.rcp.y), e.scs.z * fabsf(r.rcp.z));
+        const uint32_t x = (uint32_t)e.sc.x, y = (uint32_t)e.sc.y, z = (uint32_t)e.sc.z, sz = e.c0 * e.c1;
+        const bool px = r.rcp.x > 0.f, py = r.rcp.y > 0.f, pz = r.rcp.z > 0.f;
+        c.incx = px ? 1u : 0u - 1u;
+        c.incy = py ? e.c0 : 0u - e.c0;
+        c.incz = pz ? sz : 0u - sz;
+        c.cell = base + x + y * e.c0 + z * sz;
+        c.rem = (256u - (px ? e.c0 - x : x + 1u)) | (256u - (py ? e.c1 - y : y + 1u)) << 9 |
+                (256u - (pz ? e.c2 - z : z + 1u)) << 18;
+    }
+    SG_D bool step(const Ray&) { return cells_step(c, kLeafRem); }
+    SG_D uint2 load(const GView& g, const GParams& p) const {
+        return c.cell < p.C2 ? ld2(g.leaves + 2 * (size_t)c.cell) : make_uint2(0u, 0u);
+    }
+};
+
+// Any leaf level: a resolution of 0 puts the entry cell at -1, and the guard
+// ends walks that never reach an exit.
+struct LeafAny {
+    v3 sc, stMax, scs, cres;
+    uint32_t base, left;        // left: steps the guard still admits
+
+    SG_D v3 tmax() const { return stMax; }
+    SG_D void enter(const LeafEntry& e, uint32_t first, const Ray&) {
+        sc = e.sc;
+        stMax = e.stMax;
+        scs = e.scs;
+        cres = mk((float)e.c0, (float)e.c1, (float)e.c2);
+        base = first;
+        // the guard admits 2 (c0 + c1 + c2) + 16 leaf cells, the entry cell one of them
+        left = 2u * (e.c0 + e.c1 + e.c2) + 15u;
+    }
+    SG_D bool step(const Ray& r) { return dda_step(min_axis(stMax), sc, stMax, r.rcp, scs, cres) && take_step(left); }
+    SG_D uint2 load(const GView& g, const GParams& p) const {
+        const uint32_t li = base + f2u(sc.x + cres.x * sc.y + cres.x * cres.y * sc.z);
+        return li < p.C2 ? ld2(g.leaves + 2 * (size_t)li) : make_uint2(0u, 0u);
+    }
+};
 
 // Two levels: the first kTopAhead lanes of a ray's group take the next top
 // cells and set up their leaf walks; groups of kLeafAhead lanes then walk the
@@ -973,6 +952,125 @@ SG_D void walk_twolevel_ahead(const GView& g, const GParams& p, Ray& r, Walk& w,
     }
 }
 
+template <bool SHADOW, class Leaf, bool FEW>
+SG_D void walk_twolevel(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t& lsteps, uint32_t& tsteps,
+                        uint32_t& entered) {
+    const uint32_t cap = step_cap(p);
+    Refs q;
+    q.it = q.e = 0;
+    Leaf L;
+    bool in_leaf = false;
+    // enter the top cell at w.cell: a non-empty one starts its leaf walk
+    auto top_cell = [&]() {
+        if (!(w.guard++ < cap)) {
+            w.active = false;
+            return;
+        }
+        const uint2 top = load_cell(g, p, w.cell);
+        if (top.y & kNotEmpty) {
+            ++entered;
+            L.enter(leaf_entry(p, g, r, w, top), top.x, r);
+            in_leaf = true;
+            refs_begin(g, q, L.load(g, p), r);
+        }
+    };
+    if (w.active) top_cell();
+    // A lane done with its top cell waits (top_wait) until the wave takes its
+    // top steps together: at least kTopBatch lanes waiting, a lane waiting
+    // kTopWaitMax iterations, or no lane with anything else to do.  The top
+    // step and the set-up of the next leaf walk are the longest code of the
+    // loop; batching them runs that code in fewer iterations.
+    bool top_wait = false;
+    uint32_t waited = 0;
+    uint64_t act;
+    while ((act = __ballot(w.active)) && !(FEW && few_left(act))) {
+        refs_coop(g, q, r, (uint32_t)__popcll(act) / 2u + 2u);
+        const bool test = q.it < q.e;
+        RefRec x;
+        if (test) ref_load(g, q, x);
+        // a lane whose leaf cell ends in this iteration takes the leaf DDA
+        // step before its test, as in the uniform walk
+        const bool fin = w.active && !top_wait && q.it + 1u >= q.e;
+        float tm = 0.f;
+        bool stepped = false;
+        uint2 nr = make_uint2(0u, 0u);
+        if (fin && in_leaf) {
+            tm = tmin(L.tmax());
+            stepped = L.step(r);
+            if (stepped) nr = L.load(g, p);
+        }
+        if (test) {
+            mt_test(x.a, x.b, x.c, q.it, r);
+            ++q.it;
+        }
+        if (fin) {
+            bool top_next = !in_leaf;
+            if (in_leaf) {
+                // a leaf cell is done: t check, then the leaf step taken above
+                const bool go = SHADOW ? !(r.t < kShadowT) : r.t > tm;
+                if (go) ++lsteps;
+                if (go && stepped) {
+                    refs_begin(g, q, nr, r);
+                } else {
+                    in_leaf = false;
+                    top_next = true;
+                }
+            }
+            top_wait = top_next;
+        }
+        const uint64_t waiting = __ballot(w.active && top_wait);
+        if (waiting) {
+            const bool go = __popcll(waiting) >= kTopBatch || !__ballot(w.active && !top_wait) ||
+                            __ballot(w.active && top_wait && waited >= kTopWaitMax);
+            if (w.active && top_wait) {
+                if (!go) {
+                    ++waited;
+                } else {
+                    top_wait = false;
+                    waited = 0;
+                    // the top cell is done: t check, top DDA step, next top cell
+                    if (SHADOW ? r.t < kShadowT : !(r.t > w.tMax.x || r.t > w.tMax.y || r.t > w.tMax.z)) {
+                        w.active = false;
+                    } else {
+                        ++tsteps;
+                        const Step a = min_axis(w.tMax);
+                        w.tEntry = sel(a, w.tMax.x, w.tMax.y, w.tMax.z);
+                        w.active = dda_step(a, w.cell, w.tMax, r.rcp, p.cs, p.resf);
+                        if (w.active) top_cell();
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (FEW) {
+        if (act) {
+            const Few f = few_split(act);
+            Ray x = few_ray(f, r);
+            Walk y;
+            y.cell = shfl_v(w.cell, f.src);
+            y.tMax = shfl_v(w.tMax, f.src);
+            y.tEntry = 0.f;
+            y.guard = shfl_u(w.guard, f.src);
+            // the rest of the current leaf walk, then on from the top cell
+            const uint64_t leaf_m = __ballot(in_leaf);
+            cells_ahead(g, kLeafRem, x, shfl_cells(L.c, f.src), f.active && ((leaf_m >> f.src) & 1ull), f.G,
+                        [&](uint32_t k) {
+                            return k < p.C2 ? ld2(g.leaves + 2 * (size_t)k) : make_uint2(0u, 0u);
+                        },
+                        [](float t, float tm) { return SHADOW ? t < kShadowT : !(t > tm); });
+            y.active = f.active && !(SHADOW ? x.t < kShadowT
+                                            : !(x.t > y.tMax.x || x.t > y.tMax.y || x.t > y.tMax.z));
+            if (y.active) {
+                const Step a = min_axis(y.tMax);
+                y.tEntry = sel(a, y.tMax.x, y.tMax.y, y.tMax.z);
+                y.active = dda_step(a, y.cell, y.tMax, x.rcp, p.cs, p.resf);
+            }
+            walk_twolevel_ahead<SHADOW>(g, p, x, y, f.G);
+            ray_back(f, act, x, r);
+        }
+    }
+}
+
 // A ray's start: rcp(dir) as the trace kernel computes it
 // (src/Engine/RayTracingKernels.h:111-113) and the intersector's recomputed
 // direction D = 1/rcp (src/Intersector/SimpleIntersector.hpp:58)
@@ -987,18 +1085,18 @@ SG_D void ray_begin(Ray& r, v3 o, v3 d, float t) {
 }
 
 // traverse (both traversers): leaves r.t and r.best (a reference index)
-template <int KIND, bool SHADOW>
+template <int KIND, bool SHADOW, bool FEW>
 SG_D void ray_walk(const GView& g, const GParams& p, Ray& r, uint32_t& s1, uint32_t& s2, uint32_t& s3) {
     Walk w;
     if (KIND == 0) {
         walk_init_uniform<SHADOW>(p, r, w);
-        walk_uniform<SHADOW>(g, p, r, w, s1);
+        walk_uniform<SHADOW, FEW>(g, p, r, w, s1);
     } else {
         walk_init_twolevel<SHADOW>(p, r, w);
         if (__builtin_amdgcn_readfirstlane((int)(g.hdr->status & ST_LEAF_RES)))
-            walk_twolevel<SHADOW, LeafAny>(g, p, r, w, s1, s2, s3);
+            walk_twolevel<SHADOW, LeafAny, false>(g, p, r, w, s1, s2, s3);
         else
-            walk_twolevel<SHADOW, LeafCells>(g, p, r, w, s1, s2, s3);
+            walk_twolevel<SHADOW, LeafCells, FEW>(g, p, r, w, s1, s2, s3);
     }
 }
 
@@ -1027,7 +1125,7 @@ SG_D void trace_one(const GView& g, const GRays& rays, uint32_t i, gptr<uint32_t
     ray_begin(r, mk(rays.a[0][j], rays.a[1][j], rays.a[2][j]), mk(rays.a[3][j], rays.a[4][j], rays.a[5][j]),
               SPARSE && !valid ? 0.f : rays.a[6][j]);   // t = 0: never traversed
     uint32_t s1 = 0, s2 = 0, s3 = 0;
-    ray_walk<KIND, SHADOW>(g, p, r, s1, s2, s3);
+    ray_walk<KIND, SHADOW, SPARSE && !STATS>(g, p, r, s1, s2, s3);
     if (SPARSE && !valid) return;
     prim[i] = r.best == kMiss ? kMiss : g.indices[r.best];
     tout[i] = r.t;
@@ -1087,9 +1185,10 @@ SG_D void trace_ahead(const GView& g, const GRays& rays, uint32_t i, gptr<uint32
 // or 1 rays (see cells_ahead), with up to 2 fill waves: more lanes per ray
 // than that were slower on rays that end soon, fewer on the rest (49,000 rays:
 // 8 / 4 / 2 rays per wave 230 / 199 / 196 us two-level, 125 / 130 / 156
-// uniform).  Up to 32 rays per wave of the chip a wave takes 32, whose idle
-// lanes help through the wave-shared tests (196,000 rays: 605 us against 632
-// walking ahead, two-level soup; 459 against 609, dense cluster).
+// uniform).  Up to 32 rays per wave of the chip a wave takes 32 and finishes
+// the last of them ahead (see Few); with larger batches at 32 rays a wave
+// there are more waves than the chip holds, and 64 were faster (250,000 rays:
+// 465 against 537 us, 300,000: 523 against 683, two-level soup).
 constexpr uint32_t kAheadRays = 8;
 constexpr uint32_t kSparseFill = 2;   // waves of a sparse launch / fill, at most
 SG_HD uint32_t rays_per_wave(uint32_t n, uint32_t fill) {
@@ -1220,18 +1319,18 @@ SG_D uint32_t xcd_group_block(uint32_t b, uint32_t nb) {
 // (src/Engine/RayBuffers.h:52-77) with the direction the trace kernel
 // restores, 1 / rcp (src/Engine/RayTracingKernels.h:128-130), and bestHit =
 // the reference index the traverser returns (0xFFFFFFFF on a miss).
-// AHEAD: a small batch, walked ahead of as by k_trace's sparse form
+// SPARSE: a small batch, walked ahead of as by k_trace's sparse form
 // (256 x 256 camera rays, 10,000 triangles, uniform: 38.8 -> 30.3 us; 24,000
 // camera rays, 500,000-triangle height field, two-level: 162 -> 58 us).
-template <int KIND, bool CAM, bool AHEAD>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(AHEAD ? 4 : 5))) void k_trace_gen(
+template <int KIND, bool CAM, bool SPARSE>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ? 4 : 5))) void k_trace_gen(
     GridView g, RaySoA rays, CamArgs cam, uint32_t cap, const uint32_t* d_n, uint32_t fill, TraceOut out) {
     const uint32_t n = (!CAM && d_n) ? min(*d_n, cap) : cap;
     const GView gv = gview(g);
     const uint32_t block = CAM ? xcd_group_block(blockIdx.x, gridDim.x) : blockIdx.x;
     uint32_t i = block * blockDim.x + threadIdx.x, G = 1;
     bool valid = i < n;
-    if (AHEAD) {   // one-wave blocks
+    if (SPARSE) {   // one-wave blocks
         const uint32_t R = rays_per_wave(n, fill), l = (uint32_t)lane_id();
         if (block * R >= n) return;
         // failed builds and irregular leaf levels go the general way
@@ -1253,18 +1352,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(AHEAD ? 
             const float v[7] = {o.x, o.y, o.z, d.x, d.y, d.z, 3.402823466e+38f};
             for (int k = 0; k < 7; ++k) out.rays[k][slot] = v[k];
         }
-        ray_begin(r, o, d, !AHEAD || valid ? 3.402823466e+38f : 0.f);
+        ray_begin(r, o, d, !SPARSE || valid ? 3.402823466e+38f : 0.f);
     } else {
         const GRays gr = grays(rays);
         ray_begin(r, mk(gr.a[0][slot], gr.a[1][slot], gr.a[2][slot]), mk(gr.a[3][slot], gr.a[4][slot], gr.a[5][slot]),
-                  !AHEAD || valid ? gr.a[6][slot] : 0.f);
+                  !SPARSE || valid ? gr.a[6][slot] : 0.f);
     }
     if (!failed) {
         uint32_t s1 = 0, s2 = 0, s3 = 0;
-        if (AHEAD && G > 1u) ray_walk_ahead<KIND, false>(gv, p, r, valid, G);
-        else ray_walk<KIND, false>(gv, p, r, s1, s2, s3);
+        if (SPARSE && G > 1u) ray_walk_ahead<KIND, false>(gv, p, r, valid, G);
+        else ray_walk<KIND, false, false>(gv, p, r, s1, s2, s3);
     }
-    if (AHEAD && !(valid && ((uint32_t)lane_id() & (G - 1u)) == 0u)) return;
+    if (SPARSE && !(valid && ((uint32_t)lane_id() & (G - 1u)) == 0u)) return;
     if (out.prim) out.prim[slot] = r.best == kMiss ? kMiss : gv.indices[r.best];
     if (out.t) out.t[slot] = r.t;
     if (out.raybuf) {
@@ -1292,11 +1391,11 @@ void launch_trace_gen(const GridView& g, const RaySoA& r, const CamArgs* cam, ui
     const uint32_t fill = device_fill();
     // a count in device memory takes the dense form
     const uint32_t R = d_n ? 64u : rays_per_wave(n, fill);
-    const bool ahead = R <= kAheadRays;
-    const dim3 grid((n + (ahead ? R : B) - 1) / (ahead ? R : B)), tb(B);
+    const bool sparse = R <= kAheadRays;   // 32 rays a wave gain nothing on camera rays
+    const dim3 grid((n + (sparse ? R : B) - 1) / (sparse ? R : B)), tb(B);
 #define SG_GEN(K, C)                                                                                               \
     do {                                                                                                           \
-        if (ahead) hipLaunchKernelGGL((k_trace_gen<K, C, true>), grid, tb, 0, st, g, r, c, n, d_n, fill, out);     \
+        if (sparse) hipLaunchKernelGGL((k_trace_gen<K, C, true>), grid, tb, 0, st, g, r, c, n, d_n, fill, out);     \
         else hipLaunchKernelGGL((k_trace_gen<K, C, false>), grid, tb, 0, st, g, r, c, n, d_n, fill, out);          \
     } while (0)
     if (g.kind == 0) {

@@ -121,7 +121,7 @@ def test_trace_store_equals_oracle(ctx, oracle, kind):
 
 
 @pytest.mark.parametrize("kind", [0, 1])
-@pytest.mark.parametrize("res", [(1, 1), (3, 5), (96, 128), (97, 127), (256, 192), (257, 192), (256, 384), (257, 384)])
+@pytest.mark.parametrize("res", [(1, 1), (3, 5), (96, 128), (97, 127), (256, 192), (257, 192), (256, 384), (257, 384), (512, 384), (512, 385)])
 def test_small_images_walk_ahead(ctx, oracle, kind, res):
     """images on either side of every count of rays per wave, with every output"""
     opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)

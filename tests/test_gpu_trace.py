@@ -438,7 +438,7 @@ def test_small_batches_walk_ahead(ctx, oracle, scene, kind, shadow):
     b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
     b.init(sa.FaceSoup(ctx, a))
     g = b.build()
-    sizes = [1, 63, 1_000, 12_288, 12_289, 24_576, 24_577, 49_152, 49_153, 98_304, 98_305]
+    sizes = [1, 63, 1_000, 12_288, 12_289, 24_576, 24_577, 49_152, 49_153, 98_304, 98_305, 196_608, 196_609]
     rays = sa.gen_random_rays(95, max(sizes), -0.2, 1.2)
     n = rays.shape[1]
     rays[3, ::11] = 0.0

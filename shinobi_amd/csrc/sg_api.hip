@@ -257,7 +257,7 @@ static size_t grid_layout(sg_grid* g, char* pool) {
         g->large.prej = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
         g->large.sacc = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
         g->large.srej = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
-        g->large.scan_scratch = take(scan_scratch_bytes(g->cap_P1));
+        g->large.scan_scratch = take(2 * scan_scratch_bytes(g->cap_P1));
     }
     if (g->p.keep_debug) {
         g->dbg_tri = (uint32_t*)take((size_t)N * 4 + 16);

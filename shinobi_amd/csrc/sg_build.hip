@@ -864,11 +864,12 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                                        uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
                                                        uint32_t* __restrict__ prej) {
     constexpr int kSlots = 4;
-    __shared__ uint32_t s_acc[kSlots], s_rej[kSlots];
+    __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots], s_info[kSlots][4];
     const uint32_t P1v = h->P1_valid;
     const uint32_t base = blockIdx.x * kBlock;
     if (base >= P1v) return;
-    if (threadIdx.x < kSlots) s_acc[threadIdx.x] = s_rej[threadIdx.x] = 0;
+    if (threadIdx.x < kSlots) s_acc[threadIdx.x] = s_rej[threadIdx.x] = s_open[threadIdx.x] = 0;
+    if (threadIdx.x < 4 * kSlots) s_info[threadIdx.x >> 2][threadIdx.x & 3] = 0;
     const LeafParams L = read_leaf_params(h);
     const uint32_t Tp = leaf_sums_stride(T);
     const uint32_t i = base + threadIdx.x;
@@ -916,13 +917,17 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
         }
         const uint2 box = pair_box(st, c, mask);
         boxes[i] = box;
-        if (box.x == kBoxOpen && tile < T) info[4 * (size_t)T + tile] = 1u;
+        if (box.x == kBoxOpen && tile < T) {
+            const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
+            if (slot < kSlots) s_open[slot] = 1u;
+            else info[4 * (size_t)T + tile] = 1u;
+        }
         if (counted && pacc) {   // per-pair totals for the parallel emission of oversize tiles
             pacc[i] = acc;
             prej[i] = c - acc;
         }
         if (tile < T) {
-            if (counted) {
+            if (counted && !pacc) {
                 const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
                 if (slot < kSlots) {
                     if (acc) atomicAdd(&s_acc[slot], acc);
@@ -935,10 +940,16 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
             if (rg.x == i) {   // first pair of its top cell
                 const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
                 const uint32_t nl = (cl.y & 0xFFu) * ((cl.y >> 8) & 0xFFu) * ((cl.y >> 16) & 0xFFu);
-                atomicMax(&info[4 * (size_t)tile + 0], ~i);
-                atomicMax(&info[4 * (size_t)tile + 1], rg.y);
-                atomicMax(&info[4 * (size_t)tile + 2], ~cl.x);
-                atomicMax(&info[4 * (size_t)tile + 3], cl.x + nl);
+                // folded in LDS: the top cells of a tile, up to 512 where they
+                // hold few pairs each, would wait for the same four words in
+                // memory (502,000-triangle cluster, 9,000 such cells: k_leaf_count
+                // 103 -> 10 us)
+                const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
+                const uint32_t v[4] = {~i, rg.y, ~cl.x, cl.x + nl};
+                if (slot < kSlots)
+                    for (int k = 0; k < 4; ++k) atomicMax(&s_info[slot][k], v[k]);
+                else
+                    for (int k = 0; k < 4; ++k) atomicMax(&info[4 * (size_t)tile + k], v[k]);
             }
         }
     }
@@ -949,7 +960,28 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
         if (tile < T && (slot == 0 || tile != tile0)) {
             if (s_acc[slot]) atomicAdd(&sums[tile], s_acc[slot]);
             if (s_rej[slot]) atomicAdd(&sums[Tp + tile], s_rej[slot]);
+            if (s_open[slot]) info[4 * (size_t)T + tile] = 1u;
+            if (s_info[slot][0])
+                for (int k = 0; k < 4; ++k) atomicMax(&info[4 * (size_t)tile + k], s_info[slot][k]);
         }
+    }
+}
+
+// the grand totals (accepted ta, rejected tr) and the header's leaf-pair counts
+SG_D void leaf_totals(GridHeader* h, const BuildArgs& a, uint32_t* __restrict__ sums, uint32_t T, uint32_t ta,
+                      uint32_t tr) {
+    const uint32_t Tp = leaf_sums_stride(T);
+    const uint64_t total = (uint64_t)ta + tr;
+    sums[2 * (size_t)Tp] = ta;
+    sums[2 * (size_t)Tp + 1] = tr;
+    h->need_P2 = (uint32_t)min(total, (uint64_t)0xFFFFFFFFu);
+    if (total > a.cap_P2) {
+        atomicOr(&h->status, ST_CAP_P2);
+        h->P2 = a.cap_P2;
+        h->P2_valid = min(ta, a.cap_P2);
+    } else {
+        h->P2 = (uint32_t)total;
+        h->P2_valid = ta;
     }
 }
 
@@ -963,8 +995,7 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
                                                     const uint32_t* __restrict__ top_vals,
                                                     const uint32_t* __restrict__ ranges,
                                                     const uint32_t* __restrict__ cells, uint32_t* __restrict__ sums,
-                                                    uint32_t T, uint32_t* __restrict__ pacc,
-                                                    uint32_t* __restrict__ prej) {
+                                                    uint32_t T) {
     constexpr int kPer = 16;
     __shared__ uint32_t s_w[16];
     __shared__ uint32_t s_tot[2];
@@ -980,10 +1011,6 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
             const uint32_t acc = wide_count<16>(L, st, s_tab, s_w);
             if (threadIdx.x == 0) {
                 const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
-                if (pacc) {
-                    pacc[i] = acc;
-                    prej[i] = c - acc;
-                }
                 if (tile < T) {
                     sums[tile] += acc;
                     sums[Tp + tile] += c - acc;
@@ -1042,21 +1069,61 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
     }
     if (tt == 0) s_tot[half] = run;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t ta = s_tot[0], tr = s_tot[1];
-        const uint64_t total = (uint64_t)ta + tr;
-        sums[2 * (size_t)Tp] = ta;
-        sums[2 * (size_t)Tp + 1] = tr;
-        h->need_P2 = (uint32_t)min(total, (uint64_t)0xFFFFFFFFu);
-        if (total > a.cap_P2) {
-            atomicOr(&h->status, ST_CAP_P2);
-            h->P2 = a.cap_P2;
-            h->P2_valid = min(ta, a.cap_P2);
-        } else {
-            h->P2 = (uint32_t)total;
-            h->P2_valid = ta;
+    if (threadIdx.x == 0) leaf_totals(h, a, sums, T, s_tot[0], s_tot[1]);
+}
+
+// With per-pair totals (LeafLarge), in place of k_leaf_scan: the tile totals
+// come from the scans of those, so that k_leaf_count's blocks need not add to
+// the totals of one tile, a dense top cell's, in turn (507,000 pairs, with
+// the scans side by side: rebuild 350 -> 329 us).  First the wide boxes k_leaf_count listed, a block each ...
+__global__ __launch_bounds__(1024) void k_leaf_wide(TriSoA t, GridHeader* h, const uint32_t* __restrict__ top_keys,
+                                                    const uint32_t* __restrict__ top_vals,
+                                                    const uint32_t* __restrict__ cells,
+                                                    const uint32_t* __restrict__ sums, uint32_t T,
+                                                    uint32_t* __restrict__ pacc, uint32_t* __restrict__ prej) {
+    __shared__ uint32_t s_w[16];
+    __shared__ float s_tab[3][kAxisMax];
+    const uint32_t* list = sums + 2 * (size_t)leaf_sums_stride(T) + 2;
+    const uint32_t n_wide = min(list[0], kWideCap);
+    if (blockIdx.x >= n_wide) return;
+    const LeafParams L = read_leaf_params(h);
+    for (uint32_t k = blockIdx.x; k < n_wide; k += gridDim.x) {
+        const uint32_t i = list[2 + k];
+        LeafSetup st;
+        const uint32_t c = leaf_pair(t, L, h, top_keys[i], top_vals[i], cells, st);
+        const uint32_t acc = wide_count<16>(L, st, s_tab, s_w);
+        if (threadIdx.x == 0) {
+            pacc[i] = acc;
+            prej[i] = c - acc;
         }
     }
+}
+
+// ... then, from the exclusive scans of the per-pair totals, the totals before
+// each tile: those before the first top cell that starts at or after pair
+// kLeafTile * tile.
+__global__ __launch_bounds__(kBlock) void k_leaf_tile_sums(GridHeader* h, BuildArgs a,
+                                                           const uint32_t* __restrict__ top_keys,
+                                                           const uint32_t* __restrict__ ranges,
+                                                           const uint32_t* __restrict__ pacc,
+                                                           const uint32_t* __restrict__ prej,
+                                                           const uint32_t* __restrict__ sacc,
+                                                           const uint32_t* __restrict__ srej,
+                                                           uint32_t* __restrict__ sums, uint32_t T) {
+    const uint32_t P1v = min(h->P1_valid, a.cap_P1), C1 = h->C1, tile = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t ta = P1v ? sacc[P1v - 1u] + pacc[P1v - 1u] : 0u, tr = P1v ? srej[P1v - 1u] + prej[P1v - 1u] : 0u;
+    if (tile == 0) leaf_totals(h, a, sums, T, ta, tr);
+    if (tile >= T) return;
+    uint32_t i = tile * kLeafTile;
+    if (i < P1v) {
+        const uint32_t key = top_keys[i];
+        if (key < C1) {
+            const uint2 rg = reinterpret_cast<const uint2*>(ranges)[key];
+            if (rg.x != i) i = rg.y;
+        }
+    }
+    sums[tile] = i < P1v ? sacc[i] : ta;
+    sums[leaf_sums_stride(T) + tile] = i < P1v ? srej[i] : tr;
 }
 
 // Where tile b's pairs go: prefixes from k_leaf_scan, tile bounds and leaf
@@ -1799,8 +1866,18 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
                            sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr);
-    hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges, cells, sums, T,
-                       large ? large->pacc : nullptr, large ? large->prej : nullptr);
+    if (large) {
+        const uint32_t* in[2] = {large->pacc, large->prej};
+        uint32_t* out[2] = {large->sacc, large->srej};
+        hipLaunchKernelGGL(k_leaf_wide, dim3(64), dim3(1024), 0, st, t, h, top_keys, top_vals, cells, sums, T,
+                           large->pacc, large->prej);
+        launch_scan_two(in, out, a.cap_P1, large->scan_scratch, st);
+        hipLaunchKernelGGL(k_leaf_tile_sums, dim3((T + kBlock - 1) / kBlock), dim3(kBlock), 0, st, h, a, top_keys,
+                           ranges, large->pacc, large->prej, large->sacc, large->srej, sums, T);
+    } else {
+        hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges, cells, sums,
+                           T);
+    }
     // with `large`, the global sort and k_ranges need every key; without it
     // the tiles write the leaf ranges and the keys are kept for keep_debug
     uint32_t* lv = large ? nullptr : leaves;
@@ -1812,8 +1889,6 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
                        top_keys, top_vals, cells, boxes, keys, vals, refs, sums, info, T, lv, write_keys, todo, todo + 1,
                        tmp_keys, tmp_vals);
     if (large) {
-        launch_scan(large->pacc, large->sacc, a.cap_P1, false, large->scan_scratch, st);
-        launch_scan(large->prej, large->srej, a.cap_P1, false, large->scan_scratch, st);
         uint32_t pb = (a.cap_P1 + kBlock - 1) / kBlock;
         pb = pb < 1 ? 1 : (pb > 4096 ? 4096 : pb);
         hipLaunchKernelGGL(k_leaf_emit_par, dim3(pb), dim3(kBlock), 0, st, t, h, a, top_keys, top_vals, ranges, cells,

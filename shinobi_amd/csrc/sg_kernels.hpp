@@ -144,7 +144,7 @@ size_t leaf_info_words(uint32_t n);
 // them such a tile is emitted by one block.
 struct LeafLarge {
     uint32_t *pacc, *prej, *sacc, *srej;
-    void* scan_scratch;   // scan_scratch_bytes(cap_P1)
+    void* scan_scratch;   // twice scan_scratch_bytes(cap_P1)
 };
 // refs: reference records of the accepted pairs of sorted tiles.  Without
 // `large`, a tile too large for LDS is emitted and sorted by one block
@@ -238,6 +238,8 @@ void launch_multi_sort(MultiSortStep step, int rb, int pass, const UniJob* jobs,
 size_t scan_scratch_bytes(uint32_t n);
 void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, bool inclusive, void* scratch,
                  hipStream_t st);
+// exclusive scans of two arrays; scratch: twice scan_scratch_bytes(n)
+void launch_scan_two(const uint32_t* const in[2], uint32_t* const out[2], uint32_t n, void* scratch, hipStream_t st);
 
 // ---------------------------------------------------------------- traversal
 void launch_prep_tris(const TriSoA& t, uint32_t n, hipStream_t st);

@@ -369,9 +369,19 @@ size_t scan_scratch_bytes(uint32_t n) {
     return ((tiles + 4) * sizeof(uint32_t) + 15) & ~(size_t)15;
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_up(const uint32_t* __restrict__ in, uint32_t n,
-                                                    uint32_t* __restrict__ sums) {
+// one or two arrays of the same length, each with its own tile sums: grid row
+// blockIdx.y takes one (two scans of half a million values: 31 us one after the
+// other, 16 us side by side)
+struct ScanArrays {
+    const uint32_t* in[2];
+    uint32_t* out[2];
+    uint32_t* sums[2];
+};
+
+__global__ __launch_bounds__(kBlock) void k_scan_up(ScanArrays a, uint32_t n) {
     __shared__ uint32_t s_red[kBlock / 64];
+    const uint32_t* __restrict__ in = a.in[blockIdx.y];
+    uint32_t* __restrict__ sums = a.sums[blockIdx.y];
     const uint32_t base = blockIdx.x * kScanTile;
     uint32_t acc = 0;
     for (uint32_t i = base + threadIdx.x; i < min(n, base + (uint32_t)kScanTile); i += kBlock) acc += in[i];
@@ -380,8 +390,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_up(const uint32_t* __restrict__
 }
 
 // exclusive scan of the tile sums in place (one block of 1024 threads)
-__global__ __launch_bounds__(1024) void k_scan_sums(uint32_t* sums, uint32_t tiles) {
+__global__ __launch_bounds__(1024) void k_scan_sums(ScanArrays a, uint32_t tiles) {
     __shared__ uint32_t s_scan[16];
+    uint32_t* sums = a.sums[blockIdx.y];
     uint32_t run = 0;
     for (uint32_t c0 = 0; c0 < tiles; c0 += 1024 * 4) {
         const uint32_t t0 = c0 + threadIdx.x * 4;
@@ -402,9 +413,11 @@ __global__ __launch_bounds__(1024) void k_scan_sums(uint32_t* sums, uint32_t til
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                      uint32_t n, int inclusive, const uint32_t* __restrict__ sums) {
+__global__ __launch_bounds__(kBlock) void k_scan_down(ScanArrays a, uint32_t n, int inclusive) {
     __shared__ uint32_t s_scan[kBlock / 64];
+    const uint32_t* __restrict__ in = a.in[blockIdx.y];
+    uint32_t* __restrict__ out = a.out[blockIdx.y];
+    const uint32_t* __restrict__ sums = a.sums[blockIdx.y];
     const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
     uint32_t sum = 0;
@@ -439,14 +452,25 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t* __restrict
     }
 }
 
-// in and out must be 16-byte aligned (device allocations are)
-void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, bool inclusive, void* scratch, hipStream_t st) {
+static void scan_arrays(const ScanArrays& a, uint32_t count, uint32_t n, bool inclusive, hipStream_t st) {
     if (n == 0) return;
     const uint32_t tiles = (n + kScanTile - 1) / kScanTile;
-    uint32_t* sums = reinterpret_cast<uint32_t*>(scratch);
-    hipLaunchKernelGGL(k_scan_up, dim3(tiles), dim3(kBlock), 0, st, in, n, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, st, sums, tiles);
-    hipLaunchKernelGGL(k_scan_down, dim3(tiles), dim3(kBlock), 0, st, in, out, n, inclusive ? 1 : 0, sums);
+    hipLaunchKernelGGL(k_scan_up, dim3(tiles, count), dim3(kBlock), 0, st, a, n);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1, count), dim3(1024), 0, st, a, tiles);
+    hipLaunchKernelGGL(k_scan_down, dim3(tiles, count), dim3(kBlock), 0, st, a, n, inclusive ? 1 : 0);
+}
+
+// in and out must be 16-byte aligned (device allocations are)
+void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, bool inclusive, void* scratch, hipStream_t st) {
+    scan_arrays(ScanArrays{{in, nullptr}, {out, nullptr}, {reinterpret_cast<uint32_t*>(scratch), nullptr}}, 1, n,
+                inclusive, st);
+}
+
+void launch_scan_two(const uint32_t* const in[2], uint32_t* const out[2], uint32_t n, void* scratch, hipStream_t st) {
+    char* p = reinterpret_cast<char*>(scratch);
+    scan_arrays(ScanArrays{{in[0], in[1]}, {out[0], out[1]},
+                           {reinterpret_cast<uint32_t*>(p), reinterpret_cast<uint32_t*>(p + scan_scratch_bytes(n))}},
+                2, n, false, st);
 }
 
 }  // namespace sg

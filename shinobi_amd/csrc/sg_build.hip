@@ -899,6 +899,10 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
             if (!plane_tested(st) && kmax < L.C2) {
                 acc = c;
                 mask = c >= 32u ? 0xFFFFFFFFu : (1u << c) - 1u;
+                if (pacc && wide_box(L, st, c)) {   // listed for its emission
+                    const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
+                    if (w < kWideCap) sums[2 * (size_t)Tp + 4 + w] = i;
+                }
             } else {
                 if (wide_box(L, st, c)) {   // k_leaf_scan counts it
                     const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
@@ -1729,6 +1733,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
     __shared__ float s_tab[3][kAxisMax];
     const LeafParams L = read_leaf_params(h);
     const uint32_t P1v = min(h->P1_valid, a.cap_P1);
+    const bool listed = sums[2 * (size_t)leaf_sums_stride(T) + 2] <= kWideCap;   // k_leaf_wide_emit has the wide boxes
     for (uint32_t base = blockIdx.x * kBlock; base < P1v; base += gridDim.x * kBlock) {
         if (threadIdx.x == 0) s_nwide = 0;
         __syncthreads();
@@ -1754,7 +1759,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
             LeafSetup s;
             const uint32_t c = leaf_pair(t, L, h, key, tri, cells, s);
             if (wide_box(L, s, c)) {
-                s_wide[atomicAdd(&s_nwide, 1u)] = i;
+                if (!listed) s_wide[atomicAdd(&s_nwide, 1u)] = i;
             } else if (c) {
                 uint32_t pa = acc_slot(i), pr = rej_slot(i);
                 leaf_visit(L, s, [&](uint32_t k2, bool ok) {
@@ -1775,6 +1780,47 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
             wide_emit<kBlock / 64>(L, s, s_tab, s_scan, wtri, acc_slot(w), rej_slot(w), prej[w], a.cap_P2, keys, vals);
         }
         __syncthreads();   // the list is free for the next chunk
+    }
+}
+
+// The wide boxes of oversize tiles, when k_leaf_count could list them all: one
+// block of k_leaf_emit_par took 40 us for the 66,612 cells of one box, 63,000
+// of them rejected.  While there are fewer of them than blocks, several blocks
+// share a box: its rejected pairs, all alike, are split over them and the
+// first emits the accepted ones.
+constexpr uint32_t kWideBlocks = 64;
+__global__ __launch_bounds__(1024) void k_leaf_wide_emit(TriSoA t, GridHeader* h, BuildArgs a,
+                                                         const uint32_t* __restrict__ top_keys,
+                                                         const uint32_t* __restrict__ top_vals,
+                                                         const uint32_t* __restrict__ ranges,
+                                                         const uint32_t* __restrict__ cells,
+                                                         uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                         const uint32_t* __restrict__ sums,
+                                                         const uint32_t* __restrict__ info, uint32_t T,
+                                                         const uint32_t* __restrict__ prej,
+                                                         const uint32_t* __restrict__ sacc,
+                                                         const uint32_t* __restrict__ srej) {
+    __shared__ uint32_t s_scan[16];
+    __shared__ float s_tab[3][kAxisMax];
+    const uint32_t* list = sums + 2 * (size_t)leaf_sums_stride(T) + 2;
+    const uint32_t n = list[0];
+    if (n == 0 || n > kWideCap) return;
+    const uint32_t parts = max(1u, gridDim.x / n), part = blockIdx.x % parts;
+    const LeafParams L = read_leaf_params(h);
+    for (uint32_t k = blockIdx.x / parts; k < n; k += gridDim.x / parts) {
+        const uint32_t i = list[2 + k], key = top_keys[i], tri = top_vals[i];
+        const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
+        LeafTilePlan q;
+        q.mode = LEAF_NONE;
+        if (tile < T) leaf_tile_plan(a, sums, info, T, tile, q);
+        if (q.mode != LEAF_OVERSIZE) continue;
+        const uint32_t pr = q.tot_acc + q.pre_rej + (srej[i] - srej[q.a0]), rej = prej[i];
+        for (uint32_t j = part * 1024u + threadIdx.x; j < rej; j += parts * 1024u)
+            leaf_reject(pr + j, 1u, tri, a.cap_P2, L.C2, keys, vals, 1);
+        if (part) continue;
+        LeafSetup s;
+        leaf_pair(t, L, h, key, tri, cells, s);
+        wide_emit<16>(L, s, s_tab, s_scan, tri, q.pre_acc + (sacc[i] - sacc[q.a0]), 0u, 0u, a.cap_P2, keys, vals);
     }
 }
 
@@ -1869,7 +1915,7 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     if (large) {
         const uint32_t* in[2] = {large->pacc, large->prej};
         uint32_t* out[2] = {large->sacc, large->srej};
-        hipLaunchKernelGGL(k_leaf_wide, dim3(64), dim3(1024), 0, st, t, h, top_keys, top_vals, cells, sums, T,
+        hipLaunchKernelGGL(k_leaf_wide, dim3(kWideBlocks), dim3(1024), 0, st, t, h, top_keys, top_vals, cells, sums, T,
                            large->pacc, large->prej);
         launch_scan_two(in, out, a.cap_P1, large->scan_scratch, st);
         hipLaunchKernelGGL(k_leaf_tile_sums, dim3((T + kBlock - 1) / kBlock), dim3(kBlock), 0, st, h, a, top_keys,
@@ -1893,6 +1939,8 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
         pb = pb < 1 ? 1 : (pb > 4096 ? 4096 : pb);
         hipLaunchKernelGGL(k_leaf_emit_par, dim3(pb), dim3(kBlock), 0, st, t, h, a, top_keys, top_vals, ranges, cells,
                            keys, vals, sums, info, T, large->prej, large->sacc, large->srej);
+        hipLaunchKernelGGL(k_leaf_wide_emit, dim3(kWideBlocks), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges,
+                           cells, keys, vals, sums, info, T, large->prej, large->sacc, large->srej);
     }
 }
 

@@ -22,10 +22,12 @@ namespace sg {
 // Keys per thread.  A tile of 16 x 256 keys writes its digit runs in whole
 // cache lines; a small sort then has few tiles, and each waits for 16 ranking
 // rounds in a row, so sorts of up to kSmallSort pairs take 4 keys per thread.
-// (26,000 pairs: k_sort_down 11.4 -> 6.5 us a pass, k_sort_up 4.1 -> 2.4; at
-// 2.46 M pairs the smaller tiles were 10 us slower.)
+// (26,000 pairs: k_sort_down 11.4 -> 6.5 us a pass, k_sort_up 4.1 -> 2.4; 546,000
+// pairs of a capacity of a million and more: 11.2 -> 7.8 and 4.7 -> 4.3; at
+// 2.46 M pairs the smaller tiles were 10 us slower.)  The line is drawn on the
+// capacity, which a grid's build leaves at about twice its pairs.
 constexpr int kSortItems = 16, kSmallItems = 4;
-constexpr uint32_t kSmallSort = 1u << 20;
+constexpr uint32_t kSmallSort = 1u << 21;
 // Up to this many tiles a tile's digit offsets are folded by the downsweep
 // itself from counts stored [tile][digit] (one row of them per tile before
 // it), and the scan launch between the sweeps, 3 us and a gap, falls away.

@@ -42,7 +42,7 @@ def test_sort_is_stable_and_matches_numpy(ctx, radix_bits, n, key_bits, dup):
 
 
 @pytest.mark.parametrize("radix_bits", [4, 6, 8])
-@pytest.mark.parametrize("n", [255, 1023, 1025, 65_535, 65_536, 65_537, 2**20 - 1, 2**20, 2**20 + 1])
+@pytest.mark.parametrize("n", [255, 1023, 1025, 65_535, 65_536, 65_537, 2**21 - 1, 2**21, 2**21 + 1])
 def test_sort_forms_at_their_edges(ctx, radix_bits, n):
     """tiles of 1024 and 4096 keys, digit offsets folded in the downsweep (up
     to 64 tiles) or scanned by a launch of their own: either side of each edge"""

@@ -159,9 +159,34 @@ static TriSoA scene_soa(const sg_scene* s) {
     return t;
 }
 
+// Can a kernel read the scene's n floats at p?  Memory of the scene's device,
+// within one allocation, aligned, outside the scene's own arrays; anything
+// else is left to the runtime's copies, which check it or reach it.
+static bool kernel_source(const sg_scene* s, const float* p) {
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeDevice || a.device != s->device ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+        clear_last_error();
+        return false;
+    }
+    const uintptr_t q = (uintptr_t)p, b = (uintptr_t)base, own = (uintptr_t)s->soa;
+    const size_t bytes = (size_t)s->n * sizeof(float), own_bytes = 9 * s->stride * sizeof(float);
+    return q % sizeof(float) == 0 && q >= b && q - b <= size && bytes <= size - (q - b) &&
+           (q + bytes <= own || q >= own + own_bytes);
+}
+
 static sg_status scene_upload(sg_scene* s, const float* const soa9[9], int on_dev, hipStream_t st) {
     clear_last_error();
     const size_t b = (size_t)s->n * sizeof(float);
+    bool direct = on_dev != 0;
+    for (int i = 0; direct && i < 9; ++i) direct = soa9[i] && kernel_source(s, soa9[i]);
+    if (direct) {
+        launch_set_tris(soa9, s->soa, s->stride, s->rec, s->n, st);
+        HIPCHK(hipGetLastError());
+        return SG_OK;
+    }
     for (int i = 0; i < 9; ++i) {
         if (!soa9[i]) return SG_ERR_INVALID_ARG;
         HIPCHK(hipMemcpyAsync(s->soa + (size_t)i * s->stride, soa9[i], b,

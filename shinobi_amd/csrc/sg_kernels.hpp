@@ -243,6 +243,7 @@ void launch_scan_two(const uint32_t* const in[2], uint32_t* const out[2], uint32
 
 // ---------------------------------------------------------------- traversal
 void launch_prep_tris(const TriSoA& t, uint32_t n, hipStream_t st);
+void launch_set_tris(const float* const src[9], float* soa, size_t stride, float* rec, uint32_t n, hipStream_t st);
 // one (grid, ray batch) item of a multi-batch launch; chunk0 = first 64-ray
 // chunk of the item in the concatenation of all items (items sorted by it)
 struct TraceItem {

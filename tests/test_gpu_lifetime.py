@@ -52,3 +52,43 @@ def test_grid_destroyed_after_its_context_c_abi():
     with sa.Context(0) as ctx:
         _, _, (pg, tg) = _trace_once(ctx, scene9, rays7)
         assert (pg != sa.MISS).any()
+
+
+@pytest.mark.parametrize("n", [100, 255, 257, 10_001])
+def test_scene_update_from_device_memory(ctx, n):
+    """one launch for sources a kernel may read, copies for the scene's own
+    arrays: the scene then builds as from host memory, also under capture"""
+    from shinobi_amd import _lib as L
+    lib = sa.lib()
+    a, b = sa.gen_soup(5, n, 0.05), sa.gen_soup(6, n, 0.05)
+    buf = ctx.upload(b)
+    base = int(buf.ptr.value)
+    ptrs = L.Float9(*[base + 4 * n * i for i in range(9)])
+
+    def arrays(scene):
+        d = sa.FastSimpleGridBuilder(ctx, lam=5.0)
+        d.init(scene)
+        g = d.build()
+        return g.download("top_ranges"), g.download("indices")
+
+    ref = arrays(sa.FaceSoup(ctx, b))
+    scene = sa.FaceSoup(ctx, a)
+    assert lib.sg_scene_update(scene.h, ptrs, 1, ctx.stream) == 0
+    for x, y in zip(arrays(scene), ref):
+        np.testing.assert_array_equal(x, y)
+    # captured, with other vertices in the source at the replay
+    scene2 = sa.FaceSoup(ctx, b)
+    with sa.Graph.capture(ctx) as graph:
+        assert lib.sg_scene_update(scene2.h, ptrs, 1, ctx.stream) == 0
+    buf.upload(a)
+    graph.launch()
+    ctx.sync()
+    for x, y in zip(arrays(scene2), arrays(sa.FaceSoup(ctx, a))):
+        np.testing.assert_array_equal(x, y)
+    # the scene's own arrays as the source: unchanged
+    own = L.Float9()
+    assert lib.sg_scene_device_soa(scene.h, own) == 0
+    assert lib.sg_scene_update(scene.h, own, 1, ctx.stream) == 0
+    for x, y in zip(arrays(scene), ref):
+        np.testing.assert_array_equal(x, y)
+    assert lib.sg_scene_update(scene.h, L.Float9(*([None] * 9)), 1, ctx.stream) != 0

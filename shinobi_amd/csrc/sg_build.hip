@@ -8,6 +8,8 @@
 // every pair lands at the slot that a serial scan of the counts in canonical
 // order would give it: triangles (or sorted top pairs) ascending, then the
 // reference's z/y/x loop order.
+#include <type_traits>
+
 #include "sg_device.hpp"
 #include "sg_kernels.hpp"
 
@@ -1175,22 +1177,34 @@ SG_D uint32_t count_add(uint16_t* s_cnt, uint32_t k) {
 // Exclusive scan of s_cnt[0..span) in place by a block of NW waves, and the
 // ranges of the tile's leaf cells, which no other tile holds: {first, last+1}
 // of its references, {0, 0} without (the leaf cells of empty top cells between
-// the tile's are zero as well); n_ranges of them lie below C2.
-template <int NW>
+// the tile's are zero as well); n_ranges of them lie below C2.  W words, 2 W
+// cells, per thread and round: one where a tile rarely takes two rounds (the
+// ranges' stores are then contiguous; four cost the height field 1 %), four for
+// larger tiles, whose rounds of two barriers took a tenth of their time.
+template <int NW, int W>
 SG_D void leaf_scan_counts(uint16_t* s_cnt, uint32_t span, uint32_t first, uint32_t* s_scan,
                            uint2* __restrict__ ranges, uint32_t n_ranges) {
+    uint32_t* words = reinterpret_cast<uint32_t*>(s_cnt);
     uint32_t run = 0;
-    for (uint32_t k0 = 0; k0 < span; k0 += NW * 128) {   // two cells, one word, per thread
-        const uint32_t k = k0 + 2u * threadIdx.x;
-        const uint32_t w = k < span ? reinterpret_cast<uint32_t*>(s_cnt)[k >> 1] : 0u;
-        const uint32_t n0 = w & 0xFFFFu, n1 = w >> 16;
+    for (uint32_t k0 = 0; k0 < span; k0 += NW * 128 * W) {
+        const uint32_t k = k0 + 2u * W * threadIdx.x;
+        uint32_t w[W], sum = 0;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            w[j] = k + 2u * j < span ? words[(k >> 1) + j] : 0u;
+            sum += (w[j] & 0xFFFFu) + (w[j] >> 16);
+        }
         uint32_t agg;
-        const uint32_t p = run + block_excl_scan<NW>(n0 + n1, &agg, s_scan);
-        if (k < span) reinterpret_cast<uint32_t*>(s_cnt)[k >> 1] = p | (p + n0) << 16;
-        const uint32_t f = first + p;
-        if (k < n_ranges && k < span) ranges[k] = n0 ? make_uint2(f, f + n0) : make_uint2(0u, 0u);
-        if (k + 1u < n_ranges && k + 1u < span)
-            ranges[k + 1u] = n1 ? make_uint2(f + n0, f + n0 + n1) : make_uint2(0u, 0u);
+        uint32_t p = run + block_excl_scan<NW>(sum, &agg, s_scan);
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            const uint32_t c = k + 2u * j, n0 = w[j] & 0xFFFFu, n1 = w[j] >> 16, f = first + p;
+            if (c < span) words[(k >> 1) + j] = p | (p + n0) << 16;
+            if (c < n_ranges && c < span) ranges[c] = n0 ? make_uint2(f, f + n0) : make_uint2(0u, 0u);
+            if (c + 1u < n_ranges && c + 1u < span)
+                ranges[c + 1u] = n1 ? make_uint2(f + n0, f + n0 + n1) : make_uint2(0u, 0u);
+            p += n0 + n1;
+        }
         run += agg;
     }
     __syncthreads();
@@ -1328,7 +1342,7 @@ SG_D void leaf_emit_small(const LeafTilePlan& q, const uint2* __restrict__ boxes
         }
     }
     __syncthreads();
-    leaf_scan_counts<NW>(s_cnt, q.span, q.pre_acc, s_scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
+    leaf_scan_counts<NW, 1>(s_cnt, q.span, q.pre_acc, s_scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
                          leaves && C2 > q.kbase ? C2 - q.kbase : 0u);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -1464,7 +1478,8 @@ struct BigLds {
 // rounds, open boxes visited again, wide ones by the block.  Slice 0 also
 // writes the rejected pairs and the leaf ranges.  200,000-triangle sphere (12
 // such tiles, the largest of 20,456 accepted pairs): one block per tile 147
-// us, in slices 84 us (two fifths counting, one fifth listing); the global
+// us, in slices 84 us; with a count pass that does not wait for LDS and fewer
+// scan rounds 81 us (38,665-triangle ruins: rebuild 292 -> 274 us).  The global
 // sort and range passes that such tiles needed before took 130 us.
 SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams& L, GridHeader* h, const uint2* __restrict__ boxes,
                         const TriSoA& t, uint32_t cap, const uint32_t* __restrict__ top_keys,
@@ -1475,8 +1490,11 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
     for (uint32_t k = threadIdx.x; 2u * k < q.span; k += kBigBlock) reinterpret_cast<uint32_t*>(s.cnt)[k] = 0;
     uint32_t run = q.tot_acc + q.pre_rej, k0 = 0, k1 = q.span, base = 0;
     if (threadIdx.x == 0) s.k0 = s.k1 = q.span;
-    // pass 0 counts and writes the rejected pairs, pass 1 fills the lists
-    for (int pass = 0; pass < 2; ++pass) {
+    // One pass over the top pairs counts and writes the rejected pairs, another
+    // fills the lists; apart, so that the first adds without waiting for the
+    // old counts.
+    auto over_tops = [&](auto list) {
+        constexpr bool LIST = decltype(list)::value;
         for (uint32_t c0 = q.a0; c0 < q.a1; c0 += kBigBlock) {
             __syncthreads();
             if (threadIdx.x == 0) s.n_wide = 0;
@@ -1485,9 +1503,12 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
             uint32_t rej = 0, tri = 0;
             // a leaf cell of the tile that pair p lies in
             auto add = [&](uint32_t k, uint32_t p) {
-                if (k < k0 || k >= k1) return;
-                const uint32_t at = count_add(s.cnt, k) - base;
-                if (pass && at < kLeafSlice + LeafBig::tops) s.ord[at] = k << kTopBits | (p - q.a0);
+                if (!LIST) {
+                    if (k < q.span) count_add(s.cnt, k);
+                } else if (k >= k0 && k < k1) {
+                    const uint32_t at = count_add(s.cnt, k) - base;
+                    if (at < kLeafSlice + LeafBig::tops) s.ord[at] = k << kTopBits | (p - q.a0);
+                }
             };
             if (i < q.a1) {
                 const uint32_t key = top_keys[i];
@@ -1524,7 +1545,7 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
                 acc = block_sum<NW>(acc, s.scan);
                 if (threadIdx.x == s.wide[w]) rej = c - acc;
             }
-            if (pass || slice || !q.rej) continue;
+            if (LIST || slice || !q.rej) continue;
             uint32_t agg;
             const uint32_t r = run + block_excl_scan<NW>(rej, &agg, s.scan);
             run += agg;
@@ -1548,24 +1569,23 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
             }
         }
         __syncthreads();
-        if (pass == 0) {
-            leaf_scan_counts<NW>(s.cnt, q.span, q.pre_acc, s.scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
-                                 leaves && slice == 0 && L.C2 > q.kbase ? L.C2 - q.kbase : 0u);
-            // the slice's leaf cells [k0, k1) and the place of its first pair
-            for (uint32_t k = threadIdx.x; k < q.span; k += kBigBlock) {
-                const uint32_t at = s.cnt[k], lo = slice * kLeafSlice, hi = lo + kLeafSlice;
-                const bool start = k == 0u;
-                const uint32_t before = start ? 0u : s.cnt[k - 1u];
-                if (at >= lo && (start || before < lo)) s.k0 = k;
-                if (at >= hi && (start || before < hi)) s.k1 = k;
-            }
-            __syncthreads();
-            k0 = s.k0;
-            k1 = s.k1;
-            base = k0 < q.span ? s.cnt[k0] : q.acc;
-        }
+    };
+    over_tops(std::false_type{});
+    leaf_scan_counts<NW, 4>(s.cnt, q.span, q.pre_acc, s.scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
+                         leaves && slice == 0 && L.C2 > q.kbase ? L.C2 - q.kbase : 0u);
+    // the slice's leaf cells [k0, k1) and the place of its first pair
+    for (uint32_t k = threadIdx.x; k < q.span; k += kBigBlock) {
+        const uint32_t at = s.cnt[k], lo = slice * kLeafSlice, hi = lo + kLeafSlice;
+        const bool start = k == 0u;
+        const uint32_t before = start ? 0u : s.cnt[k - 1u];
+        if (at >= lo && (start || before < lo)) s.k0 = k;
+        if (at >= hi && (start || before < hi)) s.k1 = k;
     }
     __syncthreads();
+    k0 = s.k0;
+    k1 = s.k1;
+    base = k0 < q.span ? s.cnt[k0] : q.acc;
+    over_tops(std::true_type{});
     if (k0 >= k1) return;
     leaf_sort_long<NW>(s.ord, s.cnt, k0, k1, base, s.bm + LeafBig::tops / 32 * wave_id(), (q.a1 - q.a0 + 31u) / 32u);
     const uint32_t n = min((uint32_t)s.cnt[k1 - 1u] - base, kLeafSlice + LeafBig::tops);

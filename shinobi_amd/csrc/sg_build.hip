@@ -555,8 +555,11 @@ struct LeafBig {
 // A tile of the larger kernel is taken by several blocks: slice s holds the
 // leaf cells whose lists begin in [s * kLeafSlice, (s+1) * kLeafSlice) of the
 // tile's accepted pairs.  Every block counts the whole tile, then lists, sorts
-// and writes its slice only.
-constexpr uint32_t kLeafSlice = 4096;
+// and writes its slice only.  Few tiles are so large, so their slices are small
+// to use the chip: 4096 / 2048 / 1024 / 512 / 256 pairs rebuild a 200,000-
+// triangle sphere in 174 / 162 / 153 / 147 / 164 us, the ruins scene, with more
+// such tiles, in 274 / 263 / 254 / 286 / 356 us.
+constexpr uint32_t kLeafSlice = 1024;
 constexpr uint32_t kSliceShift = 24, kSlicesMax = (LeafBig::pairs + kLeafSlice - 1) / kLeafSlice;
 constexpr int kTopBits = 13;                          // a list entry's top pair bits
 static_assert(LeafBig::tops <= 1u << kTopBits && LeafBig::pairs < 65536u, "list entries and 16-bit counts");
@@ -1478,8 +1481,9 @@ struct BigLds {
 // rounds, open boxes visited again, wide ones by the block.  Slice 0 also
 // writes the rejected pairs and the leaf ranges.  200,000-triangle sphere (12
 // such tiles, the largest of 20,456 accepted pairs): one block per tile 147
-// us, in slices 84 us; with a count pass that does not wait for LDS and fewer
-// scan rounds 81 us (38,665-triangle ruins: rebuild 292 -> 274 us).  The global
+// us, in slices of 4096 pairs 84 us; with a count pass that does not wait for
+// LDS and fewer scan rounds 81 us (38,665-triangle ruins: rebuild 292 -> 274
+// us), in slices of 1024 pairs 60 us.  The global
 // sort and range passes that such tiles needed before took 130 us.
 SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams& L, GridHeader* h, const uint2* __restrict__ boxes,
                         const TriSoA& t, uint32_t cap, const uint32_t* __restrict__ top_keys,

@@ -1531,7 +1531,12 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
                     }
                 } else if (box.x != kBoxEmpty) {
                     const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
-                    box_visit(box, cl.x - q.kbase, cl.y, [&](uint32_t k) { add(k, i); });
+                    // a box beside the slice has nothing to list
+                    const uint32_t crx = cl.y & 0xFFu, lo = cl.x - q.kbase + (box.x & 0xFFFFu),
+                                   hi = lo + ((box.x >> 16) & 31u) +
+                                        (((box.x >> 21) & 31u) + ((box.x >> 26) & 31u) * ((cl.y >> 8) & 0xFFu)) * crx;
+                    if (!LIST || (hi >= k0 && lo < k1))
+                        box_visit(box, cl.x - q.kbase, cl.y, [&](uint32_t k) { add(k, i); });
                     rej = box_cells(box.x) - (uint32_t)__popc(box.y);
                 }
             }

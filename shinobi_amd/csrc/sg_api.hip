@@ -332,7 +332,7 @@ static sg_status grid_alloc(sg_grid* g) {
 
 // Enqueue the whole build on `st`.  marks (optional, n_marks entries) are
 // hipEvent_t recorded at the phase boundaries: [0] start, [1] after
-// init+bounds, [2] top emission, [3] top sort, [4] top ranges, then for the
+// init+bounds, [2] parameters and top emission, [3] top sort, [4] top ranges, then for the
 // two-level grid [5] leaf cells, [6] leaf emission, [7] leaf sort, [8] leaf
 // ranges.
 // the build arguments of a grid's (re)build
@@ -419,9 +419,8 @@ static void enqueue_build(sg_grid* g, bool fixed_res, hipStream_t st, void* cons
     const ZeroSegs z = zero_segs(g);
     mark(0);
     launch_init_bounds(g->hdr, N, z, t, g->bpart, st);
-    launch_params(g->hdr, a, g->bpart, N, true, st);
     mark(1);
-    launch_top_emit(t, N, g->hdr, a, g->k1[0], g->v1[0], g->dbg_tri, g->sums_top, st);
+    launch_top_emit(t, N, g->hdr, a, g->bpart, g->k1[0], g->v1[0], g->dbg_tri, g->sums_top, st);
     mark(2);
     launch_sort_pairs(g->k1[0], g->v1[0], g->k1[1], g->v1[1], &g->hdr->P1, g->cap_P1, g->key_bits1, g->rb, g->sort1,
                       st);

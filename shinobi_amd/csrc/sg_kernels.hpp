@@ -126,8 +126,9 @@ void launch_params(GridHeader* h, const BuildArgs& a, const uint32_t* part, uint
 // triangles or top pairs, cell_tiles(C1) for the leaf-cell kernels
 size_t emit_tiles(uint32_t n);
 size_t cell_tiles(uint32_t n);
-void launch_top_emit(const TriSoA& t, uint32_t n, GridHeader* h, const BuildArgs& a, uint32_t* keys,
-                     uint32_t* vals, uint32_t* dbg, uint32_t* sums, hipStream_t st);
+// the parameters from the bounds partials (launch_params), then the top pairs
+void launch_top_emit(const TriSoA& t, uint32_t n, GridHeader* h, const BuildArgs& a, const uint32_t* part,
+                     uint32_t* keys, uint32_t* vals, uint32_t* dbg, uint32_t* sums, hipStream_t st);
 void launch_ranges(const uint32_t* keys, const uint32_t* d_n, uint32_t cap, const uint32_t* d_C,
                    uint32_t* cells, uint32_t* d_pvalid, hipStream_t st);
 void launch_leaf_cells(GridHeader* h, const BuildArgs& a, const uint32_t* ranges, uint32_t* cells,

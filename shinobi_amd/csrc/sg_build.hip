@@ -1784,7 +1784,7 @@ __global__ __launch_bounds__(kBigBlock) void k_leaf_emit_big(
 // Oversize tiles with one thread per top pair: pair i of tile t writes its
 // accepted pairs from pre_acc(t) + (sacc[i] - sacc[first pair of t]) and its
 // rejected ones likewise (sacc / srej: exclusive scans of the per-pair totals
-// of k_leaf_count), so the output is k_leaf_emit_large's, in parallel -- a
+// of k_leaf_count), so the output is leaf_emit_oversize's, in parallel -- a
 // top cell of 500k pairs (a dense cluster) no longer runs on one block.
 __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* h, BuildArgs a,
                                                           const uint32_t* __restrict__ top_keys,

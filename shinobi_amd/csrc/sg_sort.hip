@@ -14,6 +14,8 @@
 //
 // Scan (src/Utils/Scan.h:35-68): block sums, one-block scan of the sums,
 // then each block rescans its tile from its offset.
+#include <algorithm>
+
 #include "sg_device.hpp"
 #include "sg_kernels.hpp"
 
@@ -50,7 +52,11 @@ uint32_t multi_sort_tiles(uint32_t cap) { return (uint32_t)sort_tiles(cap, kSort
 size_t sort_scratch_words(uint32_t cap, int key_bits, int radix_bits) {
     const size_t R = (size_t)1 << radix_bits;
     const size_t passes = (size_t)sort_passes(key_bits, radix_bits);
-    size_t w = passes * R + R * (sort_tiles(cap, sort_items(cap)) + 1);
+    // a larger capacity never needs less: scratch grown by a larger call serves
+    // a smaller one under capture
+    size_t tiles = sort_tiles(cap, sort_items(cap));
+    if (cap > kSmallSort) tiles = std::max(tiles, sort_tiles(kSmallSort, kSmallItems));
+    size_t w = passes * R + R * (tiles + 1);
     return (w + 3) & ~(size_t)3;   // 16-byte multiple
 }
 

@@ -54,3 +54,26 @@ def test_sort_forms_at_their_edges(ctx, radix_bits, n):
     order = np.argsort(keys, kind="stable")
     np.testing.assert_array_equal(k, keys[order])
     np.testing.assert_array_equal(v, vals[order])
+
+
+def test_scratch_of_a_larger_sort_serves_a_smaller_one(ctx):
+    """across the size at which the sort's tiles change: a bounce whose scratch
+    a slightly larger call grew can be captured"""
+    n = 2**21 + 64
+    a = sa.gen_soup(3, 1_000, 0.05)
+    scene = sa.FaceSoup(ctx, a)
+    b = sa.FastSimpleGridBuilder(ctx, lam=5.0)
+    b.init(scene)
+    g = b.build()
+    rays, out = sa.RayBatch(ctx, sa.gen_random_rays(4, n, 0.0, 1.0)), sa.RayBatch(ctx, capacity=n)
+    prim, t = g.trace(rays)
+    order, count = sa.bounce_order("exit", grid=g), sa.DeviceBuffer(ctx, 4)
+    sa.bounce(ctx, scene, rays, prim, t, 7, out, count=count, order=order)
+    ctx.sync()
+    rays.n = 2**21
+    with sa.Graph.capture(ctx) as graph:
+        sa.bounce(ctx, scene, rays, prim, t, 7, out, count=count, order=order)
+    graph.launch()
+    ctx.sync()
+    hits = int((prim.download(np.uint32, 2**21) != sa.MISS).sum())
+    assert int(count.download(np.uint32, 1)[0]) == hits > 0

@@ -584,7 +584,10 @@ SG_D void uniform_start(const GView& g, const GParams& p, Ray& r, Walk& w, RemBi
 // 198 -> 40 us, 49,000 rays 430 -> 199; uniform 123 -> 39 and 223 -> 129;
 // 500,000-triangle dense cluster, 1,000 camera rays 146 -> 56 us (360 before
 // the whole wave tested its cells of hundreds of references).
-constexpr uint32_t kAheadCoop = 32;   // references left in a cell that make the whole wave test them
+// References left in a cell that make the whole wave test them: at 32, 98,000
+// random rays through the uniform grid of a height field took 153 us, at 20 131;
+// at 16 small images of it took 8 % longer again.
+constexpr uint32_t kAheadCoop = 20;
 SG_D uint64_t lanes_mask(uint32_t first, uint32_t count) {
     return (count >= 64u ? ~0ull : (1ull << count) - 1ull) << first;
 }
@@ -888,7 +891,11 @@ struct LeafAny {
 // non-empty ones side by side, or the whole group the first of them when its
 // leaf walk is long (a dense top cell).  A leaf walk starts with the t of
 // before; once one lowered it, the later ones are walked again.
-constexpr uint32_t kTopAhead = 16, kLeafAhead = 8, kLeafLong = 24;
+// (kLeafLong, the sum of the top cell's resolutions: a height field's leaf
+// walks end soon although its top cells are divided finely; 1,000 rays 36 us at
+// 24, 31 at 48, 12,000 rays 68 and 54, the dense cluster and soups equal.  16
+// lanes for a leaf walk: soup 40 -> 47 us; 8 top cells ahead: 3-10 % slower.)
+constexpr uint32_t kTopAhead = 16, kLeafAhead = 8, kLeafLong = 48;
 
 template <bool SHADOW>
 SG_D void walk_twolevel_ahead(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t G) {

@@ -366,7 +366,8 @@ static ZeroSegs zero_segs(const sg_grid* g) {
     };
     seg(g->ranges1, (size_t)g->cap_C1 * 8);
     if (two) {
-        // without the global leaf sort the emission writes every leaf range
+        // without the global leaf sort the leaf ranges are cleared where they
+        // are not written (see launch_leaf_emit)
         if (g->large_path) seg(g->leaves, (size_t)g->cap_C2 * 8);
         seg(g->sums_leaf, leaf_sums_words(g->cap_P1) * 4);
         seg(g->leaf_info, leaf_info_words(g->cap_P1) * 4);

@@ -544,7 +544,8 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
     if (k < C1) {
         reinterpret_cast<uint2*>(cells)[k] = make_uint2(prefix + local, bits);
         // an empty top cell's one leaf cell; the others' are written by the
-        // tiles that emit their pairs, so nothing else clears them
+        // tiles that emit their pairs, so nothing else clears them while the
+        // leaf resolutions lie in 1..255 (k_leaf_count clears the rest)
         if (leaves && !(bits & kNotEmpty) && prefix + local < a.cap_C2)
             reinterpret_cast<uint2*>(leaves)[prefix + local] = make_uint2(0u, 0u);
     }
@@ -906,9 +907,17 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                                        uint32_t* __restrict__ sums, uint32_t* __restrict__ info,
                                                        uint32_t T, uint32_t* __restrict__ dbg_counts,
                                                        uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
-                                                       uint32_t* __restrict__ prej) {
+                                                       uint32_t* __restrict__ prej, uint32_t* __restrict__ leaves) {
     constexpr int kSlots = 4;
     __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots], s_info[kSlots][4];
+    // A top cell reserves its leaf cells by the whole resolutions, its tile
+    // writes those within the packed bytes: beyond 255 on an axis (flagged by
+    // k_leaf_cells_count) the others are nobody's, so all are cleared here.
+    if (leaves && (h->status & ST_LEAF_RES)) {
+        const uint32_t C2 = h->C2;
+        for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < C2; k += gridDim.x * kBlock)
+            reinterpret_cast<uint2*>(leaves)[k] = make_uint2(0u, 0u);
+    }
     const uint32_t P1v = h->P1_valid;
     const uint32_t base = blockIdx.x * kBlock;
     if (base >= P1v) return;
@@ -1980,7 +1989,8 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     const uint32_t blocks = (a.cap_P1 + kBlock - 1) / kBlock;
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
-                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr);
+                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr,
+                           large ? nullptr : leaves);
     if (large) {
         const uint32_t* in[2] = {large->pacc, large->prej};
         uint32_t* out[2] = {large->sacc, large->srej};

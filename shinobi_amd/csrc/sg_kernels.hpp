@@ -152,10 +152,12 @@ struct LeafLarge {
 // (using tmp_keys / tmp_vals, buffers of the pairs' size) and no global leaf
 // sort is needed; with `large`, such tiles are emitted in parallel and left
 // to the global sort (launch_leaf_sort_fixup + launch_ref_records).
-// Without `large` the tiles also write the leaf ranges (`leaves`, zeroed by
-// the build's first launch) and the leaf keys only with a.keep_debug; with
-// it, every key is
-// written for the global sort and k_ranges.
+// Without `large` the tiles also write the leaf ranges and the leaf keys only
+// with a.keep_debug; with it, every key is written for the global sort and
+// k_ranges.  Who clears `leaves`: with `large`, the build's first launch, all
+// of it.  Without, launch_leaf_cells the one leaf cell of each empty top cell
+// and each tile its span before it writes the ranges there; in a grid flagged
+// ST_LEAF_RES, whose tiles' spans leave gaps, k_leaf_count all of it first.
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
                       const uint32_t* top_vals, const uint32_t* ranges, const uint32_t* cells, uint32_t* keys,
                       uint32_t* vals, uint32_t* tmp_keys, uint32_t* tmp_vals, float* refs, uint32_t* dbg,

@@ -451,3 +451,58 @@ def test_top_emission_forms_at_their_edges(ctx, oracle, n, size):
     _assert_top_level(g, og)
     g.rebuild()
     _assert_top_level(g, og)
+
+
+def _bar(n, seed, axis, thin, pile):
+    """n small triangles in the unit cube, the two other axes scaled by thin,
+    the first `pile` of them crowded into the lower half of the axis"""
+    r = np.random.default_rng(seed)
+    c = r.random((3, n)).astype(np.float32)
+    c[axis, : int(pile * n)] *= np.float32(0.45)
+    v = np.clip(c[None] + (r.random((3, 3, n)) - 0.5).astype(np.float32) * np.float32(0.01), 0, 1).astype(np.float32)
+    v *= np.array([1.0 if k == axis else thin for k in range(3)], np.float32)[:, None]
+    v[0, :, 0], v[0, axis, 1] = 0.0, 1.0
+    return np.ascontiguousarray(v.reshape(9, n), dtype=np.float32)
+
+
+@pytest.mark.parametrize("first", ["build", "rebuild"])
+@pytest.mark.parametrize("n,axis,thin,lam,cells,pile", [
+    (2060, 0, 1 / 64, 2.0, 1, 0.0),      # 256 leaf cells along the axis: the packed byte is 0
+    (2060, 2, 1 / 64, 3.0, 1, 0.0),      # 293: the byte is 37
+    (8000, 1, 1 / 256, 2.0, 3, 0.0),     # three top cells of more pairs than a small leaf tile holds
+    (900, 2, 1 / 256, 10.0, 3, 0.0),     # two top cells in a tile, one in the next
+    (300, 0, 1 / 256, 30.0, 3, 0.0),     # tiles of the small kernel
+    (12000, 1, 1 / 64, 2.0, 2, 0.95),    # rebuilt: an oversize tile that the grid's build did not meet
+])
+def test_leaf_ranges_beyond_the_packed_resolutions(ctx, oracle, n, axis, thin, lam, cells, pile, first):
+    """a grid flagged for leaf resolutions beyond 255, built or reached by a
+    rebuild: the reserved leaf cells that no tile writes are empty"""
+    res = tuple(cells if k == axis else 1 for k in range(3))
+    opt = dict(lam=5.0, top_divisor=1, lambda_leaf=lam, leaf_min_refs=16, res_override=res)
+    bar = _bar(n, 5, axis, thin, pile)
+    og = oracle.build_twolevel(bar, **opt)
+    assert og.status != 0
+    scene = sa.FaceSoup(ctx, bar if first == "build" else _bar(n, 6, axis, 1.0, 0.0))
+    b = sa.FastTwoLevelGridBuilder(ctx, **opt)
+    b.init(scene)
+    g = b.build()
+    if first == "rebuild":
+        assert g.info().status == 0
+        scene.upload_vertices(bar)
+        g.rebuild()
+    info = g.info()
+    assert info.status != 0 and (info.C2, info.P2, info.P2_valid) == (og.C2, og.P2, og.P2_valid)
+    np.testing.assert_array_equal(g.download("top_cells"), og.top_cells)
+    np.testing.assert_array_equal(g.download("leaves"), og.leaves)
+    np.testing.assert_array_equal(g.download("indices"), og.indices)
+    rays = sa.gen_random_rays(98, 20_000, -0.1, 1.1)
+    for k in range(3):
+        if k != axis:
+            rays[[k, 3 + k]] *= np.float32(thin)
+    for shadow in (False, True):
+        if shadow:
+            rays[6] = 1.0
+        pg, tg = g.trace_host(rays, shadow=shadow)
+        po, to = og.trace(rays, shadow=shadow)[:2]
+        np.testing.assert_array_equal(pg, po)
+        np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))

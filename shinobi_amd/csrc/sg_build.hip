@@ -895,6 +895,12 @@ SG_D void box_visit(uint2 box, uint32_t first, uint32_t res, F&& f) {
 // and its accepted / rejected leaf-pair totals in sums[t] / sums[Tp + t].
 SG_HD uint32_t leaf_sums_stride(uint32_t T) { return (T + 15u) & ~15u; }
 
+// empty leaf ranges, by the whole launch
+SG_D void clear_leaves(uint32_t* __restrict__ leaves, uint32_t n) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
+        reinterpret_cast<uint2*>(leaves)[k] = make_uint2(0u, 0u);
+}
+
 // One sorted top pair per lane: the lane with the most leaf cells to visit
 // sets a wave's time, and with four consecutive pairs per lane (one 16-byte
 // load per array) those lanes ran four set-ups and visits in a row --
@@ -907,17 +913,15 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                                        uint32_t* __restrict__ sums, uint32_t* __restrict__ info,
                                                        uint32_t T, uint32_t* __restrict__ dbg_counts,
                                                        uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
-                                                       uint32_t* __restrict__ prej, uint32_t* __restrict__ leaves) {
+                                                       uint32_t* __restrict__ prej, uint32_t* __restrict__ leaves,
+                                                       uint32_t cap_C2) {
     constexpr int kSlots = 4;
     __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots], s_info[kSlots][4];
     // A top cell reserves its leaf cells by the whole resolutions, its tile
     // writes those within the packed bytes: beyond 255 on an axis (flagged by
-    // k_leaf_cells_count) the others are nobody's, so all are cleared here.
-    if (leaves && (h->status & ST_LEAF_RES)) {
-        const uint32_t C2 = h->C2;
-        for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < C2; k += gridDim.x * kBlock)
-            reinterpret_cast<uint2*>(leaves)[k] = make_uint2(0u, 0u);
-    }
+    // k_leaf_cells_count) the others are nobody's, so all are cleared here; so
+    // are those of a build that has failed already.
+    if (leaves && (h->status & ~ST_NEG_EXTENT)) clear_leaves(leaves, cap_C2);
     const uint32_t P1v = h->P1_valid;
     const uint32_t base = blockIdx.x * kBlock;
     if (base >= P1v) return;
@@ -1435,6 +1439,9 @@ __global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8)))
     LeafTilePlan q;
     leaf_tile_plan(a, sums, info, T, blockIdx.x, q);
     if (q.mode != LEAF_SMALL) {
+        // too many leaf pairs: no tile has a plan, and the ranges would be
+        // those of an earlier build
+        if (q.mode == LEAF_NONE && leaves && (h->status & ST_CAP_P2)) clear_leaves(leaves, a.cap_C2);
         // oversize tiles of a grid with the parallel emission are its
         const uint32_t n = q.mode == LEAF_BIG ? max(1u, (q.acc + kLeafSlice - 1u) / kLeafSlice)
                                               : (q.mode == LEAF_OVERSIZE && !large ? 1u : 0u);
@@ -1990,7 +1997,7 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
                            sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr,
-                           large ? nullptr : leaves);
+                           large ? nullptr : leaves, a.cap_C2);
     if (large) {
         const uint32_t* in[2] = {large->pacc, large->prej};
         uint32_t* out[2] = {large->sacc, large->srej};

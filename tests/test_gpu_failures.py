@@ -168,3 +168,19 @@ def test_scratch_is_per_stream(ctx):
     finally:
         for s in streams:
             ctx._l.sg_stream_destroy(ctx.h, s)
+
+
+@pytest.mark.parametrize("pairs", ["leaf", "top"])
+def test_overflowing_rebuild_leaves_no_old_ranges(ctx, pairs):
+    """a rebuild of more leaf pairs than its grid holds, with the top pairs of
+    before (one top cell) or more than it holds as well: the leaf ranges that
+    kernels over the device view read are empty, not the former build's"""
+    n, kw = (600, dict(res_override=(1, 1, 1))) if pairs == "leaf" else (5000, {})
+    soup, g = _grid(ctx, sa.gen_soup(63, n, 0.01), 1, lam=5.0, lambda_leaf=20.0, **kw)
+    assert g.download("leaves").any()
+    print(f"overflow pairs={pairs}: rebuild of a much larger mesh", flush=True)
+    soup.upload_vertices(sa.gen_soup(63, n, 0.6))
+    g.rebuild()
+    info = g.info()
+    assert info.status == CAPACITY and (info.P1 == n) == (pairs == "leaf")
+    assert not g.download("leaves").any()

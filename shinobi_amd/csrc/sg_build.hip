@@ -526,14 +526,25 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_count(GridHeader* h, Buil
     if (threadIdx.x == 0) sums[blockIdx.x] = s;
 }
 
+// empty leaf ranges, by the whole launch
+SG_D void clear_leaves(uint32_t* __restrict__ leaves, uint32_t n) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
+        reinterpret_cast<uint2*>(leaves)[k] = make_uint2(0u, 0u);
+}
+
 __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, BuildArgs a,
                                                              const uint32_t* __restrict__ ranges,
                                                              uint32_t* __restrict__ cells,
                                                              const uint32_t* __restrict__ sums,
                                                          uint32_t* __restrict__ leaves) {
     __shared__ uint32_t s_scan[kBlock / 64];
-    const uint32_t C1 = h->C1;
+    const uint32_t C1 = h->C1, failed = h->status & ~ST_NEG_EXTENT;
     const uint32_t base = blockIdx.x * kBlock;
+    // A top cell reserves its leaf cells by the whole resolutions, its tile
+    // writes those within the packed bytes: beyond 255 on an axis (flagged by
+    // k_leaf_cells_count) the others are nobody's, so all are cleared here; so
+    // are those of a build that has failed already.
+    if (leaves && failed) clear_leaves(leaves, a.cap_C2);
     if (base >= C1) return;
     const uint32_t prefix = block_prefix_of<kBlock / 64>(sums, blockIdx.x, s_scan);
     const uint32_t k = base + threadIdx.x;
@@ -545,7 +556,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
         reinterpret_cast<uint2*>(cells)[k] = make_uint2(prefix + local, bits);
         // an empty top cell's one leaf cell; the others' are written by the
         // tiles that emit their pairs, so nothing else clears them while the
-        // leaf resolutions lie in 1..255 (k_leaf_count clears the rest)
+        // leaf resolutions lie in 1..255 (then all are cleared above)
         if (leaves && !(bits & kNotEmpty) && prefix + local < a.cap_C2)
             reinterpret_cast<uint2*>(leaves)[prefix + local] = make_uint2(0u, 0u);
     }
@@ -895,12 +906,6 @@ SG_D void box_visit(uint2 box, uint32_t first, uint32_t res, F&& f) {
 // and its accepted / rejected leaf-pair totals in sums[t] / sums[Tp + t].
 SG_HD uint32_t leaf_sums_stride(uint32_t T) { return (T + 15u) & ~15u; }
 
-// empty leaf ranges, by the whole launch
-SG_D void clear_leaves(uint32_t* __restrict__ leaves, uint32_t n) {
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
-        reinterpret_cast<uint2*>(leaves)[k] = make_uint2(0u, 0u);
-}
-
 // One sorted top pair per lane: the lane with the most leaf cells to visit
 // sets a wave's time, and with four consecutive pairs per lane (one 16-byte
 // load per array) those lanes ran four set-ups and visits in a row --
@@ -913,15 +918,9 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
                                                        uint32_t* __restrict__ sums, uint32_t* __restrict__ info,
                                                        uint32_t T, uint32_t* __restrict__ dbg_counts,
                                                        uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
-                                                       uint32_t* __restrict__ prej, uint32_t* __restrict__ leaves,
-                                                       uint32_t cap_C2) {
+                                                       uint32_t* __restrict__ prej) {
     constexpr int kSlots = 4;
     __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots], s_info[kSlots][4];
-    // A top cell reserves its leaf cells by the whole resolutions, its tile
-    // writes those within the packed bytes: beyond 255 on an axis (flagged by
-    // k_leaf_cells_count) the others are nobody's, so all are cleared here; so
-    // are those of a build that has failed already.
-    if (leaves && (h->status & ~ST_NEG_EXTENT)) clear_leaves(leaves, cap_C2);
     const uint32_t P1v = h->P1_valid;
     const uint32_t base = blockIdx.x * kBlock;
     if (base >= P1v) return;
@@ -1984,8 +1983,9 @@ void launch_leaf_cells(GridHeader* h, const BuildArgs& a, const uint32_t* ranges
     const uint32_t blocks = (a.cap_C1 + kBlock - 1) / kBlock;
     if (blocks == 0) return;
     hipLaunchKernelGGL(k_leaf_cells_count, dim3(blocks), dim3(kBlock), 0, st, h, a, ranges, sums, dbg);
-    hipLaunchKernelGGL(k_leaf_cells_write, dim3(blocks), dim3(kBlock), 0, st, h, a, ranges, cells, sums,
-                       leaves);
+    // blocks enough to clear the leaf ranges of a flagged grid of few top cells
+    hipLaunchKernelGGL(k_leaf_cells_write, dim3(blocks < 256u ? 256u : blocks), dim3(kBlock), 0, st, h, a, ranges,
+                       cells, sums, leaves);
 }
 
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
@@ -1996,8 +1996,7 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     const uint32_t blocks = (a.cap_P1 + kBlock - 1) / kBlock;
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
-                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr,
-                           large ? nullptr : leaves, a.cap_C2);
+                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr);
     if (large) {
         const uint32_t* in[2] = {large->pacc, large->prej};
         uint32_t* out[2] = {large->sacc, large->srej};

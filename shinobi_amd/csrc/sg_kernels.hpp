@@ -155,11 +155,10 @@ struct LeafLarge {
 // Without `large` the tiles also write the leaf ranges and the leaf keys only
 // with a.keep_debug; with it, every key is written for the global sort and
 // k_ranges.  Who clears `leaves`: with `large`, the build's first launch, all
-// of it.  Without, launch_leaf_cells the one leaf cell of each empty top cell
-// and each tile its span before it writes the ranges there; in a grid flagged
-// ST_LEAF_RES, whose tiles' spans leave gaps, and in a build that failed before
-// the leaf pairs k_leaf_count all of it first, and in one of more leaf pairs
-// than a.cap_P2, whose tiles write nothing, k_leaf_emit.
+// of it.  Without, launch_leaf_cells the one leaf cell of each empty top cell,
+// or all of it in a grid flagged ST_LEAF_RES, whose tiles' spans leave gaps, and
+// in a build that has failed before; then each tile its span before it writes
+// the ranges there, or k_leaf_emit all of it when the leaf pairs overflow.
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
                       const uint32_t* top_vals, const uint32_t* ranges, const uint32_t* cells, uint32_t* keys,
                       uint32_t* vals, uint32_t* tmp_keys, uint32_t* tmp_vals, float* refs, uint32_t* dbg,

@@ -729,7 +729,8 @@ SG_D uint32_t leaf_pair(const TriSoA& t, const LeafParams& L, GridHeader* h, uin
 // cells in a 502,000-triangle cluster: k_leaf_count 5.6 ms, its emission
 // 8.6 ms).  A box of at least kWideBox cells is therefore visited by its
 // block, one (y, z) row of leaf cells per thread (k_leaf_count lists it and
-// k_leaf_scan's one block counts it; the emission kernels emit it in place).
+// k_leaf_scan or k_leaf_wide counts it; k_leaf_emit_big emits it in place, with
+// the parallel emission k_leaf_wide_emit).
 // Along a row the plane distance never changes direction -- each binary32
 // operation between the cell centre and the distance is monotone -- so a
 // row's accepted cells are one interval, found by two binary searches.  The
@@ -1046,25 +1047,30 @@ SG_D void leaf_totals(GridHeader* h, const BuildArgs& a, uint32_t* __restrict__ 
 }
 
 // First the wide boxes k_leaf_count listed are counted into their tiles'
-// totals.  Then the exclusive scan, in place, of the accepted (sums[0..T)) and
-// rejected (sums[Tp..Tp+T)) tile totals, both halves at once (waves 0-7 and
-// 8-15); sums[2Tp], sums[2Tp+1] receive the grand totals and the header the
-// leaf-pair counts (one block of 1024 threads).
+// totals, a box to a block, and the last block that ends does the rest (one
+// block for all took 3.2 us a box: 947 boxes in 200 dense cells 3.02 ms, with
+// kScanBlocks of them 37 us; without wide boxes every block but the first
+// leaves at once).  Then the exclusive scan, in place, of the accepted
+// (sums[0..T)) and rejected (sums[Tp..Tp+T)) tile totals, both halves at once
+// (waves 0-7 and 8-15); sums[2Tp], sums[2Tp+1] receive the grand totals and
+// the header the leaf-pair counts (by one block of 1024 threads).
+constexpr uint32_t kScanBlocks = 128;
 __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, BuildArgs a,
                                                     const uint32_t* __restrict__ top_keys,
                                                     const uint32_t* __restrict__ top_vals,
                                                     const uint32_t* __restrict__ ranges,
-                                                    const uint32_t* __restrict__ cells, uint32_t* __restrict__ sums,
+                                                    const uint32_t* __restrict__ cells, uint32_t* sums,
                                                     uint32_t T) {
     constexpr int kPer = 16;
     __shared__ uint32_t s_w[16];
     __shared__ uint32_t s_tot[2];
     __shared__ float s_tab[3][kAxisMax];
+    __shared__ bool s_last;
     const uint32_t Tp = leaf_sums_stride(T);
     const uint32_t n_wide = min(sums[2 * (size_t)Tp + 2], kWideCap);
     if (n_wide) {
         const LeafParams L = read_leaf_params(h);
-        for (uint32_t k = 0; k < n_wide; ++k) {
+        for (uint32_t k = blockIdx.x; k < n_wide; k += gridDim.x) {
             const uint32_t i = sums[2 * (size_t)Tp + 4 + k], key = top_keys[i];
             LeafSetup st;
             const uint32_t c = leaf_pair(t, L, h, key, top_vals[i], cells, st);
@@ -1072,13 +1078,20 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
             if (threadIdx.x == 0) {
                 const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
                 if (tile < T) {
-                    sums[tile] += acc;
-                    sums[Tp + tile] += c - acc;
+                    atomicAdd(&sums[tile], acc);
+                    atomicAdd(&sums[Tp + tile], c - acc);
                 }
             }
         }
-        __threadfence_block();
+        if (threadIdx.x == 0) {
+            __threadfence();
+            s_last = atomicAdd(&sums[2 * (size_t)Tp + 3], 1u) == gridDim.x - 1u;
+        }
         __syncthreads();
+        if (!s_last) return;
+        __threadfence();   // the other blocks' totals
+    } else if (blockIdx.x) {
+        return;
     }
     const int w = wave_id(), half = w >> 3;
     const uint32_t tt = threadIdx.x & 511u;
@@ -2006,8 +2019,8 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
         hipLaunchKernelGGL(k_leaf_tile_sums, dim3((T + kBlock - 1) / kBlock), dim3(kBlock), 0, st, h, a, top_keys,
                            ranges, large->pacc, large->prej, large->sacc, large->srej, sums, T);
     } else {
-        hipLaunchKernelGGL(k_leaf_scan, dim3(1), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges, cells, sums,
-                           T);
+        hipLaunchKernelGGL(k_leaf_scan, dim3(kScanBlocks), dim3(1024), 0, st, t, h, a, top_keys, top_vals, ranges,
+                           cells, sums, T);
     }
     // with `large`, the global sort and k_ranges need every key; without it
     // the tiles write the leaf ranges and the keys are kept for keep_debug
@@ -2194,9 +2207,9 @@ size_t leaf_tiles(uint32_t n) {
     const size_t t = ((size_t)n + kLeafTile - 1) / kLeafTile;
     return t ? t : 1;
 }
-// accepted and rejected totals, their grand totals, the list of wide boxes, the
-// number of work items of k_leaf_emit_big (all cleared before each build), then
-// the items
+// accepted and rejected totals, their grand totals, the number of wide boxes and
+// of k_leaf_scan's blocks that have ended, the list of wide boxes, the number of
+// work items of k_leaf_emit_big (all cleared before each build), then the items
 size_t leaf_sums_words(uint32_t n) {
     return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap + 1;
 }

@@ -181,6 +181,37 @@ def test_wide_leaf_boxes_bit_exact(ctx, oracle, n_small):
         g.rebuild()
 
 
+def _dense_cells_under_large_triangles(n_cells, n_small, n_large):
+    """n_cells groups of n_small tiny triangles, each within a cell of a 21^3
+    lattice of the unit cube and crossed by n_large tilted triangles"""
+    r = np.random.default_rng(7)
+    m = 21
+    k = r.permutation(m ** 3)[:n_cells]
+    o = (np.stack([k % m, (k // m) % m, k // m // m], 1) + 0.1) / m
+    n = n_cells * n_small
+    small = (np.repeat(o, n_small, 0) + r.random((n, 3)) * 0.8 / m)[None] + (r.random((3, n, 3)) - 0.5) * 0.02 / m
+    q = r.random((3, n_cells * n_large, 3)) * 0.1 + np.array([[0, 0, 0], [.81, .18, .81], [.09, .81, .72]])[:, None]
+    large = np.repeat(o, n_large, 0)[None] + q * 0.8 / m
+    ends = np.array([[[0, 0, 0], [1, 1, 1]], [[.001, 0, 0], [.999, 1, 1]], [[0, .001, 0], [1, .999, 1]]])
+    v = np.concatenate([small, large, ends], 1)
+    return np.ascontiguousarray(v.transpose(0, 2, 1).reshape(9, -1), dtype=np.float32)
+
+
+@pytest.mark.parametrize("n_cells,n_small,n_large", [(60, 2_000, 5), (230, 2_000, 6)])
+def test_many_wide_leaf_boxes_bit_exact(ctx, oracle, n_cells, n_small, n_large):
+    """more wide boxes than blocks count them, and more than are counted by
+    blocks (1,024); the tiles are not oversize, so one launch counts and scans"""
+    a = _dense_cells_under_large_triangles(n_cells, n_small, n_large)
+    kw = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, res_override=(21, 21, 21))
+    og = oracle.build_twolevel(a, **kw)
+    assert og.status == 0 and (og.pair_counts >= 1024).sum() > (1_024 if n_cells > 200 else 128)
+    _, g = _gpu_build(ctx, a, 1, **kw)
+    for _ in range(3):
+        _assert_top_level(g, og)
+        _assert_leaf_level(g, og)
+        g.rebuild()
+
+
 @pytest.mark.parametrize("n_small", [3_000, 30_000])
 def test_rebuild_into_wide_leaf_boxes(ctx, oracle, n_small):
     """the same meshes met first by a rebuild: the grid is built while the

@@ -306,6 +306,7 @@ static size_t grid_layout(sg_grid* g, char* pool) {
         g->passes2 = sort_passes(g->key_bits2, g->rb);
         g->sort2_words = sort_scratch_words(g->cap_P2, g->key_bits2, g->rb);
         g->sort2 = (uint32_t*)take(g->sort2_words * 4);
+        g->box_pool = (uint32_t*)take(leaf_pool_words(g->cap_P2) * 4);
     }
     return align_up(off, 256);
 }
@@ -437,7 +438,7 @@ static void enqueue_build(sg_grid* g, bool fixed_res, hipStream_t st, void* cons
                       st);
     mark(5);
     launch_leaf_emit(t, g->hdr, a, g->k1[f1], g->v1[f1], g->ranges1, g->cells1, g->k2[0], g->v2[0], g->k2[1],
-                     g->v2[1], g->refs, g->dbg_pair, g->sums_leaf, g->leaf_info, g->boxes,
+                     g->v2[1], g->refs, g->dbg_pair, g->sums_leaf, g->leaf_info, g->boxes, g->box_pool,
                      g->large_path ? &g->large : nullptr, g->leaves, st);
     mark(6);
     // Only a grid whose build met leaf tiles too large for the LDS sort has

@@ -595,10 +595,13 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
 constexpr uint32_t kLeafTile = 512;                   // nominal sorted top pairs per leaf tile
 constexpr int kLeafBlock = 512;                       // threads of the leaf emission kernel
 constexpr int kBigBlock = 1024;                       // threads of its form for larger tiles
-// What a tile may hold in LDS: accepted pairs, leaf cells, top pairs.  A tile
-// beyond LeafSmall goes to the larger kernel, one beyond LeafBig is oversize.
+// What a tile may hold: accepted pairs, leaf cells, top pairs.  A tile beyond
+// LeafSmall goes to the larger kernel, one beyond LeafBig is oversize.  The
+// small kernel takes a tile's leaf cells in windows and a window's pairs in
+// chunks of what its LDS holds (see leaf_emit_small).
 struct LeafSmall {
-    static constexpr uint32_t pairs = 4096, span = 4096, tops = 1536;
+    static constexpr uint32_t pairs = 4 * 4096, span = 65536, tops = 1536;
+    static constexpr uint32_t chunk = 4096, window = 8192;
 };
 struct LeafBig {
     static constexpr uint32_t pairs = 65024, span = 16384, tops = 8192;
@@ -749,25 +752,32 @@ SG_D bool plane_tested(const LeafSetup& s) {
 // Monotone needs finite terms: coordinates below 1e18 keep every product of
 // the distance in range (a normal of zeros, infinities or NaN then rejects
 // every cell or, all zero, accepts every cell, in the search as in the walk).
-SG_D bool wide_box(const LeafParams& L, const LeafSetup& s, uint32_t c) {
-    if (c < kWideBox) return false;
+SG_D bool finite_box(const LeafParams& L, const LeafSetup& s) {
     auto ok = [](v3 a) { return fabsf(a.x) < 1e18f && fabsf(a.y) < 1e18f && fabsf(a.z) < 1e18f; };
     return ok(s.v0) && ok(s.v1) && ok(s.v2) && ok(s.org) && ok(s.org + L.cs);
 }
 
-// Every thread of the block calls this with the same pair.  f(live, key0, xa,
-// xb) once per round of rows: cells [xa, xb) of the thread's row are accepted,
-// key0 the key of the row's cell 0 (live false: no row, xa == xb).
-template <class F>
+SG_D bool wide_box(const LeafParams& L, const LeafSetup& s, uint32_t c) { return c >= kWideBox && finite_box(L, s); }
+
+// Every thread of the block, or with WAVE of the wave, calls this with the same
+// pair.  f(r, key0, xa, xb) once per round of rows: cells [xa, xb) of the
+// thread's row r are accepted, key0 the key of the row's cell 0 (xa == xb
+// without a row).
+template <bool WAVE = false, class F>
 SG_D void wide_visit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], F&& f) {
     const int ex = s.hp[0] - s.lo[0], ey = s.hp[1] - s.lo[1], ez = s.hp[2] - s.lo[2];
     const uint32_t crx = f2u(s.cres.x), crxy = f2u(s.cres.x * s.cres.y);
     const bool plane = plane_tested(s);
     const v3 n_ = normalize(cross(s.v1 - s.v0, s.v2 - s.v0));
     const v3 scs = L.cs / s.cres;
-    __syncthreads();   // tab is free again
-    if (threadIdx.x < 3) {
-        const int a = (int)threadIdx.x;
+    const int tid = WAVE ? lane_id() : (int)threadIdx.x, threads = WAVE ? 64 : (int)blockDim.x;
+    auto sync = [&]() {
+        if (WAVE) __threadfence_block();
+        else __syncthreads();
+    };
+    sync();   // tab is free again
+    if (tid < 3) {
+        const int a = tid;
         const v3 c0 = (mk((float)s.lo[0], (float)s.lo[1], (float)s.lo[2]) * scs + s.org) + scl(scs, 0.5f);
         const float step = comp(scs, a);
         float c = comp(c0, a) - step;
@@ -777,11 +787,11 @@ SG_D void wide_visit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxis
             tab[a][i] = c;
         }
     }
-    __syncthreads();
+    sync();
     const float hx = scs.x * 0.5f + kEps, hy = scs.y * 0.5f + kEps, hz = scs.z * 0.5f + kEps;
     const int rows = ey * ez;
-    for (int r0 = 0; r0 < rows; r0 += (int)blockDim.x) {
-        const int r = r0 + (int)threadIdx.x;
+    for (int r0 = 0; r0 < rows; r0 += threads) {
+        const int r = r0 + tid;
         const bool live = r < rows;
         int xa = 0, xb = 0;
         uint32_t key0 = 0;
@@ -818,7 +828,7 @@ SG_D void wide_visit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxis
             xb = min(xb, room);
             xa = min(xa, xb);
         }
-        f(live, key0, xa, xb);
+        f((uint32_t)r, key0, xa, xb);
     }
 }
 
@@ -826,7 +836,7 @@ SG_D void wide_visit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxis
 template <int NW>
 SG_D uint32_t wide_count(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], uint32_t* s_red) {
     uint32_t acc = 0;
-    wide_visit(L, s, tab, [&](bool, uint32_t, int xa, int xb) { acc += (uint32_t)(xb - xa); });
+    wide_visit(L, s, tab, [&](uint32_t, uint32_t, int xa, int xb) { acc += (uint32_t)(xb - xa); });
     return block_sum<NW>(acc, s_red);
 }
 
@@ -836,7 +846,7 @@ template <int NW>
 SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisMax], uint32_t* s_scan, uint32_t tri,
                     uint32_t pa, uint32_t pr, uint32_t rej, uint32_t cap, uint32_t* __restrict__ keys,
                     uint32_t* __restrict__ vals) {
-    wide_visit(L, s, tab, [&](bool, uint32_t key0, int xa, int xb) {
+    wide_visit(L, s, tab, [&](uint32_t, uint32_t key0, int xa, int xb) {
         uint32_t agg;
         uint32_t p = pa + block_excl_scan<NW>((uint32_t)(xb - xa), &agg, s_scan);
         for (int x = xa; x < xb; ++x, ++p)
@@ -857,35 +867,81 @@ SG_D void wide_emit(const LeafParams& L, const LeafSetup& s, float (*tab)[kAxisM
 // the triangle nor forms its box and plane again.  x: the leaf cell of the
 // box's corner within its top cell (16 bits) and the box's extents less one
 // (5 bits each); y: the accepted cells, bit k for the k-th in z/y/x order.
-// Boxes of up to 32 cells with a corner below 2^16 have this form; others
-// are open (kBoxOpen: the emission visits the box again), pairs without leaf
-// cells empty.
-constexpr uint32_t kBoxOpen = 0x80000000u, kBoxEmpty = 0x7FFFFFFFu;
+// Boxes of up to 32 cells with a corner below 2^16 have this form.  Larger
+// ones are stored in the pool of masks: x is kBoxOpen and the place of
+// {corner, extents (8 bits each) and kBoxFull when every cell is accepted,
+// otherwise the masks, 32 cells each}, y the number of accepted cells.  (406,002
+// triangles, three large ones across each of 2,000 top cells: rebuild 568 us with
+// such boxes visited again by the emission, 170 stored.)  Boxes that a block
+// visits together, and those that find no place, are kBoxWide: the emission
+// visits them again.  Pairs without leaf cells: empty.
+constexpr uint32_t kBoxOpen = 0x80000000u, kBoxEmpty = 0x7FFFFFFFu, kBoxWide = 0xFFFFFFFFu;
+constexpr uint32_t kBoxFull = 0x80000000u;
+// The pool is cut in kPools parts, each with its counter in a cache line of its
+// own, used by every kPools-th block: adds of many waves to one counter wait
+// for each other.
+constexpr uint32_t kPools = 16, kPoolStride = 16;
 
-SG_D uint2 pair_box(const LeafSetup& s, uint32_t c, uint32_t mask) {
-    if (c == 0) return make_uint2(kBoxEmpty, 0u);
+struct BoxPool {
+    uint32_t* words;   // kPools parts of `part` words
+    uint32_t part;
+};
+
+// the leaf cell of the box's corner within its top cell
+SG_D uint32_t box_corner(const LeafSetup& s) {
     const uint32_t crx = f2u(s.cres.x), crxy = f2u(s.cres.x * s.cres.y);
-    const uint32_t corner = (uint32_t)s.lo[0] + (uint32_t)s.lo[1] * crx + (uint32_t)s.lo[2] * crxy;
-    if (c > 32u || corner >= 65536u) return make_uint2(kBoxOpen, 0u);
-    return make_uint2(corner | (uint32_t)(s.hp[0] - s.lo[0] - 1) << 16 | (uint32_t)(s.hp[1] - s.lo[1] - 1) << 21 |
-                          (uint32_t)(s.hp[2] - s.lo[2] - 1) << 26,
-                      mask);
+    return (uint32_t)s.lo[0] + (uint32_t)s.lo[1] * crx + (uint32_t)s.lo[2] * crxy;
 }
 
-// cells of the box (0: empty)
+struct BoxExtent {
+    uint32_t corner, ex, ey, ez;
+};
+
+SG_D BoxExtent box_extent(uint2 box, const uint32_t* __restrict__ pool) {
+    BoxExtent e;
+    if (box.x < kBoxOpen) {
+        e.corner = box.x & 0xFFFFu;
+        e.ex = ((box.x >> 16) & 31u) + 1u;
+        e.ey = ((box.x >> 21) & 31u) + 1u;
+        e.ez = ((box.x >> 26) & 31u) + 1u;
+    } else {
+        const uint32_t* q = pool + (box.x & ~kBoxOpen);
+        const uint32_t x = q[1];
+        e.corner = q[0];
+        e.ex = x & 0xFFu;
+        e.ey = (x >> 8) & 0xFFu;
+        e.ez = (x >> 16) & 0xFFu;
+    }
+    return e;
+}
+
+// cells of a box of the first form (0: empty)
 SG_D uint32_t box_cells(uint32_t x) {
     if (x >= kBoxEmpty) return 0u;
     return (((x >> 16) & 31u) + 1u) * (((x >> 21) & 31u) + 1u) * (((x >> 26) & 31u) + 1u);
 }
 
-// f(leaf cell) for every accepted cell of a box that is not open, `first` the
-// tile's index of the top cell's leaf cell 0, res its packed resolution
+// rejected cells of a box (not kBoxWide)
+SG_D uint32_t box_rejects(uint2 box, const uint32_t* __restrict__ pool) {
+    if (box.x == kBoxEmpty) return 0u;
+    const BoxExtent e = box_extent(box, pool);
+    return e.ex * e.ey * e.ez - (box.x < kBoxOpen ? (uint32_t)__popc(box.y) : box.y);
+}
+
+// the leaf cells [lo, hi] between the first and the last cell of a box
+SG_D void box_bounds(const BoxExtent& e, uint32_t first, uint32_t crx, uint32_t cry, uint32_t& lo, uint32_t& hi) {
+    lo = first + e.corner;
+    hi = lo + e.ex - 1u + (e.ey - 1u + (e.ez - 1u) * cry) * crx;
+}
+
+// f(leaf cell) for every accepted cell of a box of the first form, `first` the
+// tile's index of the top cell's leaf cell 0, crx and cry its resolution along
+// x and y
 template <class F>
-SG_D void box_visit(uint2 box, uint32_t first, uint32_t res, F&& f) {
+SG_D void box_visit(uint2 box, uint32_t first, uint32_t crx, uint32_t cry, F&& f) {
     const uint32_t ex = ((box.x >> 16) & 31u) + 1u, ey = ((box.x >> 21) & 31u) + 1u;
-    const uint32_t crx = res & 0xFFu, crxy = crx * ((res >> 8) & 0xFFu);
     uint32_t row = first + (box.x & 0xFFFFu), y = 0, x = 0;
-    const uint32_t next = crxy - (ey - 1u) * crx;   // from a slice's last row to the next slice's first
+    const uint32_t next = (cry - (ey - 1u)) * crx;   // from a slice's last row to the next slice's first
     for (uint32_t m = box.y; m; m >>= 1) {
         if (m & 1u) f(row + x);
         if (++x == ex) {
@@ -897,35 +953,133 @@ SG_D void box_visit(uint2 box, uint32_t first, uint32_t res, F&& f) {
     }
 }
 
+// the same for a stored box: the plane accepts few of its cells, so its mask is
+// read by its set bits (places below 2^10 divided exactly by a multiplication)
+template <class F>
+SG_D void stored_visit(uint2 box, const uint32_t* __restrict__ pool, uint32_t first, uint32_t crx, uint32_t cry,
+                       F&& f) {
+    if (box.y == 0u) return;
+    const BoxExtent e = box_extent(box, pool);
+    const uint32_t* q = pool + (box.x & ~kBoxOpen);
+    const bool full = (q[1] & kBoxFull) != 0u;
+    const uint32_t n = e.ex * e.ey * e.ez, crxy = crx * cry;
+    const float rx = 1.f / (float)e.ex, ry = 1.f / (float)e.ey;
+    for (uint32_t k0 = 0; k0 < n; k0 += 32u) {
+        uint32_t m = full ? 0xFFFFFFFFu : q[2u + (k0 >> 5)];
+        if (n - k0 < 32u) m &= (1u << (n - k0)) - 1u;
+        for (; m; m &= m - 1u) {
+            const uint32_t k = k0 + (uint32_t)__ffs((int)m) - 1u, r = (uint32_t)(((float)k + 0.5f) * rx),
+                           z = (uint32_t)(((float)r + 0.5f) * ry);
+            f(first + e.corner + (k - r * e.ex) + (r - z * e.ey) * crx + z * crxy);
+        }
+    }
+}
+
 // Leaf tile of a sorted top pair: tile t holds the top cells that start in
 // [t*kLeafTile, (t+1)*kLeafTile), so pair i belongs to tile
 // floor(start of its top cell / kLeafTile).  Per tile the count kernel
 // records (zero-initialised words, combined with atomicMax):
 //   info[4t+0] = ~first pair   info[4t+1] = end pair
 //   info[4t+2] = ~first leaf key   info[4t+3] = last leaf key + 1
-//   info[4T+t] = 1 when a pair of the tile has an open box
+//   info[4T+t] = 1 when a pair of the tile has a stored box (kBoxOpen)
+//   info[5T+t] = 1 when one has a kBoxWide box
 // and its accepted / rejected leaf-pair totals in sums[t] / sums[Tp + t].
 SG_HD uint32_t leaf_sums_stride(uint32_t T) { return (T + 15u) & ~15u; }
+
+// The wave's boxes that are stored (need: their words in the pool), with the
+// plane test counted on the way: acc and box of those lanes.  The whole wave
+// calls this.  A box of kCoopBox cells or more is visited by the wave, a row of
+// cells per lane (see wide_visit), its mask put together in LDS: a lane alone
+// walks a cell in some 60 ns, and its wave waits.  (401,002 triangles, 1,000 boxes
+// of some 1,000 cells: k_leaf_count 149 -> 20 us; 603,002 triangles, 3,000 of
+// some 300: 103 -> 55.  From 128 cells on, the ruins rebuild took 295 us for 238,
+// from 512 on the two scenes 2 and 9 % longer.)
+constexpr uint32_t kCoopBox = 256;
+SG_D void store_boxes(const TriSoA& t, const LeafParams& L, GridHeader* h, uint32_t key, uint32_t tri,
+                      const uint32_t* __restrict__ cells, const BoxPool& pool, uint32_t* __restrict__ pool_n,
+                      uint32_t need, float (*tab)[kAxisMax], uint32_t* s_mask, uint32_t& acc, uint2& box) {
+    const uint32_t part = blockIdx.x % kPools, inc = wave_incl_scan(need), l = (uint32_t)lane_id();
+    uint32_t place = 0;
+    if (l == 63u) place = atomicAdd(&pool_n[part * kPoolStride], inc);
+    place = (uint32_t)__shfl((int)place, 63, 64) + inc - need;
+    const bool room = place + need <= pool.part;   // otherwise the box is only counted
+    uint32_t* words = pool.words + (size_t)part * pool.part + place;
+    auto head = [&](const LeafSetup& s, uint32_t* w, bool full) {
+        w[0] = box_corner(s);
+        w[1] = (uint32_t)(s.hp[0] - s.lo[0]) | (uint32_t)(s.hp[1] - s.lo[1]) << 8 |
+               (uint32_t)(s.hp[2] - s.lo[2]) << 16 | (full ? kBoxFull : 0u);
+    };
+    bool mine = need != 0u;
+    for (uint64_t m = __ballot(need >= 2u + kCoopBox / 32u); m; m &= m - 1ull) {
+        const int o = __ffsll((long long)m) - 1;
+        LeafSetup s;
+        const uint32_t c = leaf_pair(t, L, h, (uint32_t)__builtin_amdgcn_readlane((int)key, o),
+                                     (uint32_t)__builtin_amdgcn_readlane((int)tri, o), cells, s);
+        if (!finite_box(L, s)) continue;   // walked below
+        const uint32_t ex = (uint32_t)(s.hp[0] - s.lo[0]);
+        uint32_t n = 0;
+        if (l < kWideBox / 32u) s_mask[l] = 0;
+        wide_visit<true>(L, s, tab, [&](uint32_t r, uint32_t, int xa, int xb) {
+            n += (uint32_t)(xb - xa);
+            for (uint32_t k = r * ex + (uint32_t)xa, e = r * ex + (uint32_t)xb; k < e;) {
+                const uint32_t to = min(e, (k | 31u) + 1u), c2 = to - k;
+                atomicOr(&s_mask[k >> 5], (c2 < 32u ? (1u << c2) - 1u : 0xFFFFFFFFu) << (k & 31u));
+                k = to;
+            }
+        });
+        __threadfence_block();
+        n = wave_sum(n);
+        if (__builtin_amdgcn_readlane((int)room, o)) {
+            const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)place, o);
+            uint32_t* w = pool.words + (size_t)part * pool.part + at;
+            if (l < (c + 31u) / 32u) w[2u + l] = s_mask[l];
+            if (l == 0u) head(s, w, false);
+        }
+        __threadfence_block();   // s_mask is free again
+        if ((int)l == o) {
+            acc = n;
+            mine = false;
+        }
+    }
+    if (mine) {
+        LeafSetup s;
+        leaf_pair(t, L, h, key, tri, cells, s);
+        if (need > 2u) {   // with a plane test
+            uint32_t bit = 0, mask = 0, *w = words + 2;
+            leaf_visit(L, s, [&](uint32_t, bool ok) {
+                acc += ok ? 1u : 0u;
+                mask |= ok ? 1u << (bit & 31u) : 0u;
+                if ((++bit & 31u) == 0u) {
+                    if (room) *w = mask;
+                    ++w;
+                    mask = 0;
+                }
+            });
+            if (room && (bit & 31u)) *w = mask;
+        }
+        if (room) head(s, words, need == 2u);
+    }
+    if (need && room) box = make_uint2(kBoxOpen | (part * pool.part + place), acc);
+}
 
 // One sorted top pair per lane: the lane with the most leaf cells to visit
 // sets a wave's time, and with four consecutive pairs per lane (one 16-byte
 // load per array) those lanes ran four set-ups and visits in a row --
 // height-field rebuild 0.387 -> 0.364 ms, ruins 0.392 -> 0.315 ms with one.
-__global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
-                                                       const uint32_t* __restrict__ top_keys,
-                                                       const uint32_t* __restrict__ top_vals,
-                                                       const uint32_t* __restrict__ ranges,
-                                                       const uint32_t* __restrict__ cells,
-                                                       uint32_t* __restrict__ sums, uint32_t* __restrict__ info,
-                                                       uint32_t T, uint32_t* __restrict__ dbg_counts,
-                                                       uint2* __restrict__ boxes, uint32_t* __restrict__ pacc,
-                                                       uint32_t* __restrict__ prej) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_leaf_count(
+    TriSoA t, GridHeader* h, const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
+    const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ cells, uint32_t* __restrict__ sums,
+    uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ dbg_counts, uint2* __restrict__ boxes,
+    BoxPool pool, uint32_t* __restrict__ pool_n, uint32_t* __restrict__ pacc, uint32_t* __restrict__ prej) {
     constexpr int kSlots = 4;
-    __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots], s_info[kSlots][4];
+    __shared__ uint32_t s_acc[kSlots], s_rej[kSlots], s_open[kSlots][2], s_info[kSlots][4];
+    __shared__ float s_tab[kBlock / 64][3][kAxisMax];
+    __shared__ uint32_t s_mask[kBlock / 64][kWideBox / 32];
     const uint32_t P1v = h->P1_valid;
     const uint32_t base = blockIdx.x * kBlock;
     if (base >= P1v) return;
-    if (threadIdx.x < kSlots) s_acc[threadIdx.x] = s_rej[threadIdx.x] = s_open[threadIdx.x] = 0;
+    if (threadIdx.x < kSlots) s_acc[threadIdx.x] = s_rej[threadIdx.x] = 0;
+    if (threadIdx.x < 2 * kSlots) s_open[threadIdx.x >> 1][threadIdx.x & 1] = 0;
     if (threadIdx.x < 4 * kSlots) s_info[threadIdx.x >> 2][threadIdx.x & 3] = 0;
     const LeafParams L = read_leaf_params(h);
     const uint32_t Tp = leaf_sums_stride(T);
@@ -938,50 +1092,59 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
     const uint32_t tile0 = first_key < L.C1 ? reinterpret_cast<const uint2*>(ranges)[first_key].x / kLeafTile : 0u;
     const uint32_t tile1 = base / kLeafTile;
     __syncthreads();
-    if (i < P1v && key < L.C1) {
-        const uint2 rg = reinterpret_cast<const uint2*>(ranges)[key];
-        const uint32_t tile = rg.x / kLeafTile;
+    const bool live = i < P1v && key < L.C1;
+    const uint2 rg = live ? reinterpret_cast<const uint2*>(ranges)[key] : make_uint2(0u, 0u);
+    uint32_t c = 0, acc = 0, need = 0;
+    uint2 box = make_uint2(kBoxEmpty, 0u);
+    bool counted = true;
+    if (live) {
         LeafSetup st;
-        const uint32_t c = leaf_pair(t, L, h, key, tri, cells, st);
+        c = leaf_pair(t, L, h, key, tri, cells, st);
         if (dbg_counts) dbg_counts[i] = c;
-        uint32_t acc = 0, mask = 0;
-        bool counted = true;
         if (c) {
             // a box of one leaf cell on some axis has no plane test: every
             // cell is accepted unless its key reaches C2, and the largest
             // key is that of the far corner -- then the count is the volume
-            const uint32_t crx = f2u(st.cres.x), crxy = f2u(st.cres.x * st.cres.y);
+            const uint32_t crx = f2u(st.cres.x), crxy = f2u(st.cres.x * st.cres.y), corner = box_corner(st);
             const uint32_t kmax = (uint32_t)(st.hp[0] - 1) + (uint32_t)(st.hp[1] - 1) * crx +
                                   (uint32_t)(st.hp[2] - 1) * crxy + st.px;
-            if (!plane_tested(st) && kmax < L.C2) {
-                acc = c;
-                mask = c >= 32u ? 0xFFFFFFFFu : (1u << c) - 1u;
-                if (pacc && wide_box(L, st, c)) {   // listed for its emission
+            const bool plane = plane_tested(st) || kmax >= L.C2;
+            box.x = corner | (uint32_t)(st.hp[0] - st.lo[0] - 1) << 16 | (uint32_t)(st.hp[1] - st.lo[1] - 1) << 21 |
+                    (uint32_t)(st.hp[2] - st.lo[2] - 1) << 26;
+            if (c > 32u || corner >= 65536u) {
+                box.x = kBoxWide;
+                if (c < kWideBox) {
+                    // (a top cell of more than 2^16 leaf cells makes its tile oversize)
+                    if (corner < 65536u) need = 2u + (plane ? (c + 31u) / 32u : 0u);
+                } else if (finite_box(L, st) && (pacc || plane)) {
+                    // listed: counted by blocks, and for its emission
                     const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
                     if (w < kWideCap) sums[2 * (size_t)Tp + 4 + w] = i;
-                }
-            } else {
-                if (wide_box(L, st, c)) {   // k_leaf_scan counts it
-                    const uint32_t w = atomicAdd(&sums[2 * (size_t)Tp + 2], 1u);
-                    counted = w >= kWideCap;
-                    if (!counted) sums[2 * (size_t)Tp + 4 + w] = i;
-                }
-                if (counted) {
-                    uint32_t bit = 0;
-                    leaf_visit(L, st, [&](uint32_t, bool ok) {
-                        acc += ok ? 1u : 0u;
-                        mask |= ok && bit < 32u ? 1u << bit : 0u;
-                        ++bit;
-                    });
+                    counted = !plane || w >= kWideCap;
                 }
             }
+            if (!plane) {
+                acc = c;
+                box.y = c >= 32u ? 0xFFFFFFFFu : (1u << c) - 1u;
+            } else if (counted && !need) {
+                uint32_t bit = 0;
+                leaf_visit(L, st, [&](uint32_t, bool ok) {
+                    acc += ok ? 1u : 0u;
+                    box.y |= ok && bit < 32u ? 1u << bit : 0u;
+                    ++bit;
+                });
+            }
         }
-        const uint2 box = pair_box(st, c, mask);
+    }
+    if (__builtin_expect(__ballot(need != 0u) != 0ull, 0))
+        store_boxes(t, L, h, key, tri, cells, pool, pool_n, need, s_tab[wave_id()], s_mask[wave_id()], acc, box);
+    if (live) {
+        const uint32_t tile = rg.x / kLeafTile;
         boxes[i] = box;
-        if (box.x == kBoxOpen && tile < T) {
-            const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u;
-            if (slot < kSlots) s_open[slot] = 1u;
-            else info[4 * (size_t)T + tile] = 1u;
+        if (box.x >= kBoxOpen && tile < T) {
+            const uint32_t slot = tile == tile0 ? 0u : tile - tile1 + 1u, wide = box.x == kBoxWide ? 1u : 0u;
+            if (slot < kSlots) s_open[slot][wide] = 1u;
+            else info[(4 + wide) * (size_t)T + tile] = 1u;
         }
         if (counted && pacc) {   // per-pair totals for the parallel emission of oversize tiles
             pacc[i] = acc;
@@ -1021,7 +1184,9 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
         if (tile < T && (slot == 0 || tile != tile0)) {
             if (s_acc[slot]) atomicAdd(&sums[tile], s_acc[slot]);
             if (s_rej[slot]) atomicAdd(&sums[Tp + tile], s_rej[slot]);
-            if (s_open[slot]) info[4 * (size_t)T + tile] = 1u;
+            // (plain stores: the blocks of a dense top cell do not wait for each other)
+            for (uint32_t w = 0; w < 2u; ++w)
+                if (s_open[slot][w]) info[(4 + w) * (size_t)T + tile] = 1u;
             if (s_info[slot][0])
                 for (int k = 0; k < 4; ++k) atomicMax(&info[4 * (size_t)tile + k], s_info[slot][k]);
         }
@@ -1029,12 +1194,14 @@ __global__ __launch_bounds__(kBlock) void k_leaf_count(TriSoA t, GridHeader* h,
 }
 
 // the grand totals (accepted ta, rejected tr) and the header's leaf-pair counts
-SG_D void leaf_totals(GridHeader* h, const BuildArgs& a, uint32_t* __restrict__ sums, uint32_t T, uint32_t ta,
-                      uint32_t tr) {
+SG_D void leaf_totals(GridHeader* h, uint32_t status, const BuildArgs& a, uint32_t* __restrict__ sums, uint32_t T,
+                      uint32_t ta, uint32_t tr) {
     const uint32_t Tp = leaf_sums_stride(T);
     const uint64_t total = (uint64_t)ta + tr;
-    sums[2 * (size_t)Tp] = ta;
-    sums[2 * (size_t)Tp + 1] = tr;
+    // top pairs that were cut off leave keys of no build: no tile gets a plan
+    const bool cut = (status & ST_CAP_P1) != 0u;
+    sums[2 * (size_t)Tp] = cut ? 0xFFFFFFFFu : ta;
+    sums[2 * (size_t)Tp + 1] = cut ? 0xFFFFFFFFu : tr;
     h->need_P2 = (uint32_t)min(total, (uint64_t)0xFFFFFFFFu);
     if (total > a.cap_P2) {
         atomicOr(&h->status, ST_CAP_P2);
@@ -1063,11 +1230,11 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
                                                     uint32_t T) {
     constexpr int kPer = 16;
     __shared__ uint32_t s_w[16];
-    __shared__ uint32_t s_tot[2];
+    __shared__ uint32_t s_tot[2], s_tiles;
     __shared__ float s_tab[3][kAxisMax];
     __shared__ bool s_last;
     const uint32_t Tp = leaf_sums_stride(T);
-    const uint32_t n_wide = min(sums[2 * (size_t)Tp + 2], kWideCap);
+    const uint32_t status = h->status, n_wide = min(sums[2 * (size_t)Tp + 2], kWideCap);
     if (n_wide) {
         const LeafParams L = read_leaf_params(h);
         for (uint32_t k = blockIdx.x; k < n_wide; k += gridDim.x) {
@@ -1096,7 +1263,8 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
     const int w = wave_id(), half = w >> 3;
     const uint32_t tt = threadIdx.x & 511u;
     uint32_t* row = sums + (size_t)half * Tp;
-    uint32_t run = 0;
+    uint32_t run = 0, tiles = 0;   // tiles: those with pairs
+    if (threadIdx.x == 0) s_tiles = 0;
     for (uint32_t c0 = 0; c0 < T; c0 += 512u * kPer) {
         const uint32_t i0 = c0 + tt * kPer;
         uint32_t v[kPer], sum = 0;
@@ -1114,6 +1282,7 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
         for (int k = 0; k < kPer; ++k) {
             if (i0 + k >= T) v[k] = 0;
             sum += v[k];
+            tiles += v[k] ? 1u : 0u;
         }
         const uint32_t inc = wave_incl_scan(sum);
         if (lane_id() == 63) s_w[w] = inc;
@@ -1141,8 +1310,13 @@ __global__ __launch_bounds__(1024) void k_leaf_scan(TriSoA t, GridHeader* h, Bui
         run += tot;
     }
     if (tt == 0) s_tot[half] = run;
+    tiles = wave_sum(tiles);
+    if (half == 0 && lane_id() == 0) atomicAdd(&s_tiles, tiles);
     __syncthreads();
-    if (threadIdx.x == 0) leaf_totals(h, a, sums, T, s_tot[0], s_tot[1]);
+    if (threadIdx.x == 0) {
+        leaf_totals(h, status, a, sums, T, s_tot[0], s_tot[1]);
+        sums[2 * (size_t)Tp + 3] = s_tiles;
+    }
 }
 
 // With per-pair totals (LeafLarge), in place of k_leaf_scan: the tile totals
@@ -1185,7 +1359,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_tile_sums(GridHeader* h, BuildA
                                                            uint32_t* __restrict__ sums, uint32_t T) {
     const uint32_t P1v = min(h->P1_valid, a.cap_P1), C1 = h->C1, tile = blockIdx.x * kBlock + threadIdx.x;
     const uint32_t ta = P1v ? sacc[P1v - 1u] + pacc[P1v - 1u] : 0u, tr = P1v ? srej[P1v - 1u] + prej[P1v - 1u] : 0u;
-    if (tile == 0) leaf_totals(h, a, sums, T, ta, tr);
+    if (tile == 0) leaf_totals(h, h->status, a, sums, T, ta, tr);
     if (tile >= T) return;
     uint32_t i = tile * kLeafTile;
     if (i < P1v) {
@@ -1205,10 +1379,11 @@ enum LeafMode : uint32_t { LEAF_NONE, LEAF_SMALL, LEAF_BIG, LEAF_OVERSIZE };
 struct LeafTilePlan {
     uint32_t a0, a1, pre_acc, pre_rej, acc, rej, tot_acc, kbase, span;
     LeafMode mode;
+    bool simple;   // LEAF_SMALL: one window, one chunk, no stored boxes
 };
 
-SG_D void leaf_tile_plan(const BuildArgs& a, const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info,
-                         uint32_t T, uint32_t b, LeafTilePlan& q) {
+SG_D void leaf_tile_plan(const BuildArgs& a, bool large, const uint32_t* __restrict__ sums,
+                         const uint32_t* __restrict__ info, uint32_t T, uint32_t b, LeafTilePlan& q) {
     const uint32_t Tp = leaf_sums_stride(T);
     const uint32_t tot_acc = sums[2 * (size_t)Tp], tot_rej = sums[2 * (size_t)Tp + 1];
     q.mode = LEAF_NONE;
@@ -1226,13 +1401,22 @@ SG_D void leaf_tile_plan(const BuildArgs& a, const uint32_t* __restrict__ sums, 
     q.kbase = ~inf.z;
     q.span = inf.w >= q.kbase ? inf.w - q.kbase : 0xFFFFFFFFu;
     const uint32_t tops = q.a1 - q.a0;
-    if (q.acc <= LeafSmall::pairs && q.span <= LeafSmall::span && tops <= LeafSmall::tops &&
-        info[4 * (size_t)T + b] == 0u)
-        q.mode = LEAF_SMALL;
-    else if (q.acc <= LeafBig::pairs && q.span <= LeafBig::span && tops <= LeafBig::tops)
-        q.mode = LEAF_BIG;
-    else
-        q.mode = LEAF_OVERSIZE;
+    const bool stored = info[4 * (size_t)T + b] != 0u, wide = info[5 * (size_t)T + b] != 0u;
+    const bool one = q.span <= LeafSmall::window && q.acc <= LeafSmall::chunk;
+    q.simple = !stored && !wide && one;
+    // a heavy tile among light ones is better cut in slices than left to a block
+    // (sphere 160 against 141 us, ruins 275 against 236); where most are heavy, as
+    // many blocks as tiles use the chip already (518,162-triangle height field, top
+    // cells of 345 triangles: 208 against 287)
+    auto heavy = [&]() {
+        return q.acc > LeafSmall::chunk && 2ull * q.acc * sums[2 * (size_t)Tp + 3] > 3ull * tot_acc;
+    };
+    const bool small = (one || (!large && q.acc <= LeafSmall::pairs && q.span <= LeafSmall::span)) &&
+                       tops <= LeafSmall::tops && !wide,
+               big = !large && q.acc <= LeafBig::pairs && q.span <= LeafBig::span && tops <= LeafBig::tops;
+    if (small && !(big && heavy())) q.mode = LEAF_SMALL;
+    else if (big) q.mode = LEAF_BIG;
+    else q.mode = LEAF_OVERSIZE;
 }
 
 // 16-bit counters in LDS, two to a word: add one, return the old value
@@ -1241,7 +1425,8 @@ SG_D uint32_t count_add(uint16_t* s_cnt, uint32_t k) {
     return (atomicAdd(reinterpret_cast<uint32_t*>(s_cnt) + (k >> 1), 1u << sh) >> sh) & 0xFFFFu;
 }
 
-// Exclusive scan of s_cnt[0..span) in place by a block of NW waves, and the
+// Exclusive scan of s_cnt[0..span) in place by a block of NW waves, its total,
+// and the
 // ranges of the tile's leaf cells, which no other tile holds: {first, last+1}
 // of its references, {0, 0} without (the leaf cells of empty top cells between
 // the tile's are zero as well); n_ranges of them lie below C2.  W words, 2 W
@@ -1249,7 +1434,7 @@ SG_D uint32_t count_add(uint16_t* s_cnt, uint32_t k) {
 // ranges' stores are then contiguous; four cost the height field 1 %), four for
 // larger tiles, whose rounds of two barriers took a tenth of their time.
 template <int NW, int W>
-SG_D void leaf_scan_counts(uint16_t* s_cnt, uint32_t span, uint32_t first, uint32_t* s_scan,
+SG_D uint32_t leaf_scan_counts(uint16_t* s_cnt, uint32_t span, uint32_t first, uint32_t* s_scan,
                            uint2* __restrict__ ranges, uint32_t n_ranges) {
     uint32_t* words = reinterpret_cast<uint32_t*>(s_cnt);
     uint32_t run = 0;
@@ -1275,6 +1460,7 @@ SG_D void leaf_scan_counts(uint16_t* s_cnt, uint32_t span, uint32_t first, uint3
         run += agg;
     }
     __syncthreads();
+    return run;
 }
 
 // The lists of the tile's leaf cells, s_ord[end of cell k-1 .. end of cell k)
@@ -1359,80 +1545,159 @@ SG_D void leaf_reject(uint32_t r, uint32_t n, uint32_t tri, uint32_t cap, uint32
 // sort of staged pairs with the boxes formed again from the gathered
 // triangles, took 174 us.  Two pairs per lane in the write-out, so that their
 // gathers overlap, changed nothing.
-SG_D void leaf_emit_small(const LeafTilePlan& q, const uint2* __restrict__ boxes, const TriSoA& t, uint32_t n_tris,
-                          uint32_t C1, uint32_t C2, uint32_t cap, const uint32_t* __restrict__ top_keys,
-                          const uint32_t* __restrict__ top_vals, const uint32_t* __restrict__ cells,
-                          uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
-                          uint32_t* __restrict__ leaves, int write_keys, uint16_t* s_cnt, uint32_t* s_ord,
-                          uint32_t* s_tri, uint32_t* s_bm, uint32_t* s_scan) {
+// A tile of more leaf cells than the LDS counts hold is sorted in windows of
+// them, one of more pairs than the LDS lists hold in chunks of its counted
+// cells (a cell's list is no longer than the tile's top pairs, so every chunk
+// holds a cell); most tiles are one chunk of one window, without stored boxes
+// (SIMPLE), whose boxes stay in registers.  (Left to k_leaf_emit_big, which counts
+// a tile once per slice and has one block to a CU: 200,000 triangles of 5.8 M
+// references, 4,900 to a tile, rebuild 1,805 us, as chunks 366; the same number
+// with 32 leaf cells to a triangle 287 and, as windows, 135; a window of 4096
+// cells instead of 8192 was up to 20 % slower there and 1 % faster on the height
+// field.)
+template <bool SIMPLE>
+SG_D void leaf_emit_small(const LeafTilePlan& q, const uint2* __restrict__ boxes, const uint32_t* __restrict__ pool,
+                          const TriSoA& t, uint32_t n_tris, uint32_t C1, uint32_t C2, uint32_t cap,
+                          const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
+                          const uint32_t* __restrict__ cells, uint32_t* __restrict__ keys,
+                          uint32_t* __restrict__ vals, float* __restrict__ refs, uint32_t* __restrict__ leaves,
+                          int write_keys, uint16_t* s_cnt, uint32_t* s_ord, uint32_t* s_tri, uint32_t* s_bm,
+                          uint32_t* s_scan, uint32_t* s_k1) {
     constexpr int NW = kLeafBlock / 64;
     constexpr int R = LeafSmall::tops / kLeafBlock;   // rounds; a tile rarely needs more than two
-    for (uint32_t k = threadIdx.x; 2u * k < q.span; k += kLeafBlock) reinterpret_cast<uint32_t*>(s_cnt)[k] = 0;
+    static_assert(LeafSmall::tops <= LeafSmall::chunk && LeafSmall::window <= 1u << (32 - kTopBits),
+                  "a chunk holds a list, an entry a leaf cell of the window");
     const uint32_t tops = q.a1 - q.a0;
+    uint32_t wn = min(q.span, LeafSmall::window);   // leaf cells of the window, from w0 on
+    for (uint32_t k = threadIdx.x; 2u * k < wn; k += kLeafBlock) reinterpret_cast<uint32_t*>(s_cnt)[k] = 0;
     uint2 box[R];
-    uint32_t first[R], res[R];
+    uint32_t at[R];   // the top cell's first leaf cell in the tile (16 bits), its resolution along x and y
+    auto load = [&](uint32_t i, uint2& bx, uint32_t& a) {
+        bx = make_uint2(kBoxEmpty, 0u);
+        a = 0;
+        if (i >= q.a1) return;
+        const uint32_t key = top_keys[i];
+        const uint2 y = boxes[i];
+        if (key < C1) {
+            const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
+            bx = y;
+            a = (cl.x - q.kbase) | cl.y << 16;
+        }
+    };
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const uint32_t i = q.a0 + (uint32_t)j * kLeafBlock + threadIdx.x;
-        box[j] = make_uint2(kBoxEmpty, 0u);
-        first[j] = res[j] = 0;
-        if (i < q.a1) {
-            const uint32_t key = top_keys[i];
-            const uint2 bx = boxes[i];
-            s_tri[i - q.a0] = top_vals[i];
-            if (key < C1) {
-                const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
-                box[j] = bx;
-                first[j] = cl.x - q.kbase;
-                res[j] = cl.y;
+        if (i < q.a1) s_tri[i - q.a0] = top_vals[i];
+        if (SIMPLE) load(i, box[j], at[j]);
+    }
+    __syncthreads();
+    // f(top pair, window's leaf cell) for the accepted cells of the window's
+    // [k0, k1).  A simple tile's boxes stay in registers; the others' are read
+    // again in each round, which needs no registers beyond the simple form's.
+    auto over_tops = [&](uint32_t w0, uint32_t k0, uint32_t k1, auto&& f) {
+        if (SIMPLE) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                if ((uint32_t)j * kLeafBlock >= tops) break;
+                box_visit(box[j], at[j] & 0xFFFFu, (at[j] >> 16) & 0xFFu, at[j] >> 24, [&](uint32_t k) {
+                    if (k < k1) f((uint32_t)j * kLeafBlock + threadIdx.x, k);
+                });
+            }
+            return;
+        }
+#pragma unroll 1
+        for (uint32_t top = threadIdx.x; top < tops; top += kLeafBlock) {
+            uint2 bx;
+            uint32_t a, lo, hi;
+            load(q.a0 + top, bx, a);
+            if (bx.x == kBoxEmpty) continue;
+            const uint32_t first = a & 0xFFFFu, crx = (a >> 16) & 0xFFu, cry = a >> 24;
+            box_bounds(box_extent(bx, pool), first, crx, cry, lo, hi);
+            if (hi < w0 + k0 || lo >= w0 + k1) continue;   // a box beside the cells has nothing there
+            auto cell = [&](uint32_t k) {
+                k -= w0;
+                if (k - k0 < k1 - k0) f(top, k);
+            };
+            if (bx.x < kBoxOpen) box_visit(bx, first, crx, cry, cell);
+            else stored_visit(bx, pool, first, crx, cry, cell);
+        }
+    };
+    uint32_t done = q.pre_acc;   // the slot of the window's first pair
+    for (uint32_t w0 = 0;;) {
+        over_tops(w0, 0u, wn, [&](uint32_t, uint32_t k) { count_add(s_cnt, k); });
+        if (w0 == 0u && q.rej) {
+            uint32_t run = q.tot_acc + q.pre_rej;
+            auto round = [&](uint32_t top, uint32_t n) {
+                uint32_t agg;
+                const uint32_t r = run + block_excl_scan<NW>(n, &agg, s_scan);
+                if (n) leaf_reject(r, n, s_tri[top], cap, C2, keys, vals, write_keys);
+                run += agg;
+            };
+            if (SIMPLE) {
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    if ((uint32_t)j * kLeafBlock >= tops) break;
+                    round((uint32_t)j * kLeafBlock + threadIdx.x,
+                          box_cells(box[j].x) - (uint32_t)__popc(box[j].y));
+                }
+            } else {
+#pragma unroll 1
+                for (uint32_t top = threadIdx.x; top - threadIdx.x < tops; top += kLeafBlock) {
+                    uint2 bx;
+                    uint32_t a;
+                    load(q.a0 + top, bx, a);
+                    round(top, box_rejects(bx, pool));
+                }
             }
         }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if ((uint32_t)j * kLeafBlock >= tops) break;
-        box_visit(box[j], first[j], res[j], [&](uint32_t k) {
-            if (k < q.span) count_add(s_cnt, k);
-        });
-    }
-    if (q.rej) {
-        uint32_t run = q.tot_acc + q.pre_rej;
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if ((uint32_t)j * kLeafBlock >= tops) break;
-            const uint32_t n = box_cells(box[j].x) - (uint32_t)__popc(box[j].y);
-            uint32_t agg;
-            const uint32_t r = run + block_excl_scan<NW>(n, &agg, s_scan);
-            if (n) leaf_reject(r, n, s_tri[(uint32_t)j * kLeafBlock + threadIdx.x], cap, C2, keys, vals, write_keys);
-            run += agg;
-        }
-    }
-    __syncthreads();
-    leaf_scan_counts<NW, 1>(s_cnt, q.span, q.pre_acc, s_scan, reinterpret_cast<uint2*>(leaves) + q.kbase,
-                         leaves && C2 > q.kbase ? C2 - q.kbase : 0u);
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if ((uint32_t)j * kLeafBlock >= tops) break;
-        box_visit(box[j], first[j], res[j], [&](uint32_t k) {
-            if (k < q.span) {
-                const uint32_t p = count_add(s_cnt, k);
-                if (p < LeafSmall::pairs) s_ord[p] = k << kTopBits | ((uint32_t)j * kLeafBlock + threadIdx.x);
+        __syncthreads();
+        const uint32_t acc = leaf_scan_counts<NW, SIMPLE ? 1 : 4>(s_cnt, wn, done, s_scan,
+                                                     reinterpret_cast<uint2*>(leaves) + q.kbase + w0,
+                                                     leaves && C2 > q.kbase + w0 ? C2 - q.kbase - w0 : 0u);
+        // chunk: the leaf cells [k0, k1), their pairs from `base` on
+        for (uint32_t k0 = 0, base = 0; base < acc;) {
+            uint32_t k1 = wn, end = acc;
+            if (!SIMPLE && acc - base > LeafSmall::chunk) {   // up to the first list that ends beyond the chunk
+                for (uint32_t k = k0 + threadIdx.x; k < wn; k += kLeafBlock) {
+                    const uint32_t en = k + 1u < wn ? s_cnt[k + 1u] : acc;
+                    if (s_cnt[k] - base <= LeafSmall::chunk && en - base > LeafSmall::chunk) *s_k1 = k;
+                }
+                __syncthreads();
+                k1 = *s_k1;
+                end = s_cnt[k1];
+                __syncthreads();
             }
-        });
-    }
-    __syncthreads();
-    leaf_sort_long<NW>(s_ord, s_cnt, 0, q.span, 0, s_bm + LeafSmall::tops / 32 * wave_id(), LeafSmall::tops / 32);
-    // [0, acc) of s_ord is filled: every accepted cell was counted and listed
-    for (uint32_t j = threadIdx.x; j < q.acc; j += kLeafBlock) {
-        const uint32_t x = s_ord[j];
-        if ((x >> kTopBits) >= q.span) continue;
-        const uint32_t idx = q.pre_acc + leaf_place<4>(s_ord, s_cnt, x, j, 0, 0);
-        const uint32_t tri = s_tri[min(x & ((1u << kTopBits) - 1u), tops - 1u)];
-        if (idx >= cap) continue;
-        if (write_keys) keys[idx] = q.kbase + (x >> kTopBits);
-        vals[idx] = tri;
-        write_ref_record(refs, idx, t.rec, tri, n_tris);
+            over_tops(w0, k0, k1, [&](uint32_t top, uint32_t k) {
+                const uint32_t p = count_add(s_cnt, k) - base;
+                if (p < LeafSmall::chunk) s_ord[p] = k << kTopBits | top;
+            });
+            __syncthreads();
+            leaf_sort_long<NW>(s_ord, s_cnt, k0, k1, base, s_bm + LeafSmall::tops / 32 * wave_id(),
+                               LeafSmall::tops / 32);
+            // [0, end - base) of s_ord is filled: every accepted cell was counted and listed
+            for (uint32_t j = threadIdx.x; j < end - base; j += kLeafBlock) {
+                const uint32_t x = s_ord[j];
+                if ((x >> kTopBits) >= wn) continue;
+                const uint32_t idx = done + base + leaf_place<4>(s_ord, s_cnt, x, j, k0, base);
+                const uint32_t tri = s_tri[min(x & ((1u << kTopBits) - 1u), tops - 1u)];
+                if (idx >= cap) continue;
+                if (write_keys) keys[idx] = q.kbase + w0 + (x >> kTopBits);
+                vals[idx] = tri;
+                write_ref_record(refs, idx, t.rec, tri, n_tris);
+            }
+            if (SIMPLE) return;
+            k0 = k1;
+            base = end;
+            if (base < acc) __syncthreads();   // s_ord is free again
+        }
+        if (SIMPLE) return;
+        done += acc;
+        w0 += LeafSmall::window;
+        if (w0 >= q.span) break;
+        __syncthreads();   // the lists are read
+        wn = min(q.span - w0, LeafSmall::window);
+        for (uint32_t k = threadIdx.x; 2u * k < wn; k += kLeafBlock) reinterpret_cast<uint32_t*>(s_cnt)[k] = 0;
+        __syncthreads();
     }
 }
 
@@ -1440,16 +1705,17 @@ SG_D void leaf_emit_small(const LeafTilePlan& q, const uint2* __restrict__ boxes
 // *todo its number
 __global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_leaf_emit(
     TriSoA t, GridHeader* h, BuildArgs a, const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
-    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, uint32_t* __restrict__ keys,
-    uint32_t* __restrict__ vals, float* __restrict__ refs, const uint32_t* __restrict__ sums,
-    const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves, int write_keys, int large,
+    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, const uint32_t* __restrict__ pool,
+    uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
+    const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves,
+    int write_keys, int large,
     uint32_t* __restrict__ todo, uint32_t* __restrict__ items) {
     constexpr int NW = kLeafBlock / 64;
-    __shared__ uint32_t s_scan[NW], s_ord[LeafSmall::pairs], s_tri[LeafSmall::tops];
+    __shared__ uint32_t s_scan[NW], s_ord[LeafSmall::chunk], s_tri[LeafSmall::tops], s_k1;
     __shared__ uint32_t s_bm[LeafSmall::tops / 32 * NW];
-    __shared__ __align__(4) uint16_t s_cnt[LeafSmall::span];
+    __shared__ __align__(4) uint16_t s_cnt[LeafSmall::window];
     LeafTilePlan q;
-    leaf_tile_plan(a, sums, info, T, blockIdx.x, q);
+    leaf_tile_plan(a, large != 0, sums, info, T, blockIdx.x, q);
     if (q.mode != LEAF_SMALL) {
         // too many leaf pairs: no tile has a plan, and the ranges would be
         // those of an earlier build
@@ -1463,8 +1729,12 @@ __global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8)))
         }
         return;
     }
-    leaf_emit_small(q, boxes, t, h->n_tris, h->C1, h->C2, a.cap_P2, top_keys, top_vals, cells, keys, vals, refs, leaves,
-                    write_keys, s_cnt, s_ord, s_tri, s_bm, s_scan);
+    if (q.simple)
+        leaf_emit_small<true>(q, boxes, pool, t, h->n_tris, h->C1, h->C2, a.cap_P2, top_keys, top_vals, cells, keys,
+                              vals, refs, leaves, write_keys, s_cnt, s_ord, s_tri, s_bm, s_scan, &s_k1);
+    else
+        leaf_emit_small<false>(q, boxes, pool, t, h->n_tris, h->C1, h->C2, a.cap_P2, top_keys, top_vals, cells, keys,
+                               vals, refs, leaves, write_keys, s_cnt, s_ord, s_tri, s_bm, s_scan, &s_k1);
 }
 
 // One stable LSD pass by a block of kBigBlock threads over n (key, value)
@@ -1552,8 +1822,9 @@ struct BigLds {
 // LDS and fewer scan rounds 81 us (38,665-triangle ruins: rebuild 292 -> 274
 // us), in slices of 1024 pairs 60 us.  The global
 // sort and range passes that such tiles needed before took 130 us.
-SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams& L, GridHeader* h, const uint2* __restrict__ boxes,
-                        const TriSoA& t, uint32_t cap, const uint32_t* __restrict__ top_keys,
+SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams& L, GridHeader* h,
+                        const uint2* __restrict__ boxes, const uint32_t* __restrict__ pool, const TriSoA& t,
+                        uint32_t cap, const uint32_t* __restrict__ top_keys,
                         const uint32_t* __restrict__ top_vals, const uint32_t* __restrict__ cells,
                         uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
                         uint32_t* __restrict__ leaves, int write_keys, BigLds& s) {
@@ -1585,7 +1856,7 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
                 const uint32_t key = top_keys[i];
                 tri = top_vals[i];
                 const uint2 box = key < L.C1 ? boxes[i] : make_uint2(kBoxEmpty, 0u);
-                if (box.x == kBoxOpen) {
+                if (box.x == kBoxWide) {
                     LeafSetup st;
                     const uint32_t c = leaf_pair(t, L, h, key, tri, cells, st);
                     if (wide_box(L, st, c)) {
@@ -1599,12 +1870,14 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
                 } else if (box.x != kBoxEmpty) {
                     const uint2 cl = reinterpret_cast<const uint2*>(cells)[key];
                     // a box beside the slice has nothing to list
-                    const uint32_t crx = cl.y & 0xFFu, lo = cl.x - q.kbase + (box.x & 0xFFFFu),
-                                   hi = lo + ((box.x >> 16) & 31u) +
-                                        (((box.x >> 21) & 31u) + ((box.x >> 26) & 31u) * ((cl.y >> 8) & 0xFFu)) * crx;
-                    if (!LIST || (hi >= k0 && lo < k1))
-                        box_visit(box, cl.x - q.kbase, cl.y, [&](uint32_t k) { add(k, i); });
-                    rej = box_cells(box.x) - (uint32_t)__popc(box.y);
+                    const uint32_t first = cl.x - q.kbase, crx = cl.y & 0xFFu, cry = (cl.y >> 8) & 0xFFu;
+                    uint32_t lo, hi;
+                    box_bounds(box_extent(box, pool), first, crx, cry, lo, hi);
+                    if (!LIST || (hi >= k0 && lo < k1)) {
+                        if (box.x < kBoxOpen) box_visit(box, first, crx, cry, [&](uint32_t k) { add(k, i); });
+                        else stored_visit(box, pool, first, crx, cry, [&](uint32_t k) { add(k, i); });
+                    }
+                    if (!LIST) rej = box_rejects(box, pool);
                 }
             }
             __syncthreads();
@@ -1614,7 +1887,7 @@ SG_D void leaf_emit_big(const LeafTilePlan& q, uint32_t slice, const LeafParams&
                 LeafSetup st;
                 const uint32_t c = leaf_pair(t, L, h, top_keys[p], top_vals[p], cells, st);
                 uint32_t acc = 0;
-                wide_visit(L, st, s.tab, [&](bool, uint32_t key0, int xa, int xb) {
+                wide_visit(L, st, s.tab, [&](uint32_t, uint32_t key0, int xa, int xb) {
                     for (int x = xa; x < xb; ++x) add(key0 + (uint32_t)x - q.kbase, p);
                     acc += (uint32_t)(xb - xa);
                 });
@@ -1787,10 +2060,10 @@ SG_D void leaf_emit_oversize(const LeafTilePlan& q, const LeafParams& L, GridHea
 constexpr uint32_t kBigBlocks = 256;
 __global__ __launch_bounds__(kBigBlock) void k_leaf_emit_big(
     TriSoA t, GridHeader* h, BuildArgs a, const uint32_t* __restrict__ top_keys, const uint32_t* __restrict__ top_vals,
-    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, uint32_t* __restrict__ keys,
-    uint32_t* __restrict__ vals, float* __restrict__ refs, const uint32_t* __restrict__ sums,
-    const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves, int write_keys,
-    const uint32_t* __restrict__ todo, const uint32_t* __restrict__ items, uint32_t* __restrict__ tk,
+    const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, const uint32_t* __restrict__ pool,
+    uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
+    const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves,
+    int write_keys, const uint32_t* __restrict__ todo, const uint32_t* __restrict__ items, uint32_t* __restrict__ tk,
     uint32_t* __restrict__ tv) {
     __shared__ BigLds s;
     const uint32_t n = min(*todo, kSlicesMax * T);
@@ -1799,11 +2072,11 @@ __global__ __launch_bounds__(kBigBlock) void k_leaf_emit_big(
     for (uint32_t o = blockIdx.x; o < n; o += gridDim.x) {
         LeafTilePlan q;
         const uint32_t item = items[o];
-        leaf_tile_plan(a, sums, info, T, item & ((1u << kSliceShift) - 1u), q);
+        leaf_tile_plan(a, false, sums, info, T, item & ((1u << kSliceShift) - 1u), q);
         __syncthreads();   // s is free again
         if (q.mode == LEAF_BIG)
-            leaf_emit_big(q, item >> kSliceShift, L, h, boxes, t, a.cap_P2, top_keys, top_vals, cells, keys, vals, refs,
-                          leaves, write_keys, s);
+            leaf_emit_big(q, item >> kSliceShift, L, h, boxes, pool, t, a.cap_P2, top_keys, top_vals, cells, keys, vals,
+                          refs, leaves, write_keys, s);
         else if (q.mode == LEAF_OVERSIZE)
             leaf_emit_oversize(q, L, h, t, a.cap_P2, top_keys, top_vals, cells, keys, vals, tk, tv, refs, leaves, s);
     }
@@ -1839,7 +2112,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_emit_par(TriSoA t, GridHeader* 
             if (key >= L.C1) return false;
             const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
             if (tile >= T) return false;
-            leaf_tile_plan(a, sums, info, T, tile, q);
+            leaf_tile_plan(a, true, sums, info, T, tile, q);
             return q.mode == LEAF_OVERSIZE;
         };
         auto acc_slot = [&](uint32_t i) { return q.pre_acc + (sacc[i] - sacc[q.a0]); };
@@ -1908,7 +2181,7 @@ __global__ __launch_bounds__(1024) void k_leaf_wide_emit(TriSoA t, GridHeader* h
         const uint32_t tile = reinterpret_cast<const uint2*>(ranges)[key].x / kLeafTile;
         LeafTilePlan q;
         q.mode = LEAF_NONE;
-        if (tile < T) leaf_tile_plan(a, sums, info, T, tile, q);
+        if (tile < T) leaf_tile_plan(a, true, sums, info, T, tile, q);
         if (q.mode != LEAF_OVERSIZE) continue;
         const uint32_t pr = q.tot_acc + q.pre_rej + (srej[i] - srej[q.a0]), rej = prej[i];
         for (uint32_t j = part * 1024u + threadIdx.x; j < rej; j += parts * 1024u)
@@ -2004,12 +2277,17 @@ void launch_leaf_cells(GridHeader* h, const BuildArgs& a, const uint32_t* ranges
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
                       const uint32_t* top_vals, const uint32_t* ranges, const uint32_t* cells, uint32_t* keys,
                       uint32_t* vals, uint32_t* tmp_keys, uint32_t* tmp_vals, float* refs, uint32_t* dbg,
-                      uint32_t* sums, uint32_t* info, uint2* boxes, const LeafLarge* large, uint32_t* leaves, hipStream_t st) {
+                      uint32_t* sums, uint32_t* info, uint2* boxes, uint32_t* box_pool, const LeafLarge* large,
+                      uint32_t* leaves, hipStream_t st) {
     const uint32_t T = (uint32_t)leaf_tiles(a.cap_P1);
     const uint32_t blocks = (a.cap_P1 + kBlock - 1) / kBlock;
+    const BoxPool pool{box_pool, (uint32_t)(leaf_pool_words(a.cap_P2) / kPools)};
+    uint32_t* pool_n = sums + 2 * (size_t)leaf_sums_stride(T) + 4 + kWideCap;   // see leaf_sums_words
+    uint32_t* todo = pool_n + kPools * kPoolStride;
     if (blocks)
         hipLaunchKernelGGL(k_leaf_count, dim3(blocks), dim3(kBlock), 0, st, t, h, top_keys, top_vals, ranges, cells,
-                           sums, info, T, dbg, boxes, large ? large->pacc : nullptr, large ? large->prej : nullptr);
+                           sums, info, T, dbg, boxes, pool, pool_n, large ? large->pacc : nullptr,
+                           large ? large->prej : nullptr);
     if (large) {
         const uint32_t* in[2] = {large->pacc, large->prej};
         uint32_t* out[2] = {large->sacc, large->srej};
@@ -2025,13 +2303,16 @@ void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const 
     // with `large`, the global sort and k_ranges need every key; without it
     // the tiles write the leaf ranges and the keys are kept for keep_debug
     uint32_t* lv = large ? nullptr : leaves;
-    uint32_t* todo = sums + 2 * (size_t)leaf_sums_stride(T) + 4 + kWideCap;   // see leaf_sums_words
     const int write_keys = (large || a.keep_debug) ? 1 : 0;
-    hipLaunchKernelGGL(k_leaf_emit, dim3(T), dim3(kLeafBlock), 0, st, t, h, a, top_keys, top_vals, cells, boxes, keys,
-                       vals, refs, sums, info, T, lv, write_keys, large ? 1 : 0, todo, todo + 1);
-    hipLaunchKernelGGL(k_leaf_emit_big, dim3(kBigBlocks), dim3(kBigBlock), 0, st, t, h, a,
-                       top_keys, top_vals, cells, boxes, keys, vals, refs, sums, info, T, lv, write_keys, todo, todo + 1,
-                       tmp_keys, tmp_vals);
+    hipLaunchKernelGGL(k_leaf_emit, dim3(T), dim3(kLeafBlock), 0, st, t, h, a, top_keys, top_vals, cells, boxes,
+                       box_pool, keys, vals, refs, sums, info, T, lv, write_keys, large ? 1 : 0, todo, todo + 1);
+    // With `large` every tile beyond one chunk is oversize: its pairs are sorted by
+    // the global sort that runs anyway.  (200,000-triangle sphere, 8 / 16 leaf cells
+    // to a triangle: 303 / 371 us with them in the larger kernel, 243 / 269 so.)
+    if (!large)
+        hipLaunchKernelGGL(k_leaf_emit_big, dim3(kBigBlocks), dim3(kBigBlock), 0, st, t, h, a, top_keys, top_vals,
+                           cells, boxes, box_pool, keys, vals, refs, sums, info, T, lv, write_keys, todo, todo + 1,
+                           tmp_keys, tmp_vals);
     if (large) {
         uint32_t pb = (a.cap_P1 + kBlock - 1) / kBlock;
         pb = pb < 1 ? 1 : (pb > 4096 ? 4096 : pb);
@@ -2208,13 +2489,17 @@ size_t leaf_tiles(uint32_t n) {
     return t ? t : 1;
 }
 // accepted and rejected totals, their grand totals, the number of wide boxes and
-// of k_leaf_scan's blocks that have ended, the list of wide boxes, the number of
-// work items of k_leaf_emit_big (all cleared before each build), then the items
+// of k_leaf_scan's blocks that have ended (then of tiles with pairs), the list of wide boxes, the words used
+// of the pool's parts, the number of work items of k_leaf_emit_big (all cleared
+// before each build), then the items
 size_t leaf_sums_words(uint32_t n) {
-    return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap + 1;
+    return 2 * (size_t)leaf_sums_stride((uint32_t)leaf_tiles(n)) + 4 + kWideCap + kPools * kPoolStride + 1;
 }
 size_t leaf_item_words(uint32_t n) { return kSlicesMax * leaf_tiles(n); }
-size_t leaf_info_words(uint32_t n) { return 5 * leaf_tiles(n); }
+size_t leaf_info_words(uint32_t n) { return 6 * leaf_tiles(n); }
+// words of the pool for n leaf pairs: a stored box of c > 32 cells takes at most
+// 2 + (c + 31) / 32 <= c / 8 of them
+size_t leaf_pool_words(uint32_t n) { return (((size_t)n / 8 + 4096) / kPools) * kPools; }
 
 
 }  // namespace sg

@@ -74,6 +74,7 @@ struct sg_grid {
     uint32_t *sums_top = nullptr, *sums_cells = nullptr, *sums_leaf = nullptr;   // per-tile sums
     uint32_t* leaf_info = nullptr;                                               // per leaf tile bounds
     uint2* boxes = nullptr;                                                      // per top pair: its leaf cells (PairBox)
+    uint32_t* box_pool = nullptr;                                                // boxes too large for a PairBox
     uint32_t* bpart = nullptr;                                                   // bounds partials
     uint32_t *sort1 = nullptr, *sort2 = nullptr;
     size_t sort1_words = 0, sort2_words = 0;

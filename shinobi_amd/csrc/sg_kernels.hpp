@@ -140,6 +140,7 @@ size_t leaf_tiles(uint32_t n);
 size_t leaf_sums_words(uint32_t n);   // cleared before each build
 size_t leaf_item_words(uint32_t n);   // behind them, not cleared
 size_t leaf_info_words(uint32_t n);
+size_t leaf_pool_words(uint32_t n);   // n = cap_P2
 // Buffers of the parallel emission of tiles too large for LDS (per top pair:
 // accepted / rejected leaf-pair totals and their exclusive scans).  Without
 // them such a tile is emitted by one block.
@@ -162,8 +163,8 @@ struct LeafLarge {
 void launch_leaf_emit(const TriSoA& t, GridHeader* h, const BuildArgs& a, const uint32_t* top_keys,
                       const uint32_t* top_vals, const uint32_t* ranges, const uint32_t* cells, uint32_t* keys,
                       uint32_t* vals, uint32_t* tmp_keys, uint32_t* tmp_vals, float* refs, uint32_t* dbg,
-                      uint32_t* sums, uint32_t* info, uint2* boxes, const LeafLarge* large, uint32_t* leaves,
-                      hipStream_t st);
+                      uint32_t* sums, uint32_t* info, uint2* boxes, uint32_t* box_pool, const LeafLarge* large,
+                      uint32_t* leaves, hipStream_t st);
 // global stable sort of the leaf pairs of tiles too large for LDS (no work
 // when there are none); the result stays in (k0, v0)
 void launch_leaf_sort_fixup(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, GridHeader* h, uint32_t cap,

@@ -287,6 +287,59 @@ def test_leaf_tile_forms_bit_exact(ctx, oracle, case, keep):
         g.rebuild()
 
 
+def _plates(n):
+    """triangles without extent along z, across many leaf cells of a plane"""
+    a = sa.gen_soup(74, n, 0.3)
+    a[5], a[8] = a[2], a[2]
+    a[2, :2], a[5, :2], a[8, :2] = [0.0, 1.0], [0.0, 1.0], [0.0, 1.0]
+    return a
+
+
+@pytest.mark.parametrize("keep", [0, 1])
+@pytest.mark.parametrize("case", [
+    ("soup", 20_000, 0.06, 2.0), ("soup", 60_000, 0.04, 2.0),       # stored boxes, tiles of several chunks
+    ("soup", 20_000, 0.01, 30.0), ("soup", 20_000, 0.01, 64.0),     # tiles of several windows of leaf cells
+    ("soup", 20_000, 0.03, 20.0),                                   # both
+    ("cells", 60, 200, 3), ("cells", 40, 600, 3),                   # boxes below and above those a wave visits
+    ("plates", 1_500, 0.0, 6.0),                                    # boxes without a plane test
+    ("one", 600, 0.9, 1.5), ("one", 1_400, 0.9, 1.5),               # more stored boxes than the pool's part holds
+], ids=lambda c: "-".join(str(x) for x in c))
+def test_stored_boxes_windows_and_chunks_bit_exact(ctx, oracle, case, keep):
+    """boxes of 33 to 1,023 leaf cells, stored by the count and listed from
+    there, and tiles beyond one window of leaf cells or one chunk of pairs"""
+    name, n, x, y = case
+    kw = dict(lam=5.0, top_divisor=6, lambda_leaf=float(y))
+    if name == "soup":
+        a = sa.gen_soup(75, n, x)
+    elif name == "cells":
+        a = _dense_cells_under_large_triangles(n, x, y)
+        kw = dict(lam=5.0, lambda_leaf=2.0, res_override=(21, 21, 21))
+    elif name == "plates":
+        a = _plates(n)
+        kw = dict(lambda_leaf=y, res_override=(3, 3, 2))
+    else:
+        a = sa.gen_soup(76, n, x)
+        kw = dict(lambda_leaf=y, res_override=(1, 1, 1))
+    og = oracle.build_twolevel(a, **kw)
+    assert og.status == 0
+    if x != 0.01:
+        assert ((og.pair_counts > 32) & (og.pair_counts < 1024)).sum() > 100
+    scene = sa.FaceSoup(ctx, a)
+    b = sa.FastTwoLevelGridBuilder(ctx, keep_debug=keep, **kw)
+    b.init(scene)
+    g = b.build()
+    rays = sa.gen_random_rays(72, 20_000, 0.0, 1.0)
+    po, to = og.trace(rays)
+    for _ in range(2):
+        assert g.info().status == 0
+        for k in ("top_cells", "leaves", "leaf_vals", "indices") + (("leaf_keys", "pair_counts") if keep else ()):
+            np.testing.assert_array_equal(g.download(k), getattr(og, k))
+        pg, tg = g.trace_host(rays)
+        np.testing.assert_array_equal(pg, po)
+        np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+        g.rebuild()
+
+
 def test_twolevel_reference_leaf_lambda(ctx, oracle):
     """lambda_leaf = 1.2 (TwoLevelBuildKernels.h:49) on the 10k soup"""
     w = W.soup10k()

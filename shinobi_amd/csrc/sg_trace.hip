@@ -608,18 +608,40 @@ SG_D Cells shfl_cells(const Cells& c, uint32_t l) {
     return o;
 }
 
+// Cells that a walk still enters before its exit distance reaches t, the current
+// one included, within 1..w: how far to look ahead of a ray whose t ends it
+// soon.  A guess from the distances between the planes: a round that ends before
+// the walk does is followed by another.  (A lane's cell costs one step of the
+// chain for each cell before it, whether the ray reaches it or not: 6,144 rays
+// of a twentieth of the scene through the uniform grid of a 102,000-triangle
+// cluster 28 us looking 64 cells ahead, 14 so.)
+SG_D uint32_t cells_to(float t, v3 tMax, v3 dt, uint32_t w) {
+    if (!__ballot(t < 1e30f)) return w;   // no ray of the wave has an end
+    auto along = [&](float m, float d) { return fmaxf((t - m) * __builtin_amdgcn_rcpf(d) + 1.f, 0.f); };
+    const float n = 1.f + along(tMax.x, dt.x) + along(tMax.y, dt.y) + along(tMax.z, dt.z);
+    return n < (float)w ? (uint32_t)n : w;
+}
+
 // The walk through a level's cells by groups of w lanes (a power of two, the
 // same in the whole wave): every lane of a group comes with the group's ray,
 // cell state and `active`; r.t and r.best are left in all of them.  Every lane
 // of the wave calls this together.  range(cell): a cell's references;
 // stops(t, tm): the t check after a cell whose exit distance is tm.
-template <class Range, class Stops>
+// The first round looks kFirstAhead cells ahead: a ray that ends there does not
+// wait for 64 (one random ray through a 200,000-triangle sphere, uniform, 13.5 ->
+// 7.8 us; 1,000 two-level ones 0.4 % longer).
+constexpr uint32_t kFirstAhead = 16;
+template <bool SHADOW, class Range, class Stops>
 SG_D void cells_ahead(const GView& g, const RemBits& b, Ray& r, Cells c, bool active, uint32_t w, Range&& range,
                       Stops&& stops) {
-    const uint32_t l = (uint32_t)lane_id(), j = l & (w - 1u), l0 = l - j, last = l0 + w - 1u;
+    const uint32_t l = (uint32_t)lane_id(), j = l & (w - 1u), l0 = l - j;
     const uint64_t group = lanes_mask(l0, w);
+    uint32_t most = min(w, kFirstAhead);
     while (__ballot(active)) {
-        bool in = active;   // lane j's cell exists
+        // (8 cells are looked at as fast as guessed)
+        const uint32_t n = SHADOW || w <= 8u ? most : cells_to(r.t, c.tMax, c.dt, most), last = l0 + n - 1u;
+        most = w;
+        bool in = active && j < n;   // lane j's cell exists
         for (uint32_t i = 0; i + 1u < w; ++i) {
             const bool go = in && j > i;
             if (!__ballot(go)) break;
@@ -697,11 +719,11 @@ SG_D void uniform_ahead(const GView& g, const GParams& p, const RemBits& b, Ray&
                         uint32_t G) {
     auto stops = [](float t, float tm) { return SHADOW ? !(t >= kShadowT) : !(t > tm); };
     if ((uint32_t)p.res[0] * (uint32_t)p.res[1] * (uint32_t)p.res[2] >= kWordCells)
-        cells_ahead(g, b, r, c, active, G, [&](uint32_t k) {
+        cells_ahead<SHADOW>(g, b, r, c, active, G, [&](uint32_t k) {
             return word_range(g, *(gptr<const u4v>)(g.words + 4u * (size_t)(k >> 5)), k);
         }, stops);
     else
-        cells_ahead(g, b, r, c, active, G, [&](uint32_t k) { return ld2(g.cells + 2u * (size_t)k); }, stops);
+        cells_ahead<SHADOW>(g, b, r, c, active, G, [&](uint32_t k) { return ld2(g.cells + 2u * (size_t)k); }, stops);
 }
 
 template <bool SHADOW>
@@ -900,14 +922,18 @@ constexpr uint32_t kTopAhead = 16, kLeafAhead = 8, kLeafLong = 48;
 template <bool SHADOW>
 SG_D void walk_twolevel_ahead(const GView& g, const GParams& p, Ray& r, Walk& w, uint32_t G) {
     const uint32_t cap = step_cap(p);
-    const uint32_t l = (uint32_t)lane_id(), j = l & (G - 1u), l0 = l - j, T = min(G, kTopAhead), last = l0 + T - 1u;
+    const uint32_t l = (uint32_t)lane_id(), j = l & (G - 1u), l0 = l - j;
     const uint64_t group = lanes_mask(l0, G);
     const RemBits b = kLeafRem;
     bool active = w.active;
     while (__ballot(active)) {
         Walk q = w;
+        uint32_t T = min(G, kTopAhead);
+        if (!SHADOW)
+            T = cells_to(r.t, w.tMax, mk(p.cs.x * fabsf(r.rcp.x), p.cs.y * fabsf(r.rcp.y), p.cs.z * fabsf(r.rcp.z)), T);
+        const uint32_t last = l0 + T - 1u;
         bool in = active && j < T;   // lane j's top cell exists
-        for (uint32_t i = 0; i + 1u < T; ++i) {
+        for (uint32_t i = 0; i + 1u < kTopAhead; ++i) {
             const bool go = in && j > i;
             if (!__ballot(go)) break;
             if (go) {
@@ -947,7 +973,7 @@ SG_D void walk_twolevel_ahead(const GView& g, const GParams& p, Ray& r, Walk& w,
             const bool act = some && mine != 0ull;
             const uint32_t from = min(first_lane(mine), 63u);
             Ray x = r;
-            cells_ahead(g, b, x, shfl_cells(lc.c, from), act, n, [&](uint32_t k) {
+            cells_ahead<SHADOW>(g, b, x, shfl_cells(lc.c, from), act, n, [&](uint32_t k) {
                 return k < p.C2 ? ld2(g.leaves + 2 * (size_t)k) : make_uint2(0u, 0u);
             }, [](float t, float tm) { return SHADOW ? t < kShadowT : !(t > tm); });
             bool same = some;   // r.t is what the walk began with
@@ -1082,7 +1108,7 @@ SG_D void walk_twolevel(const GView& g, const GParams& p, Ray& r, Walk& w, uint3
             y.guard = shfl_u(w.guard, f.src);
             // the rest of the current leaf walk, then on from the top cell
             const uint64_t leaf_m = __ballot(in_leaf);
-            cells_ahead(g, kLeafRem, x, shfl_cells(L.c, f.src), f.active && ((leaf_m >> f.src) & 1ull), f.G,
+            cells_ahead<SHADOW>(g, kLeafRem, x, shfl_cells(L.c, f.src), f.active && ((leaf_m >> f.src) & 1ull), f.G,
                         [&](uint32_t k) {
                             return k < p.C2 ? ld2(g.leaves + 2 * (size_t)k) : make_uint2(0u, 0u);
                         },
@@ -1203,29 +1229,35 @@ SG_D void trace_ahead(const GView& g, const GRays& rays, uint32_t i, gptr<uint32
 // (+1-2 % over 5 waves, 15 % slower at 7); with the max-ilp scheduler this
 // unit is built with, 5 waves without spills run the height field's bounce
 // rays 4 % faster than 6 (0.667 -> 0.641 ms) and the dense-cluster paths
-// 3 % faster, the ruins scene's bounce rays 4 % slower; the camera launch
-// is unchanged (its kernel fits 6 waves either way).  coop_tests is
+// 3 % faster, the ruins scene's bounce rays 4 % slower.  coop_tests is
 // inlined: as a call it held 12 more VGPRs across the call.
 #define SG_TRACE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(5)))
 
 // Rays per wave for a batch of n rays.  A small batch -- a late path segment,
-// a small request -- lasts as long as its longest ray.  Up to 16 rays per wave
-// of the chip (`fill` waves at once) all lanes of a wave walk ahead of 8, 4, 2
-// or 1 rays (see cells_ahead), with up to 2 fill waves: more lanes per ray
-// than that were slower on rays that end soon, fewer on the rest (49,000 rays:
-// 8 / 4 / 2 rays per wave 230 / 199 / 196 us two-level, 125 / 130 / 156
-// uniform).  Up to 32 rays per wave of the chip a wave takes 32 and finishes
-// the last of them ahead (see Few); with larger batches at 32 rays a wave
-// there are more waves than the chip holds, and 64 were faster (250,000 rays:
-// 465 against 537 us, 300,000: 523 against 683, two-level soup).
+// a small request -- lasts as long as its longest ray, so all lanes of a wave
+// walk ahead of 8, 4, 2 or 1 rays (see cells_ahead); `fill` is a measure of the
+// chip, 24 waves to a CU.  Fewer rays to a wave are faster until the waves no
+// longer run at once.  Means over seven scenes: 12,288 rays at 2 to a wave against
+// 1, random / a twentieth of the scene long: 18 / 23 % shorter in uniform grids, 10
+// / 30 % in two-level ones; 24,576 at 4 against 2 10 / 19 % and 1 / 18 %; 49,152 at
+// 8 against 4, random, 2 and 11 % longer.  From 16 fill rays on (at 32 a wave below
+// that, uniform, 98,304 random rays were 13 % shorter, coherent ones 20 % longer;
+// 70,000 3 and 30 % longer) up to 32 fill a wave takes 32, or as many more as leave
+// no wave waiting for another to end (a CU holds 20 waves of the uniform kernel, 16
+// of the two-level one: 196,608 random rays 14 % shorter at 40 to a wave, uniform,
+// and 21 % at 48, two-level), and finishes the last of them ahead (see Few); with
+// larger batches there 64 were faster (250,000 rays: 465 against 537 us, 300,000:
+// 523 against 683, two-level soup).
 constexpr uint32_t kAheadRays = 8;
 constexpr uint32_t kSparseFill = 2;   // waves of a sparse launch / fill, at most
-SG_HD uint32_t rays_per_wave(uint32_t n, uint32_t fill) {
-    if (n > (uint64_t)32 * fill) return 64u;
-    if (n > (uint64_t)(kAheadRays * kSparseFill) * fill) return 32u;
-    uint32_t R = kAheadRays;
-    while (R > 1u && (uint64_t)n <= (uint64_t)(R / 2u * kSparseFill) * fill) R /= 2u;
-    return R;
+SG_HD uint32_t rays_per_wave(int kind, uint32_t n, uint32_t fill) {
+    const uint64_t f = fill;
+    if (n > 32u * f) return 64u;
+    if (n > 16u * f) {
+        const uint32_t held = fill / 6u * (kind == 0 ? 5u : 4u), R = (n + held - 1u) / held;
+        return R < 32u ? 32u : (R + 7u) & ~7u;
+    }
+    return n > 8u * f ? kAheadRays : (n > 2u * f ? 4u : (n > f ? 2u : 1u));
 }
 
 // One batch, the block size a launch parameter.  SPARSE = false: one ray
@@ -1238,7 +1270,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ?
                                                   uint32_t fill, uint32_t* __restrict__ prim,
                                                   float* __restrict__ tout, uint32_t* __restrict__ stats) {
     const uint32_t n = d_n ? min(*d_n, cap) : cap;
-    const uint32_t R = rays_per_wave(n, fill);
+    const uint32_t R = rays_per_wave(KIND, n, fill);
     if (SPARSE != (R < 64u)) return;
     if (!SPARSE) {
         const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1264,7 +1296,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ?
     }
 }
 
-// waves the device holds at once (6 per SIMD, 4 SIMDs per CU), per device
+// `fill` of rays_per_wave, per device: 6 waves to a SIMD, 4 SIMDs to a CU.  (What
+// the kernels hold differs: the uniform ones 8 waves to a SIMD, sparse 5, the
+// two-level ones 5, sparse 4.)
 static uint32_t device_fill() {
     static uint32_t cache[64] = {0};
     int dev = 0;
@@ -1291,8 +1325,8 @@ void launch_trace(const GridView& g, const RaySoA& r, uint32_t n, const uint32_t
     // dense grid: one lane per ray of the capacity; sparse grid: the waves
     // that cover every count that takes the sparse form
     const dim3 dense((n + B - 1) / B), sparse((kSparseFill * fill + B / 64 - 1) / (B / 64)), tb(B);
-    const bool want_dense = d_n || rays_per_wave(n, fill) == 64u;
-    const bool want_sparse = d_n || rays_per_wave(n, fill) < 64u;
+    const uint32_t R = rays_per_wave(g.kind, n, fill);
+    const bool want_dense = d_n || R == 64u, want_sparse = d_n || R < 64u;
 #define SG_TRACE(K, S, H)                                                                                         \
     do {                                                                                                          \
         if (want_dense)                                                                                           \
@@ -1360,7 +1394,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ?
     uint32_t i = block * blockDim.x + threadIdx.x, G = 1;
     bool valid = i < n;
     if (SPARSE) {   // one-wave blocks
-        const uint32_t R = rays_per_wave(n, fill), l = (uint32_t)lane_id();
+        const uint32_t R = rays_per_wave(KIND, n, fill), l = (uint32_t)lane_id();
         if (block * R >= n) return;
         // failed builds and irregular leaf levels go the general way
         if (!__builtin_amdgcn_readfirstlane((int)(gv.hdr->status & ~ST_NEG_EXTENT))) G = 64u / R;
@@ -1419,7 +1453,7 @@ void launch_trace_gen(const GridView& g, const RaySoA& r, const CamArgs* cam, ui
     if (cam) c = *cam;
     const uint32_t fill = device_fill();
     // a count in device memory takes the dense form
-    const uint32_t R = d_n ? 64u : rays_per_wave(n, fill);
+    const uint32_t R = d_n ? 64u : rays_per_wave(g.kind, n, fill);
     const bool sparse = R <= kAheadRays;   // 32 rays a wave gain nothing on camera rays
     const dim3 grid((n + (sparse ? R : B) - 1) / (sparse ? R : B)), tb(B);
 #define SG_GEN(K, C)                                                                                               \

@@ -478,3 +478,67 @@ def test_rays_that_never_leave_walk_ahead(ctx, oracle):
         p, t = g.trace_host(rays)
         np.testing.assert_array_equal(p, ps)
         np.testing.assert_array_equal(t.view(np.uint32), ts.view(np.uint32))
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("scene", ["soup", "cluster", "heightfield"])
+def test_short_rays_and_rays_per_wave(ctx, oracle, scene, kind, shadow):
+    """rays that end after a few cells, inside one and within the first round of
+    cells looked at, on either side of every count of rays per wave (a device of
+    256 CUs): ids and t equal the oracle's bit for bit, with the count on the
+    host and on the device"""
+    a = _ahead_scene(scene)
+    opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)
+    og = oracle.build_twolevel(a, **opt) if kind else oracle.build_uniform(a, top_divisor=1, **opt)
+    b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    sizes = [1, 2, 6_144, 6_145, 12_288, 12_289, 49_152, 49_153, 98_304, 98_305, 131_072, 131_073, 163_840, 163_841,
+             196_608, 196_609]
+    rays = sa.gen_random_rays(99, max(sizes), -0.1, 1.1)
+    n = rays.shape[1]
+    rng = np.random.default_rng(100)
+    rays[6] = rng.choice(np.array([1e-4, 0.01, 0.05, 0.2, 0.6, 3.0, 3.0e38], np.float32), n)
+    rays[3, ::19], rays[5, 7::23] = 0.0, -0.0
+    if shadow:
+        rays[3:6] *= np.minimum(rays[6], np.float32(10.0))   # the segment's length in its direction
+        rays[6] = 1.0
+    rays = np.ascontiguousarray(rays)
+    po, to = og.trace(rays, shadow=shadow)[:2]
+    assert (po != sa.MISS).sum() > 50
+    cap = sa.RayBatch(ctx, rays)
+    count = sa.DeviceBuffer(ctx, 4)
+    for m in sizes:
+        p, t = g.trace_host(np.ascontiguousarray(rays[:, :m]), shadow=shadow)
+        np.testing.assert_array_equal(p, po[:m])
+        np.testing.assert_array_equal(t.view(np.uint32), to[:m].view(np.uint32))
+        count.upload(np.array([m], np.uint32))
+        pd, td = g.trace(cap, d_count=count.ptr, n=n, shadow=shadow)
+        np.testing.assert_array_equal(pd.download(np.uint32, m), po[:m])
+        np.testing.assert_array_equal(td.download(np.float32, m).view(np.uint32), to[:m].view(np.uint32))
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_nan_and_infinite_rays_equal_the_oracle(ctx, oracle, kind, shadow):
+    """the general walk (with counters) and the walk ahead of NaN and infinite
+    rays, which only the guard of both sides ends"""
+    a = _clumped_soup(0.0)
+    opt = dict(lam=5.0, top_divisor=6, lambda_leaf=2.0, leaf_min_refs=16) if kind else dict(lam=5.0)
+    og = oracle.build_twolevel(a, **opt) if kind else oracle.build_uniform(a, top_divisor=1, **opt)
+    b = (sa.FastTwoLevelGridBuilder if kind else sa.FastSimpleGridBuilder)(ctx, **opt)
+    b.init(sa.FaceSoup(ctx, a))
+    g = b.build()
+    rays = sa.gen_random_rays(97, 640, -0.2, 1.2)
+    if shadow:
+        rays[6] = 1.0
+    rays[0, ::7], rays[3, 1::7], rays[6, 2::7], rays[4, 3::7], rays[5, 4::7] = np.nan, np.nan, np.nan, np.inf, -np.inf
+    po, to, so = og.trace(rays, with_stats=True, shadow=shadow)
+    ps, ts, ss = g.trace_host(rays, with_stats=True, shadow=shadow)
+    np.testing.assert_array_equal(ps, po)
+    np.testing.assert_array_equal(ts.view(np.uint32), to.view(np.uint32))
+    np.testing.assert_array_equal(ss, so)
+    p, t = g.trace_host(rays, shadow=shadow)
+    np.testing.assert_array_equal(p, po)
+    np.testing.assert_array_equal(t.view(np.uint32), to.view(np.uint32))

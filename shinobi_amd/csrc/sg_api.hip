@@ -276,7 +276,8 @@ static size_t grid_layout(sg_grid* g, char* pool) {
         g->leaves = (uint32_t*)take((size_t)g->cap_C2 * 8 + 16);
     }
     g->refs = (float*)take((size_t)(two ? g->cap_P2 : g->cap_P1) * 36 + 16);
-    g->words = two ? nullptr : (uint4*)take(cell_words(g->cap_C1) * sizeof(uint4));
+    // neither written nor read below kWordCells
+    g->words = two || g->cap_C1 < kWordCells ? nullptr : (uint4*)take(cell_words(g->cap_C1) * sizeof(uint4));
     if (two && g->large_path) {
         g->large.pacc = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);
         g->large.prej = (uint32_t*)take((size_t)g->cap_P1 * 4 + 16);

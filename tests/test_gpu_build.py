@@ -590,3 +590,22 @@ def test_leaf_ranges_beyond_the_packed_resolutions(ctx, oracle, n, axis, thin, l
         po, to = og.trace(rays, shadow=shadow)[:2]
         np.testing.assert_array_equal(pg, po)
         np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+
+
+def test_cell_words_only_where_they_are_read(ctx, oracle):
+    """a uniform grid of 2^17 cells holds cell words (half a byte a cell), a
+    smaller one does not; both trace as the oracle"""
+    v = np.array([[0, 0, 0], [0.01, 0, 0.01], [0, 0.01, 0.01]], np.float32)
+    soa = np.ascontiguousarray(np.stack([v, 1 - v], 2).reshape(9, 2))
+    rays = sa.gen_random_rays(99, 4000, 0.0, 0.02)
+    size = []
+    for rz in (31, 32):
+        kw = dict(lam=5.0, res_override=(64, 64, rz))
+        scene, g = _gpu_build(ctx, soa, 0, **kw)
+        size.append(g.info().device_bytes)
+        po, to = oracle.build_uniform(soa, **kw).trace(rays)[:2]
+        pg, tg = g.trace_host(rays)
+        np.testing.assert_array_equal(pg, po)
+        np.testing.assert_array_equal(tg.view(np.uint32), to.view(np.uint32))
+    ranges, words = 64 * 64 * 8, 64 * 64 * 32 // 2
+    assert abs(size[1] - size[0] - ranges - words) <= 2048

@@ -700,6 +700,7 @@ def main() -> int:
                 "frac": launches[dom]["frac"], "traffic": launches[dom]["traffic"],
                 "valu_util": launches[dom].get("valu_util"), "lanes_active": launches[dom].get("lanes_active"),
                 "l2_hit": launches[dom].get("l2_hit"),
+                "counters_from": "profiles/heightfield2m_pmc_*.json: profiled runs of this workload, not this run",
                 "flops_per_launch": launches[dom]["flops"], "launches": launches,
                 "dominant_phase": dominant[0]}
     copy = hbm_copy_rate(ctx)

@@ -170,7 +170,11 @@ sg_status sg_rebuild_many(sg_ctx *ctx, uint32_t n, sg_scene *const *scenes, sg_g
  * the analogue of the builders' phase timers (FastTwoLevelGridBuilder.h:
  * 755-781): [0] start, [1] bounds, [2] top emission, [3] top sort, [4] top
  * ranges, and for the two-level grid [5] leaf cells, [6] leaf emission,
- * [7] leaf sort, [8] leaf ranges.  Null entries are skipped. */
+ * [7] leaf sort, [8] leaf ranges.  Null entries are skipped.  A phase holds
+ * what its launches do: the grid's parameters are derived between [1] and
+ * [2] (by the reference, and by versions of this library before that, with
+ * the bounds), the leaf ranges are written by the leaf emission and [7] to
+ * [8] is empty unless the global leaf sort ran. */
 sg_status sg_rebuild_phased(sg_ctx *ctx, sg_scene *scene, sg_grid *grid, void *stream, void *const *events,
                             int n_events);
 /* waits for the grid's stream, reads the device header */

@@ -332,11 +332,6 @@ static sg_status grid_alloc(sg_grid* g) {
     return SG_OK;
 }
 
-// Enqueue the whole build on `st`.  marks (optional, n_marks entries) are
-// hipEvent_t recorded at the phase boundaries: [0] start, [1] after
-// init+bounds, [2] parameters and top emission, [3] top sort, [4] top ranges, then for the
-// two-level grid [5] leaf cells, [6] leaf emission, [7] leaf sort, [8] leaf
-// ranges.
 // the build arguments of a grid's (re)build
 static BuildArgs build_args(const sg_grid* g, bool fixed_res) {
     const bool two = g->kind == SG_GRID_TWO_LEVEL;
@@ -410,6 +405,11 @@ bool uni_job_of(sg_grid* g, UniJob* j) {
 
 extern "C" {
 
+// Enqueue the whole build on `st`.  marks (optional, n_marks entries) are
+// hipEvent_t recorded at the phase boundaries: [0] start, [1] after
+// init+bounds, [2] parameters and top emission, [3] top sort, [4] top ranges,
+// then for the two-level grid [5] leaf cells, [6] leaf emission, [7] leaf sort,
+// [8] leaf ranges.
 static void enqueue_build(sg_grid* g, bool fixed_res, hipStream_t st, void* const* marks = nullptr,
                           int n_marks = 0) {
     auto mark = [&](int i) {

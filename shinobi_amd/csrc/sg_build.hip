@@ -19,8 +19,11 @@ namespace sg {
 // Triangles per thread in the top-level count and emission: four (16-byte
 // loads), or one for scenes too small to give every CU a block that way, whose
 // time is the longest lane's emission.
-// (k_top_emit with one: 10,000-triangle soup 17.2 -> 6.8 us; with one or two
-// on the 2,093,058-triangle height field the rebuild was 4 % slower or equal.)
+// (k_top_emit with one: 10,000-triangle soup 17.2 -> 6.8 us.  Two-level
+// rebuilds with one / four, in us: soups of 300,000 triangles 98 / 103, 524,288
+// 129 / 132, 600,000 140 / 140, 1,000,000 206 / 200; height fields of 520,000
+// 126 / 131, 1,030,000 180 / 178, 2,093,058 359 / 328.  Uniform soups: 300,000
+// 105 / 112, 600,000 161 / 164, 1,000,000 281 / 291.)
 constexpr int kItems = 4;
 constexpr uint32_t kSmallTop = 1u << 19;       // triangles up to which a thread takes one
 constexpr uint32_t kStage = 1024;              // top pairs a tile stages in LDS, for each of a thread's triangles
@@ -589,9 +592,10 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells_write(GridHeader* h, Buil
 // begins and which cells of it were accepted (PairBox); the emit kernel
 // counts the tile's pairs per leaf cell in LDS, scans the counts, puts each
 // pair's index into its cells' lists and writes accepted pairs to their final
-// slots and rejected ones to the tail.  A tile too large for LDS writes
-// its pairs in emission order and raises GridHeader::leaf_sort, which enables
-// a global stable radix sort of the accepted pairs (a no-op otherwise).
+// slots and rejected ones to the tail.  An oversize tile is emitted and sorted
+// by one block; in a grid whose build has met one, its pairs are written in
+// emission order by many, and GridHeader::leaf_sort enables a global stable
+// radix sort of the accepted pairs (a no-op otherwise).
 constexpr uint32_t kLeafTile = 512;                   // nominal sorted top pairs per leaf tile
 constexpr int kLeafBlock = 512;                       // threads of the leaf emission kernel
 constexpr int kBigBlock = 1024;                       // threads of its form for larger tiles
@@ -610,9 +614,11 @@ struct LeafBig {
 // leaf cells whose lists begin in [s * kLeafSlice, (s+1) * kLeafSlice) of the
 // tile's accepted pairs.  Every block counts the whole tile, then lists, sorts
 // and writes its slice only.  Few tiles are so large, so their slices are small
-// to use the chip: 4096 / 2048 / 1024 / 512 / 256 pairs rebuild a 200,000-
-// triangle sphere in 174 / 162 / 153 / 147 / 164 us, the ruins scene, with more
-// such tiles, in 274 / 263 / 254 / 286 / 356 us.
+// to use the chip, but each costs a count of the tile.  Rebuilds with slices of
+// 2048 / 1024 / 512 pairs, in us: the 200,000-triangle sphere 150 / 143 / 142,
+// with a leaf density of 4 172 / 167 / 198, with a top divisor of 12 168 / 162 /
+// 190; the ruins scene 252 / 240 / 234; a 520,000-triangle height field with a
+// leaf density of 16 230 / 243 / 257; eleven others within 2 %.
 constexpr uint32_t kLeafSlice = 1024;
 constexpr uint32_t kSliceShift = 24, kSlicesMax = (LeafBig::pairs + kLeafSlice - 1) / kLeafSlice;
 constexpr int kTopBits = 13;                          // a list entry's top pair bits
@@ -1538,8 +1544,8 @@ SG_D void leaf_reject(uint32_t r, uint32_t n, uint32_t tri, uint32_t cap, uint32
 
 // Tiles that fit LeafSmall.  Each pair's box comes from k_leaf_count, so a
 // tile is a counting sort of its accepted cells: LDS counts, one scan, LDS
-// lists.  2,093,058-triangle height field, 6.6 M references: 139 us for 433 MB
-// (3.1 TB/s; the reference records alone are 239 MB), VALU busy for half of
+// lists.  2,093,058-triangle height field, 6.6 M references: 140 us for 443 MB
+// (3.2 TB/s; the reference records alone are 239 MB), VALU busy for half of
 // it, the rest waiting for memory in the first loads (36 % of a block's time)
 // and the write-out (40 %).  The form before it, a stable two-pass LDS radix
 // sort of staged pairs with the boxes formed again from the gathered
@@ -1708,8 +1714,7 @@ __global__ __launch_bounds__(kLeafBlock) __attribute__((amdgpu_waves_per_eu(8)))
     const uint32_t* __restrict__ cells, const uint2* __restrict__ boxes, const uint32_t* __restrict__ pool,
     uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, float* __restrict__ refs,
     const uint32_t* __restrict__ sums, const uint32_t* __restrict__ info, uint32_t T, uint32_t* __restrict__ leaves,
-    int write_keys, int large,
-    uint32_t* __restrict__ todo, uint32_t* __restrict__ items) {
+    int write_keys, int large, uint32_t* __restrict__ todo, uint32_t* __restrict__ items) {
     constexpr int NW = kLeafBlock / 64;
     __shared__ uint32_t s_scan[NW], s_ord[LeafSmall::chunk], s_tri[LeafSmall::tops], s_k1;
     __shared__ uint32_t s_bm[LeafSmall::tops / 32 * NW];
@@ -2249,7 +2254,8 @@ void launch_top_emit(const TriSoA& t, uint32_t n, GridHeader* h, const BuildArgs
     const dim3 blocks((uint32_t)top_tiles(n, items)), tb(kBlock);
     if (n == 0) return;
     if (items == 1) {
-        hipLaunchKernelGGL(k_top_count_params, blocks, tb, 0, st, t, n, h, a, part, (uint32_t)bounds_blocks(n), sums, dbg);
+        hipLaunchKernelGGL(k_top_count_params, blocks, tb, 0, st, t, n, h, a, part, (uint32_t)bounds_blocks(n), sums,
+                           dbg);
         hipLaunchKernelGGL(k_top_emit<1>, blocks, tb, 0, st, t, n, h, a, keys, vals, sums);
     } else {
         launch_params(h, a, part, n, true, st);

@@ -1266,9 +1266,9 @@ SG_HD uint32_t rays_per_wave(int kind, uint32_t n, uint32_t fill) {
 // exits unless the count is its case, so the dense kernel carries none of
 // the sparse form's registers.
 template <int KIND, bool STATS, bool SHADOW, bool SPARSE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ? 4 : 5))) void k_trace(GridView g, RaySoA rays, uint32_t cap, const uint32_t* d_n,
-                                                  uint32_t fill, uint32_t* __restrict__ prim,
-                                                  float* __restrict__ tout, uint32_t* __restrict__ stats) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPARSE ? 4 : 5))) void k_trace(
+    GridView g, RaySoA rays, uint32_t cap, const uint32_t* d_n, uint32_t fill, uint32_t* __restrict__ prim,
+    float* __restrict__ tout, uint32_t* __restrict__ stats) {
     const uint32_t n = d_n ? min(*d_n, cap) : cap;
     const uint32_t R = rays_per_wave(KIND, n, fill);
     if (SPARSE != (R < 64u)) return;
@@ -1481,8 +1481,8 @@ void launch_trace_gen(const GridView& g, const RaySoA& r, const CamArgs* cam, ui
 // kind: a kernel that could run either walk would hold the registers of
 // the larger one.
 template <int KIND, bool SHADOW>
-__global__ __launch_bounds__(kBlock) SG_TRACE_OCCUPANCY void k_trace_items(const TraceItem* __restrict__ items, uint32_t n_items,
-                                                        uint32_t total_chunks) {
+__global__ __launch_bounds__(kBlock) SG_TRACE_OCCUPANCY void k_trace_items(const TraceItem* __restrict__ items,
+                                                                           uint32_t n_items, uint32_t total_chunks) {
     const uint32_t c = blockIdx.x * (blockDim.x / 64u) + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (c >= total_chunks) return;
     // Last item whose first chunk is <= c.  The table is read with
